@@ -46,7 +46,8 @@ class OracleError(RuntimeError):
 def build(reference: bool = True) -> None:
     """Compile the oracle (and, when the reference tree exists, oracle/_ref)."""
     targets = ["all"]
-    if reference and os.path.isdir(os.environ.get("REFERENCE", "/root/reference")):
+    if reference and os.path.isdir(os.path.join(os.environ.get("REFERENCE", "/root/reference"),
+                                                "cpp")):
         targets.append("ref")
         # The reference-side hip backend needs the built HIP library.
         if os.path.exists(os.path.join(os.path.dirname(HERE), "microsimulator_amd",
