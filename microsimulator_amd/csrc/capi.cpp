@@ -1225,6 +1225,8 @@ int msim_hip_create(int device, msim_ctx** out) {
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
     ctx->impl.name = prop.name;
     if (ctx->impl.name.empty()) ctx->impl.name = prop.gcnArchName;
+    if (prop.cooperativeLaunch != 0)
+      ctx->impl.resident_blocks = static_cast<uint32_t>(prop.multiProcessorCount);
   }
   *out = ctx;
   return MSIM_OK;

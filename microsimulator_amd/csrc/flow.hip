@@ -21,6 +21,7 @@
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "persist.hpp"
 #include "stencil.hpp"
 
 namespace msim {
@@ -487,6 +488,225 @@ __global__ __launch_bounds__(kStream) void k_cg_init(const S* __restrict__ sourc
   }
 }
 
+// Jacobi-PCG iterations in one persistent launch, for systems of at most
+// kPersistSites sites. Each workgroup owns kPersistThreads * S consecutive
+// sites and holds their x, r, coefficients and half of q's use in registers;
+// the direction p of its sites and of the ny sites either side (every site its
+// stencils read) lives in LDS. Per iteration the workgroups meet twice
+// (round_sums): for p.q, and for r.r and r.z. Before the second meeting each
+// publishes z = M^-1 r of its sites, so afterwards every workgroup forms the
+// neighbours' new direction itself, z + beta p, and p is never exchanged.
+// The arithmetic per site is k_cg_apply's and k_cg_update's; the sums are
+// added in the rounds' order.
+//
+// Such systems are bound by latency, not by memory (33k to 1M sites are 3 to
+// 90 MB per FP64 iteration, cache-resident): two launches per iteration, each
+// of whose blocks re-adds the partials first, against two trips of a word to
+// memory and back. Per iteration, the launches and this kernel, on pillar
+// arrays (FP64; FP32): 64x48 15.6 and 3.6 us; 256x128 13.9 and 5.8 us;
+// 512x256 14.9 and 8.7 us; 1024x512 20.1 and 10.8 us (17.4 and 8.9); 1024x1000
+// 27.7 and 16.0 us (23.2 and 11.3). 256 or 1024 threads per workgroup lose
+// 5 to 70 % from 512x256 up.
+//
+// Starts from r, x, p, rho and beta as k_cg_init or an earlier launch left
+// them, at iteration `taken` + 1, and takes at most `budget` iterations.
+template <typename T, int S>
+__global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
+    T* __restrict__ r, T* __restrict__ xsol, T* __restrict__ p, uint64_t* words,
+    const float* __restrict__ diag, const float* __restrict__ cxl, const float* __restrict__ cyl,
+    const float* __restrict__ bc, uint32_t n, uint32_t ny, T isx, T isy, CgState* st,
+    uint64_t* slots, uint32_t tag, uint32_t budget, uint32_t taken) {
+  constexpr int NT = kPersistThreads;
+  constexpr int kAhead = 2;  // halo values polled for with the sums, per thread
+  extern __shared__ __align__(16) unsigned char s_raw[];
+  T* s_p = reinterpret_cast<T*>(s_raw);  // ny sites below, the own ones, ny above
+  __shared__ RoundLds L;
+  const int t = threadIdx.x;
+  if (t == 0) L.stalled = 0;
+  const uint32_t start = blockIdx.x * (NT * S);
+  const uint32_t own = min(n - start, static_cast<uint32_t>(NT * S));
+  const T zero = static_cast<T>(0);
+  T xv[S], rv[S], zv[S], dv[S], cb[S], cxlo[S], cxhi[S], cylo[S], cyhi[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const uint32_t l = static_cast<uint32_t>(t + s * NT);
+    xv[s] = rv[s] = zv[s] = dv[s] = cb[s] = cxlo[s] = cxhi[s] = cylo[s] = cyhi[s] = zero;
+    if (l < own) {
+      const uint32_t i = start + l;
+      xv[s] = xsol[i];
+      rv[s] = r[i];
+      dv[s] = static_cast<T>(diag[i]);
+      zv[s] = dv[s] > zero ? rv[s] / dv[s] : zero;
+      cb[s] = static_cast<T>(bc[i]);
+      // The lower couplings are zero on the grid's first row and column, and
+      // the first column's is also the last column's upper one.
+      cxlo[s] = static_cast<T>(cxl[i]) * isx;
+      cxhi[s] = i + ny < n ? static_cast<T>(cxl[i + ny]) * isx : zero;
+      cylo[s] = static_cast<T>(cyl[i]) * isy;
+      cyhi[s] = i + 1 < n ? static_cast<T>(cyl[i + 1]) * isy : zero;
+      s_p[ny + l] = p[i];
+    }
+  }
+  // Halo entry h of 2 ny: site start - ny + h below the own sites, start +
+  // own + (h - ny) above them; n where there is none.
+  auto halo_site = [&](uint32_t h) -> uint32_t {
+    if (h < ny) return start + h >= ny ? start + h - ny : n;
+    return start + own + (h - ny);
+  };
+  auto halo_slot = [&](uint32_t h) { return h < ny ? h : own + h; };
+  for (uint32_t h = t; h < 2 * ny; h += NT) {
+    const uint32_t i = halo_site(h);
+    s_p[halo_slot(h)] = i < n ? p[i] : zero;
+  }
+  double rho = st->rho, rr = st->rr, alpha_d = 0.0, beta_d = st->beta, curvature = 0.0;
+  const double threshold = st->threshold;
+  const Exchange<T> ex{words, n};
+  uint32_t failure = 0, k = 0;
+  bool halted = false, alive = true;
+  // z of the thread's first kAhead halo entries (t + u NT).
+  uint32_t site_h[kAhead];
+  T zh[kAhead];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const uint32_t h = static_cast<uint32_t>(t + u * NT);
+    site_h[u] = h < 2 * ny ? min(halo_site(h), n) : n;
+  }
+  auto z_of = [&](uint32_t i) {
+    const T d = static_cast<T>(diag[i]);
+    return d > zero ? r[i] / d : zero;
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) zh[u] = site_h[u] < n ? z_of(site_h[u]) : zero;
+  while (k < budget && failure == 0 && !halted) {
+    const T beta = static_cast<T>(beta_d);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      if (l < own) s_p[ny + l] = zv[s] + beta * s_p[ny + l];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const uint32_t h = static_cast<uint32_t>(t + u * NT);
+      if (site_h[u] < n) s_p[halo_slot(h)] = zh[u] + beta * s_p[halo_slot(h)];
+    }
+    // The rest of a wide grid's halo.
+    for (uint32_t h = t + kAhead * NT; h < 2 * ny; h += NT) {
+      const uint32_t i = halo_site(h);
+      if (i >= n) continue;
+      T z;
+      if (k == 0) {
+        z = z_of(i);
+      } else {
+        uint64_t w[Exchange<T>::kWords];
+        poll_words(
+            L, [&] { ex.load(i, w); }, [&] { return Exchange<T>::has(w, tag - 1); });
+        z = Exchange<T>::value(w);
+      }
+      s_p[halo_slot(h)] = z + beta * s_p[halo_slot(h)];
+    }
+    __syncthreads();
+    T qv[S];
+    double pq[1] = {0.0};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      qv[s] = zero;
+      if (l < own) {
+        const T c = s_p[ny + l];
+        T v = cb[s] * c;
+        v += cxlo[s] * (c - s_p[l]);
+        v += cxhi[s] * (c - s_p[l + 2 * ny]);
+        v += cylo[s] * (c - s_p[ny + l - 1]);
+        v += cyhi[s] * (c - s_p[ny + l + 1]);
+        qv[s] = v;
+        pq[0] += static_cast<double>(c) * static_cast<double>(v);
+      }
+    }
+    alive = round_sums<1>(
+        pq, slots, tag++, L, [] {}, [] { return true; });
+    if (!alive) break;
+    curvature = pq[0];
+    if (!isfinite(curvature) || curvature <= 0.0) {
+      failure = 1;
+      break;
+    }
+    alpha_d = rho / curvature;
+    if (!isfinite(alpha_d)) {
+      failure = 2;
+      break;
+    }
+    const T alpha = static_cast<T>(alpha_d);
+    double sums[2] = {0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      if (l < own) {
+        xv[s] = xv[s] + alpha * s_p[ny + l];
+        rv[s] = rv[s] - alpha * qv[s];
+        zv[s] = dv[s] > zero ? rv[s] / dv[s] : zero;
+        ex.put(start + l, tag, zv[s]);
+        sums[0] += static_cast<double>(rv[s]) * static_cast<double>(rv[s]);
+        sums[1] += static_cast<double>(rv[s]) * static_cast<double>(zv[s]);
+      }
+    }
+    uint64_t w[kAhead][Exchange<T>::kWords];
+    alive = round_sums<2>(
+        sums, slots, tag, L,
+        [&] {
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u) {
+            if (site_h[u] < n) ex.load(site_h[u], w[u]);
+          }
+        },
+        [&] {
+          bool all = true;
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u)
+            all = all && (site_h[u] >= n || Exchange<T>::has(w[u], tag));
+          return all;
+        });
+    ++tag;
+    if (!alive) break;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (site_h[u] < n) zh[u] = Exchange<T>::value(w[u]);
+    }
+    ++k;
+    rr = sums[0];
+    if (!isfinite(rr)) {
+      failure = 3;
+    } else if (rr <= threshold) {
+      halted = true;
+    } else if (!isfinite(sums[1]) || rho == 0.0) {
+      failure = 4;
+    } else {
+      beta_d = sums[1] / rho;
+      if (!isfinite(beta_d)) failure = 5;
+    }
+    rho = sums[1];
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const uint32_t l = static_cast<uint32_t>(t + s * NT);
+    if (l < own) {
+      xsol[start + l] = xv[s];
+      r[start + l] = rv[s];
+      p[start + l] = s_p[ny + l];
+    }
+  }
+  // Every workgroup read st before its first round; this one is past its last.
+  if (blockIdx.x == 0 && t == 0) {
+    st->it_update = st->it_apply = taken + k;
+    st->halt = halted ? taken + k : 0u;
+    st->rr = rr;
+    st->rho = rho;
+    st->alpha = alpha_d;
+    st->beta = beta_d;
+    st->curvature = curvature;
+    st->failure = alive ? failure : kRoundStalled;
+  }
+}
+
 // FP64 refinement update: x += scale * e.
 __global__ void k_refine(double* __restrict__ xsol, const float* __restrict__ e, double scale,
                          size_t n) {
@@ -715,6 +935,43 @@ __global__ __launch_bounds__(kStream) void k_scale(float* __restrict__ faces, si
 // Host orchestration
 // --------------------------------------------------------------------------
 
+uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words) {
+  // Fresh memory and reused tags are cleared: a word counts by its tag.
+  const bool fresh = ctx.round_slots.size() == 0 || ctx.round_tag > 0xffffffffu - rounds;
+  if (fresh) {
+    ctx.round_slots.reserve(kRoundSlots);
+    check(hipMemsetAsync(ctx.round_slots.data(), 0, kRoundSlots * sizeof(uint64_t), ctx.stream),
+          "clear rounds");
+    ctx.round_tag = 1;
+  }
+  if (words > ctx.round_words.size()) {
+    ctx.round_words.reserve(words);
+  } else if (!fresh) {
+    words = 0;
+  }
+  if (words > 0) {
+    check(hipMemsetAsync(ctx.round_words.data(), 0, ctx.round_words.size() * sizeof(uint64_t),
+                         ctx.stream),
+          "clear exchange");
+  }
+  const uint32_t tag = ctx.round_tag;
+  ctx.round_tag += rounds;
+  return tag;
+}
+
+bool launch_resident(Context& ctx, const void* kernel, uint32_t blocks, void** args, size_t lds,
+                     const char* what) {
+  const hipError_t status = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads),
+                                                       args, static_cast<uint32_t>(lds),
+                                                       ctx.stream);
+  if (status == hipErrorCooperativeLaunchTooLarge) {
+    static_cast<void>(hipGetLastError());
+    return false;
+  }
+  check(status, what);
+  return true;
+}
+
 uint32_t stream_blocks(size_t n) {
   const size_t per_block = static_cast<size_t>(kStream) * kUnroll;
   const size_t blocks = (n + per_block - 1) / per_block;
@@ -857,6 +1114,58 @@ const char* failure_text(uint32_t failure) {
   }
 }
 
+// Whether Jacobi-PCG of precision T on this system runs as one persistent
+// launch, and its shape: the fewest sites per thread that fit the device's
+// compute units, one workgroup each, with the direction and its halo of ny
+// sites either side in at most 60 KB of LDS. The line is what the registers
+// hold: eight sites per thread (FP64: 255 VGPRs), 1M sites on 256 compute
+// units, where this is still 1.7 (FP64) and 2.1 times (FP32) as fast per
+// iteration as the launches.
+struct PersistShape {
+  int sites;        // per thread; 0: not this way
+  uint32_t blocks;
+  size_t lds;
+};
+
+template <typename T>
+PersistShape persist_shape(const Context& ctx) {
+  const auto& f = ctx.flow;
+  const size_t n = f.sites();
+  for (int s : {1, 2, 4, 8}) {
+    const size_t chunk = static_cast<size_t>(kPersistThreads) * s;
+    const size_t blocks = (n + chunk - 1) / chunk;
+    const size_t lds = (std::min(chunk, n) + 2 * static_cast<size_t>(f.ny)) * sizeof(T);
+    if (blocks <= std::min<size_t>(ctx.resident_blocks, kRoundBlocks) && lds <= 60 * 1024)
+      return PersistShape{s, static_cast<uint32_t>(blocks), lds};
+  }
+  return PersistShape{0, 0, 0};
+}
+
+// One persistent launch of at most `budget` iterations; false where the
+// device does not take it (too few free compute units for the grid).
+template <typename T>
+bool launch_persistent(Context& ctx, const PersistShape& shape, T* r, T* x, T* p,
+                       uint32_t budget, uint32_t taken) {
+  auto& f = ctx.flow;
+  uint32_t n = static_cast<uint32_t>(f.sites()), ny = f.ny;
+  T isx = static_cast<T>(1.0 / (static_cast<double>(f.dx) * f.dx));
+  T isy = static_cast<T>(1.0 / (static_cast<double>(f.dy) * f.dy));
+  const float *diag = f.diag.data(), *cxl = f.cxl.data(), *cyl = f.cyl.data(), *bc = f.bc.data();
+  CgState* st = f.state.data();
+  uint32_t tag = take_rounds(ctx, 2 * budget, Exchange<T>::kWords * f.sites());
+  uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
+  void* args[] = {&r, &x, &p, &words, &diag, &cxl, &cyl, &bc, &n, &ny, &isx, &isy,
+                  &st, &slots, &tag, &budget, &taken};
+  const void* kernel = nullptr;
+  switch (shape.sites) {
+    case 1: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 1>); break;
+    case 2: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 2>); break;
+    case 4: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 4>); break;
+    default: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 8>); break;
+  }
+  return launch_resident(ctx, kernel, shape.blocks, args, shape.lds, "launch k_cg_persistent");
+}
+
 // Runs Jacobi-PCG iterations of precision T on the prepared system from the
 // state launch_init left, until the stopping test holds, a failure, or
 // `budget` iterations (conjugate_gradient.hpp:126-166: the host looks at the
@@ -884,6 +1193,34 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
     return 0;
   }
   const double rr0 = f.host_state->rr0;
+  auto judge = [&](const CgState& s) {
+    if (s.failure == kRoundStalled)
+      throw Error(MSIM_DEVICE_ERROR, "HIP depth-averaged flow conjugate gradient stalled");
+    if (s.failure != 0) {
+      throw Error(failure_status(s.failure),
+                  std::string("HIP depth-averaged flow conjugate gradient ") +
+                      failure_text(s.failure));
+    }
+    *relative = rr0 > 0.0 ? std::sqrt(std::max(0.0, s.rr)) / std::sqrt(rr0) : 0.0;
+    *converged = s.halt != 0;
+    return *converged;
+  };
+  const PersistShape shape = times == nullptr ? persist_shape<T>(ctx) : PersistShape{0, 0, 0};
+  if (shape.sites != 0 && budget > 0) {
+    // Launches of kPersistIterations, so none runs for more than some tens of
+    // milliseconds; the direction stays in pa.
+    uint32_t taken = 0;
+    while (taken < budget) {
+      const uint32_t batch = std::min(kPersistIterations, budget - taken);
+      if (!launch_persistent<T>(ctx, shape, r, x, pa, batch, taken)) break;
+      read_state(ctx);
+      if (judge(*f.host_state)) return f.host_state->halt;
+      taken += batch;
+    }
+    if (taken >= budget) return budget;
+    if (taken > 0)
+      throw Error(MSIM_DEVICE_ERROR, "HIP depth-averaged flow conjugate gradient was not resumed");
+  }
   uint32_t launched = 0;  // iterations launched
   bool tested_all = false;
   while (true) {
@@ -923,16 +1260,7 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
         times->update_launches += 1;
       }
     }
-    if (s.failure != 0) {
-      throw Error(failure_status(s.failure),
-                  std::string("HIP depth-averaged flow conjugate gradient ") +
-                      failure_text(s.failure));
-    }
-    *relative = rr0 > 0.0 ? std::sqrt(std::max(0.0, s.rr)) / std::sqrt(rr0) : 0.0;
-    if (s.halt != 0) {
-      *converged = true;
-      return s.halt;
-    }
+    if (judge(s)) return s.halt;
     if (tested_all) return budget;
   }
 }

@@ -374,6 +374,12 @@ struct Context {
   CoupledDevice coupled;
   ColonyDevice colony;
   std::shared_ptr<BatchDevice> batch;
+  // Persistent solves (persist.hpp): the rounds' words, the exchanged values'
+  // words and the next tag, and how many workgroups can be resident, one per
+  // compute unit (0: no cooperative launches on this device).
+  DeviceBuffer<uint64_t> round_slots, round_words;
+  uint32_t round_tag = 0;
+  uint32_t resident_blocks = 0;
 };
 
 // Summed event time and launch count of the two Krylov kernels of a solve.
@@ -394,6 +400,12 @@ void launch_assembly(hipStream_t stream, const uint8_t* solid, const float* mobi
 // A ported system: holds each open face at the pressure of its slot in
 // `pressure_host` (FlowEdges layout) and reassembles the right-hand side.
 void flow_hold_pressures(Context& ctx, const float* pressure_host);
+// Persistent solves: reserves `rounds` consecutive tags, returning the first,
+// and `words` words of exchange memory; launches a kernel whose workgroups (kPersistThreads threads each) must all
+// be resident, false where the device has no room for the grid.
+uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words);
+bool launch_resident(Context& ctx, const void* kernel, uint32_t blocks, void** args, size_t lds,
+                     const char* what);
 uint32_t stream_blocks(size_t n);
 uint32_t krylov_blocks(size_t n);
 void launch_residual(Context& ctx, const double* x, double* out, int mode);
