@@ -503,9 +503,9 @@ __global__ __launch_bounds__(kStream) void k_cg_init(const S* __restrict__ sourc
 // 90 MB per FP64 iteration, cache-resident): two launches per iteration, each
 // of whose blocks re-adds the partials first, against two trips of a word to
 // memory and back. Per iteration, the launches and this kernel, on pillar
-// arrays (FP64; FP32): 64x48 15.6 and 3.6 us; 256x128 13.9 and 5.8 us;
-// 512x256 14.9 and 8.7 us; 1024x512 20.1 and 10.8 us (17.4 and 8.9); 1024x1000
-// 27.7 and 16.0 us (23.2 and 11.3). 256 or 1024 threads per workgroup lose
+// arrays (FP64; FP32): 64x48 15.6 and 3.6 us; 256x128 13.9 and 4.3 us;
+// 512x256 14.9 and 6.5 us; 1024x512 20.1 and 10.8 us (17.4 and 8.9); 1024x1000
+// 27.7 and 15.9 us (23.2 and 11.3). 256 or 1024 threads per workgroup lose
 // 5 to 70 % from 512x256 up.
 //
 // Starts from r, x, p, rho and beta as k_cg_init or an earlier launch left
@@ -959,6 +959,19 @@ uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words) {
   return tag;
 }
 
+ResidentShape resident_shape(const Context& ctx, size_t entries, size_t halo, size_t bytes,
+                             size_t lds_limit) {
+  const size_t room = std::min<size_t>(ctx.resident_blocks, kRoundBlocks);
+  for (int s : {1, 2, 4, 8}) {
+    const size_t chunk = static_cast<size_t>(kPersistThreads) * s;
+    const size_t blocks = (entries + chunk - 1) / chunk;
+    const size_t lds = (std::min(chunk, entries) + 2 * halo) * bytes;
+    if (blocks <= (s < 4 ? std::min<size_t>(room, 16) : room) && lds <= lds_limit)
+      return ResidentShape{s, static_cast<uint32_t>(blocks), lds};
+  }
+  return ResidentShape{};
+}
+
 bool launch_resident(Context& ctx, const void* kernel, uint32_t blocks, void** args, size_t lds,
                      const char* what) {
   const hipError_t status = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads),
@@ -1115,36 +1128,17 @@ const char* failure_text(uint32_t failure) {
 }
 
 // Whether Jacobi-PCG of precision T on this system runs as one persistent
-// launch, and its shape: the fewest sites per thread that fit the device's
-// compute units, one workgroup each, with the direction and its halo of ny
-// sites either side in at most 60 KB of LDS. The line is what the registers
-// hold: eight sites per thread (FP64: 255 VGPRs), 1M sites on 256 compute
-// units, where this is still 1.7 (FP64) and 2.1 times (FP32) as fast per
-// iteration as the launches.
-struct PersistShape {
-  int sites;        // per thread; 0: not this way
-  uint32_t blocks;
-  size_t lds;
-};
-
+// launch, and its shape (resident_shape), with the direction and its halo of
+// ny sites either side in at most 60 KB of LDS.
 template <typename T>
-PersistShape persist_shape(const Context& ctx) {
-  const auto& f = ctx.flow;
-  const size_t n = f.sites();
-  for (int s : {1, 2, 4, 8}) {
-    const size_t chunk = static_cast<size_t>(kPersistThreads) * s;
-    const size_t blocks = (n + chunk - 1) / chunk;
-    const size_t lds = (std::min(chunk, n) + 2 * static_cast<size_t>(f.ny)) * sizeof(T);
-    if (blocks <= std::min<size_t>(ctx.resident_blocks, kRoundBlocks) && lds <= 60 * 1024)
-      return PersistShape{s, static_cast<uint32_t>(blocks), lds};
-  }
-  return PersistShape{0, 0, 0};
+ResidentShape persist_shape(const Context& ctx) {
+  return resident_shape(ctx, ctx.flow.sites(), ctx.flow.ny, sizeof(T), 60 * 1024);
 }
 
 // One persistent launch of at most `budget` iterations; false where the
 // device does not take it (too few free compute units for the grid).
 template <typename T>
-bool launch_persistent(Context& ctx, const PersistShape& shape, T* r, T* x, T* p,
+bool launch_persistent(Context& ctx, const ResidentShape& shape, T* r, T* x, T* p,
                        uint32_t budget, uint32_t taken) {
   auto& f = ctx.flow;
   uint32_t n = static_cast<uint32_t>(f.sites()), ny = f.ny;
@@ -1157,7 +1151,7 @@ bool launch_persistent(Context& ctx, const PersistShape& shape, T* r, T* x, T* p
   void* args[] = {&r, &x, &p, &words, &diag, &cxl, &cyl, &bc, &n, &ny, &isx, &isy,
                   &st, &slots, &tag, &budget, &taken};
   const void* kernel = nullptr;
-  switch (shape.sites) {
+  switch (shape.per_thread) {
     case 1: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 1>); break;
     case 2: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 2>); break;
     case 4: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 4>); break;
@@ -1205,8 +1199,8 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
     *converged = s.halt != 0;
     return *converged;
   };
-  const PersistShape shape = times == nullptr ? persist_shape<T>(ctx) : PersistShape{0, 0, 0};
-  if (shape.sites != 0 && budget > 0) {
+  const ResidentShape shape = times == nullptr ? persist_shape<T>(ctx) : ResidentShape{};
+  if (shape.per_thread != 0 && budget > 0) {
     // Launches of kPersistIterations, so none runs for more than some tens of
     // milliseconds; the direction stays in pa.
     uint32_t taken = 0;

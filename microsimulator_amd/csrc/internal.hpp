@@ -400,10 +400,28 @@ void launch_assembly(hipStream_t stream, const uint8_t* solid, const float* mobi
 // A ported system: holds each open face at the pressure of its slot in
 // `pressure_host` (FlowEdges layout) and reassembles the right-hand side.
 void flow_hold_pressures(Context& ctx, const float* pressure_host);
-// Persistent solves: reserves `rounds` consecutive tags, returning the first,
-// and `words` words of exchange memory; launches a kernel whose workgroups (kPersistThreads threads each) must all
-// be resident, false where the device has no room for the grid.
+// The shape of a persistent solve over `entries` entries whose direction, with
+// `halo` entries either side, is held in LDS: 1 or 2 entries per thread while
+// that leaves at most 16 workgroups, else 4, else 8; none (per_thread 0) where
+// the workgroups would not fit the compute units or LDS would pass lds_limit.
+// A round costs 1.2 us among 16 workgroups, 1.9 among 32 and 3.3 to 4.5 among
+// 256, so fewer, fuller workgroups win until their own work does not hide: one
+// FP64 pressure iteration at 256x128 takes 5.8, 5.2, 4.3 and 8.1 us with 1, 2,
+// 4 and 8 sites per thread (64, 32, 16 and 8 workgroups), at 64x48 3.6, 3.8,
+// 4.2 and 7.4. Eight entries fill the registers (FP64: 255 VGPRs), so 1M
+// entries on 256 compute units is the line.
+struct ResidentShape {
+  int per_thread = 0;
+  uint32_t blocks = 0;
+  size_t lds = 0;
+};
+ResidentShape resident_shape(const Context& ctx, size_t entries, size_t halo, size_t bytes,
+                             size_t lds_limit);
+// Reserves `rounds` consecutive tags, returning the first, and `words` words of
+// exchange memory.
 uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words);
+// Launches a kernel whose workgroups (kPersistThreads threads each) must all be
+// resident; false where the device has no room for the grid.
 bool launch_resident(Context& ctx, const void* kernel, uint32_t blocks, void** args, size_t lds,
                      const char* what);
 uint32_t stream_blocks(size_t n);

@@ -31,6 +31,7 @@
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "persist.hpp"
 
 namespace msim {
 namespace {
@@ -447,6 +448,220 @@ __global__ __launch_bounds__(kResBlock) void k_cg_step(ResView V, double* __rest
   }
 }
 
+// The whole momentum CG in one persistent launch (persist.hpp), for grids of
+// at most 1M faces: each workgroup owns kPersistThreads * S consecutive faces,
+// their x, r, z and coefficients in registers, and holds the direction of its
+// faces and of `halo` faces either side (the longest stride of a component's
+// lattice) in LDS. The workgroups meet for p.q, and for r.r and r.z together
+// with z of their faces, from which each forms its neighbours' next direction.
+// The arithmetic per face is k_cg_init's, k_cg_direction's and k_cg_step's;
+// the sums are added in the rounds' order. Also the pressure part of the
+// preconditioner, which is independent.
+//
+// A vector of these grids is 0.1 to 6 MB: the two launches per iteration are
+// bound by launch and by re-adding the partials, this by two trips of a word
+// to memory and back. A whole solve per inner iteration (Arnoldi steps
+// included), with the launches and with this kernel and the Arnoldi columns
+// read a step behind: 24x16x8 18.0 and 8.5 us, 48x24x12 17.7 and 10.5,
+// 64x32x16 19.8 and 12.7, 128x64x32 45.2 and 30.1.
+template <int S>
+__global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
+    ResView V, const double* __restrict__ in, double* __restrict__ out, uint64_t* words,
+    uint64_t* slots, uint32_t tag, uint32_t halo, uint32_t limit, float tolerance,
+    ResState* st) {
+  constexpr int NT = kPersistThreads;
+  constexpr int kAhead = 3;
+  extern __shared__ __align__(16) unsigned char s_raw[];
+  double* s_p = reinterpret_cast<double*>(s_raw);
+  __shared__ RoundLds L;
+  const int t = threadIdx.x;
+  if (t == 0) L.stalled = 0;
+  const uint32_t n = static_cast<uint32_t>(V.nf);
+  const uint32_t start = blockIdx.x * (NT * S);
+  const uint32_t own = min(n - start, static_cast<uint32_t>(NT * S));
+  const Exchange<double> ex{words, n};
+  double xv[S], rv[S], zv[S];
+  float drag[S], diag[S];
+  uint32_t bits[S], sx[S], sy[S];  // neighbour bits | active << 6 | component << 8; strides
+  double sums[2] = {0.0, 0.0};
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const uint32_t l = static_cast<uint32_t>(t + s * NT);
+    xv[s] = rv[s] = zv[s] = 0.0;
+    drag[s] = diag[s] = 0.0f;
+    bits[s] = sx[s] = sy[s] = 0;
+    if (l < own) {
+      const uint32_t f = start + l;
+      const int c = face_component(V, f);
+      uint32_t fd[3] = {V.dims[0], V.dims[1], V.dims[2]};
+      ++fd[c];
+      sx[s] = fd[1] * fd[2];
+      sy[s] = fd[2];
+      bits[s] = V.neighbours[f] | (V.active[f] != 0 ? 64u : 0u) | static_cast<uint32_t>(c) << 8;
+      drag[s] = V.face_drag[f];
+      diag[s] = V.diag[f];
+      rv[s] = static_cast<double>(static_cast<float>(in[f]));
+      zv[s] = diag[s] > 0.0f ? rv[s] / diag[s] : 0.0;
+      s_p[halo + l] = 0.0;
+      ex.put(f, tag, zv[s]);
+      sums[0] += rv[s] * rv[s];
+      sums[1] += rv[s] * zv[s];
+    }
+  }
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * NT + t; i < V.n;
+       i += static_cast<uint64_t>(gridDim.x) * NT) {
+    const float pd = V.pd[i];
+    out[V.nf + i] = pd > 0.0f ? -in[V.nf + i] / (V.cs * static_cast<double>(pd)) : 0.0;
+  }
+  auto halo_site = [&](uint32_t h) -> uint32_t {
+    if (h >= 2 * halo) return n;
+    if (h < halo) return start + h >= halo ? start + h - halo : n;
+    return min(start + own + (h - halo), n);
+  };
+  auto halo_slot = [&](uint32_t h) { return h < halo ? h : own + h; };
+  for (uint32_t h = t; h < 2 * halo; h += NT) s_p[halo_slot(h)] = 0.0;
+  // z of kAhead halo entries of this thread, from h0 on; entries off the
+  // lattice are never loaded.
+  uint64_t w[kAhead][2];
+  uint32_t site_h[kAhead];
+  auto aim = [&](uint32_t h0) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) site_h[u] = halo_site(h0 + static_cast<uint32_t>(u * NT));
+  };
+  auto issue = [&] {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (site_h[u] < n) ex.load(site_h[u], w[u]);
+    }
+  };
+  auto done = [&](uint32_t of) {
+    bool all = true;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      all = all && (site_h[u] >= n || Exchange<double>::has(w[u], of));
+    return all;
+  };
+  auto advance = [&](uint32_t h0, double beta) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (site_h[u] < n) {
+        double& p = s_p[halo_slot(h0 + static_cast<uint32_t>(u * NT))];
+        p = Exchange<double>::value(w[u]) + beta * p;
+      }
+    }
+  };
+  aim(t);
+  bool alive = round_sums<2>(sums, slots, tag, L, issue, [&] { return done(tag); });
+  double rho = sums[1];
+  const double rhs_norm = sqrt(sums[0]);
+  double beta = 0.0, relative = 1.0;
+  uint32_t k = 0, failure = 0;
+  bool met = sums[0] == 0.0;  // x = 0 solves it
+  while (alive && !met && failure == 0 && k < limit) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      if (l < own) s_p[halo + l] = zv[s] + beta * s_p[halo + l];
+    }
+    advance(t, beta);
+    for (uint32_t h0 = t + kAhead * NT; h0 < 2 * halo; h0 += kAhead * NT) {
+      aim(h0);
+      poll_words(L, issue, [&] { return done(tag); });
+      advance(h0, beta);
+    }
+    aim(t);
+    ++tag;
+    __syncthreads();
+    double qv[S];
+    double pq[1] = {0.0};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      qv[s] = 0.0;
+      if (l < own) {
+        const double uf = s_p[halo + l];
+        double q = 0.0;
+        if ((bits[s] & 64u) != 0) {
+          const uint32_t c = bits[s] >> 8;
+          const uint32_t stride[3] = {sx[s], sy[s], 1u};
+          q = static_cast<double>(drag[s]) * uf;
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            if (V.dims[a] == 1) continue;
+            const double mirror = static_cast<uint32_t>(a) == c ? uf : -uf;
+            const double lower =
+                ((bits[s] >> (2 * a)) & 1u) != 0 ? s_p[halo + l - stride[a]] : mirror;
+            const double upper =
+                ((bits[s] >> (2 * a + 1)) & 1u) != 0 ? s_p[halo + l + stride[a]] : mirror;
+            q -= (lower - uf) * V.inv[a];
+            q -= (upper - uf) * V.inv[a];
+          }
+        }
+        qv[s] = q;
+        pq[0] += uf * q;
+      }
+    }
+    alive = round_sums<1>(
+        pq, slots, tag++, L, [] {}, [] { return true; });
+    if (!alive) break;
+    if (!isfinite(pq[0]) || pq[0] <= 0.0) {
+      failure = MSIM_CG_CURVATURE;
+      break;
+    }
+    const double alpha = rho / pq[0];
+    if (!isfinite(alpha)) {
+      failure = MSIM_CG_STEP;
+      break;
+    }
+    sums[0] = sums[1] = 0.0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t l = static_cast<uint32_t>(t + s * NT);
+      if (l < own) {
+        xv[s] += alpha * s_p[halo + l];
+        rv[s] = rv[s] - alpha * qv[s];
+        zv[s] = diag[s] > 0.0f ? rv[s] / diag[s] : 0.0;
+        ex.put(start + l, tag, zv[s]);
+        sums[0] += rv[s] * rv[s];
+        sums[1] += rv[s] * zv[s];
+      }
+    }
+    alive = round_sums<2>(sums, slots, tag, L, issue, [&] { return done(tag); });
+    if (!alive) break;
+    ++k;
+    const double now = sqrt(sums[0] > 0.0 ? sums[0] : 0.0) / rhs_norm;
+    if (!isfinite(now)) {
+      failure = MSIM_CG_RESIDUAL;
+      break;
+    }
+    relative = now;
+    if (relative <= static_cast<double>(tolerance)) {
+      met = true;
+    } else if (k < limit) {
+      if (!isfinite(sums[1]) || rho == 0.0) {
+        failure = MSIM_CG_BREAKDOWN;
+      } else {
+        beta = sums[1] / rho;
+        if (!isfinite(beta)) failure = MSIM_CG_DIRECTION;
+      }
+    }
+    rho = sums[1];
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const uint32_t l = static_cast<uint32_t>(t + s * NT);
+    if (l < own) out[start + l] = xv[s];
+  }
+  if (lead()) {
+    st->iterations = k;
+    st->relative = relative;
+    st->stop1 = met || failure != 0 ? 1u : 0u;
+    st->stop2 = 0;
+    st->failure1 = alive ? failure : MSIM_DEVICE_ERROR;
+    st->failure2 = 0;
+  }
+}
+
 // The pressure part of the preconditioner (cpu_flow.cpp:424-431):
 // out = -in / (cs pd) where pd > 0, else 0.
 __global__ __launch_bounds__(kResBlock) void k_res_pressure_precondition(
@@ -571,6 +786,17 @@ __global__ __launch_bounds__(kResBlock) void k_res_scaled(uint64_t n, double* __
                                                           double s, const double* __restrict__ in) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kResBlock + threadIdx.x;
   if (i < n) out[i] = 0.0 + s * in[i];
+}
+
+// The next basis vector, w / |w| with |w|^2 at `square` (zero where |w| is at
+// most 1e-14: the space is exhausted).
+__global__ __launch_bounds__(kResBlock) void k_res_normalise(uint64_t n, double* __restrict__ out,
+                                                             const double* square,
+                                                             const double* __restrict__ w) {
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kResBlock + threadIdx.x;
+  const double norm = sqrt(*square);
+  const double s = norm <= 1e-14 ? 0.0 : 1 / norm;
+  if (i < n) out[i] = 0.0 + s * w[i];
 }
 
 // r = rhs + (-1) * w.
@@ -802,6 +1028,11 @@ uint32_t min_gap(const ResSystem& s) {
   return shortest;
 }
 
+// Doubles of an Arnoldi column in the device's slots.
+constexpr size_t kColumn = 2 + 2 * kRestart;
+constexpr size_t kColumnSlots = kColumn + sizeof(ResState) / sizeof(double);
+static_assert(sizeof(ResState) % sizeof(double) == 0);
+
 // Device state of one solve.
 struct ResDevice {
   ResView V{};
@@ -811,7 +1042,29 @@ struct ResDevice {
   // cg_p holds two direction buffers (iterations alternate between them).
   DeviceBuffer<double> rhs, x, r, w, basis, directions, cg_r, cg_z, cg_p, cg_q, cg_parts,
       partials, slots;
-  DeviceBuffer<ResState> state;
+  // Two Arnoldi columns (by the step's parity) in `slots`, each with the state
+  // of its momentum solve, pinned host copies of them and their events.
+  double* host_columns = nullptr;
+  hipEvent_t column_read[2] = {nullptr, nullptr};
+  ResDevice() = default;
+  ResDevice(const ResDevice&) = delete;
+  ResDevice& operator=(const ResDevice&) = delete;
+  ~ResDevice() {
+    if (host_columns != nullptr) static_cast<void>(hipHostFree(host_columns));
+    for (hipEvent_t e : column_read) {
+      if (e != nullptr) static_cast<void>(hipEventDestroy(e));
+    }
+  }
+  [[nodiscard]] double* column(uint32_t step) const {
+    return slots.data() + (step & 1u) * kColumnSlots;
+  }
+  [[nodiscard]] ResState* state(uint32_t step) const {
+    return reinterpret_cast<ResState*>(column(step) + kColumn);
+  }
+  // The momentum CG as one persistent launch (no shape: two launches per
+  // iteration), its halo of faces.
+  ResidentShape persist;
+  uint32_t persist_halo = 0;
   // Iterations the last momentum solve took: the next solve's first batch.
   uint32_t cg_expect = 16;
 };
@@ -839,6 +1092,52 @@ double read_scalar(Context& ctx, const double* slot) {
   return v;
 }
 
+// What a momentum solve's state says: adds its iterations, throws its failure.
+void judge_momentum(ResDevice& D, const ResState& s, uint64_t& inner) {
+  inner += s.iterations;
+  D.cg_expect = s.iterations;
+  const std::string label = "resolved-flow momentum conjugate gradient ";
+  switch (s.failure1 != 0 ? s.failure1 : s.failure2) {
+    case MSIM_CG_CURVATURE:
+      throw Error(MSIM_CG_CURVATURE, label + "encountered non-positive curvature");
+    case MSIM_CG_STEP: throw Error(MSIM_CG_STEP, label + "produced a non-finite step");
+    case MSIM_CG_RESIDUAL: throw Error(MSIM_CG_RESIDUAL, label + "produced a non-finite residual");
+    case MSIM_CG_BREAKDOWN:
+      throw Error(MSIM_CG_BREAKDOWN, label + "encountered a preconditioner breakdown");
+    case MSIM_CG_DIRECTION:
+      throw Error(MSIM_CG_DIRECTION, label + "produced a non-finite direction");
+    case MSIM_DEVICE_ERROR: throw Error(MSIM_DEVICE_ERROR, label + "stalled");
+    default: break;
+  }
+  if (s.stop1 == 0 && s.stop2 == 0) {
+    throw Error(MSIM_NOT_CONVERGED,
+                label + "did not converge: relative " + std::to_string(s.relative));
+  }
+}
+
+// The preconditioner by one persistent launch, on grids that fit and up to
+// kMomentumLimit iterations (one launch takes them all: well under a second);
+// false where it is not taken.
+constexpr uint32_t kMomentumLimit = 1u << 16;
+
+bool precondition_persistent(Context& ctx, ResDevice& D, const double* in, double* out,
+                             float tolerance, uint32_t max_iterations, ResState* state) {
+  if (D.persist.per_thread == 0 || max_iterations == 0 || max_iterations > kMomentumLimit) return false;
+  uint32_t tag = take_rounds(ctx, 2 * max_iterations + 1, 2 * D.V.nf);
+  uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
+  void* args[] = {&D.V,  &in,  &out,           &words,          &slots,
+                  &tag,  &D.persist_halo,      &max_iterations, &tolerance, &state};
+  const void* kernel = nullptr;
+  switch (D.persist.per_thread) {
+    case 1: kernel = reinterpret_cast<const void*>(&k_cg_momentum<1>); break;
+    case 2: kernel = reinterpret_cast<const void*>(&k_cg_momentum<2>); break;
+    case 4: kernel = reinterpret_cast<const void*>(&k_cg_momentum<4>); break;
+    default: kernel = reinterpret_cast<const void*>(&k_cg_momentum<8>); break;
+  }
+  return launch_resident(ctx, kernel, D.persist.blocks, args, D.persist.lds,
+                         "launch k_cg_momentum");
+}
+
 // The momentum block by Jacobi-PCG from zero (conjugate_gradient,
 // cpu_flow.cpp:53-103) on rhs (FP64, rounded to float as the reference
 // rounds it): the solution into `out`. Adds the iterations to `inner`. Two
@@ -851,7 +1150,7 @@ void momentum_cg(Context& ctx, ResDevice& D, const double* rhs, double* out, flo
   const ResView& V = D.V;
   const uint32_t blocks = chunks_of(V.nf, V.cg_faces * kResBlock);
   const CgParts P{D.cg_parts.data(), blocks};
-  ResState* st = D.state.data();
+  ResState* st = D.state(0);
   double* const p[2] = {D.cg_p.data(), D.cg_p.data() + V.nf};
   k_cg_init<<<blocks, kResBlock, 0, ctx.stream>>>(V, rhs, out, D.cg_r.data(), D.cg_z.data(), P,
                                                   st);
@@ -903,24 +1202,7 @@ void momentum_cg(Context& ctx, ResDevice& D, const double* rhs, double* out, flo
     check(hipStreamSynchronize(ctx.stream), "momentum CG");
     if (s.stop1 != 0 || s.stop2 != 0 || k >= max_iterations) break;
   }
-  inner += s.iterations;
-  D.cg_expect = s.iterations;
-  const std::string label = "resolved-flow momentum conjugate gradient ";
-  switch (s.failure1 != 0 ? s.failure1 : s.failure2) {
-    case MSIM_CG_CURVATURE:
-      throw Error(MSIM_CG_CURVATURE, label + "encountered non-positive curvature");
-    case MSIM_CG_STEP: throw Error(MSIM_CG_STEP, label + "produced a non-finite step");
-    case MSIM_CG_RESIDUAL: throw Error(MSIM_CG_RESIDUAL, label + "produced a non-finite residual");
-    case MSIM_CG_BREAKDOWN:
-      throw Error(MSIM_CG_BREAKDOWN, label + "encountered a preconditioner breakdown");
-    case MSIM_CG_DIRECTION:
-      throw Error(MSIM_CG_DIRECTION, label + "produced a non-finite direction");
-    default: break;
-  }
-  if (s.stop1 == 0 && s.stop2 == 0) {
-    throw Error(MSIM_NOT_CONVERGED,
-                label + "did not converge: relative " + std::to_string(s.relative));
-  }
+  judge_momentum(D, s, inner);
 }
 
 void apply_system(Context& ctx, ResDevice& D, const double* in, double* out) {
@@ -928,11 +1210,15 @@ void apply_system(Context& ctx, ResDevice& D, const double* in, double* out) {
   check(hipGetLastError(), "launch k_res_apply");
 }
 
-void precondition(Context& ctx, ResDevice& D, const double* in, double* out, float tolerance,
-                  uint32_t max_iterations, uint64_t& inner) {
+// The preconditioner; true where the momentum solve's state is still to be
+// judged once the device has it (judge_momentum).
+bool precondition(Context& ctx, ResDevice& D, const double* in, double* out, float tolerance,
+                  uint32_t max_iterations, ResState* state, uint64_t& inner) {
+  if (precondition_persistent(ctx, D, in, out, tolerance, max_iterations, state)) return true;
   momentum_cg(ctx, D, in, out, tolerance, max_iterations, inner);
   k_res_pressure_precondition<<<grid_of(D.V.n), kResBlock, 0, ctx.stream>>>(D.V, in, out);
   check(hipGetLastError(), "launch k_res_pressure_precondition");
+  return false;
 }
 
 // The device arrays of a built system, and the buffers of its solves.
@@ -981,9 +1267,21 @@ void setup_device(Context& ctx, const ResSystem& S, ResDevice& D) {
   D.cg_p.reserve(2 * S.nf);
   D.cg_parts.reserve(5 * static_cast<size_t>(chunks_of(S.nf, V.cg_faces * kResBlock)));
   D.partials.reserve((kRestart + 1) * static_cast<size_t>(chunks_of(m, V.chunk)));
-  // slots: [0] the last norm, [1 + 2 * i + pass] the Arnoldi projections.
-  D.slots.reserve(2 + 2 * kRestart + 2);
-  D.state.reserve(1);
+  // A column: [0] the norm, [1 ..] and [1 + kRestart ..] the Arnoldi
+  // projections of the two passes, [kColumn ..] the momentum solve's state.
+  D.slots.reserve(2 * kColumnSlots);
+  void* columns = nullptr;
+  check(hipHostMalloc(&columns, 2 * kColumnSlots * sizeof(double), hipHostMallocDefault),
+        "hipHostMalloc");
+  D.host_columns = static_cast<double*>(columns);
+  for (hipEvent_t& e : D.column_read)
+    check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+  for (int a = 0; a < 3; ++a) {
+    uint32_t fd[3] = {S.dims[0], S.dims[1], S.dims[2]};
+    ++fd[a];
+    D.persist_halo = std::max(D.persist_halo, fd[1] * fd[2]);
+  }
+  D.persist = resident_shape(ctx, S.nf, D.persist_halo, sizeof(double), 80 * 1024);
 }
 
 // One block solve (solve_resolved_system, cpu_flow.cpp:379-461): flexible
@@ -1040,36 +1338,48 @@ BlockSolve block_solve(Context& ctx, ResDevice& D, const std::vector<double>& rh
       double* directions = D.directions.data();
       k_res_scaled<<<grid_of(m), kResBlock, 0, ctx.stream>>>(m, basis, 1 / beta, D.r.data());
       uint32_t used = 0;
-      for (uint32_t j = 0; j < count; ++j) {
+      bool pending = false;  // the steps' momentum solves are judged from their columns
+      // Enqueues step j whole: the host is not needed for the next basis vector.
+      auto enqueue = [&](uint32_t j) {
         double* direction = directions + static_cast<size_t>(j) * m;
         const double* vj = basis + static_cast<size_t>(j) * m;
-        precondition(ctx, D, vj, direction, inner_tolerance, max_inner, out.inner);
+        double* column = D.column(j);
+        pending = precondition(ctx, D, vj, direction, inner_tolerance, max_inner, D.state(j),
+                               out.inner);
         apply_system(ctx, D, direction, D.w.data());
-        // Classical Gram-Schmidt twice, every scalar on the device: the
-        // first pass's coefficients at slot[1 ..], the second's at
-        // slot[1 + kRestart ..], the norm of what remains at slot[0].
-        {
-          const uint32_t blocks = chunks_of(m, V.chunk);
-          const uint32_t count = j + 1;
-          double* h1 = slot + 1;
-          double* h2 = slot + 1 + kRestart;
-          double* parts = D.partials.data();
-          k_res_multidot<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, count,
-                                                               D.w.data(), parts);
-          k_res_multisum<<<count, kResBlock, 0, ctx.stream>>>(parts, blocks, h1);
-          k_res_cgs<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, count, h1,
-                                                          D.w.data(), 0, parts);
-          k_res_multisum<<<count, kResBlock, 0, ctx.stream>>>(parts, blocks, h2);
-          k_res_cgs<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, count, h2,
-                                                          D.w.data(), 1, parts);
-          k_res_sum<<<1, kResBlock, 0, ctx.stream>>>(parts, blocks, slot);
-          check(hipGetLastError(), "launch Gram-Schmidt");
-        }
-        std::vector<double> col(1 + 2 * kRestart);
-        check(hipMemcpyAsync(col.data(), slot, col.size() * sizeof(double),
-                             hipMemcpyDeviceToHost, ctx.stream),
+        // Classical Gram-Schmidt twice, every scalar on the device.
+        const uint32_t blocks = chunks_of(m, V.chunk);
+        const uint32_t dots = j + 1;
+        double* h1 = column + 1;
+        double* h2 = column + 1 + kRestart;
+        double* parts = D.partials.data();
+        k_res_multidot<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, dots, D.w.data(),
+                                                             parts);
+        k_res_multisum<<<dots, kResBlock, 0, ctx.stream>>>(parts, blocks, h1);
+        k_res_cgs<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, dots, h1, D.w.data(),
+                                                        0, parts);
+        k_res_multisum<<<dots, kResBlock, 0, ctx.stream>>>(parts, blocks, h2);
+        k_res_cgs<<<blocks, kResBlock, 0, ctx.stream>>>(m, V.chunk, basis, dots, h2, D.w.data(),
+                                                        1, parts);
+        k_res_sum<<<1, kResBlock, 0, ctx.stream>>>(parts, blocks, column);
+        k_res_normalise<<<grid_of(m), kResBlock, 0, ctx.stream>>>(
+            m, basis + static_cast<size_t>(j + 1) * m, column, D.w.data());
+        check(hipGetLastError(), "launch Arnoldi step");
+        check(hipMemcpyAsync(D.host_columns + (j & 1u) * kColumnSlots, column,
+                             kColumnSlots * sizeof(double), hipMemcpyDeviceToHost, ctx.stream),
               "read Arnoldi column");
-        check(hipStreamSynchronize(ctx.stream), "Arnoldi step");
+        check(hipEventRecord(D.column_read[j & 1u], ctx.stream), "event");
+      };
+      // Takes step j's column into the least-squares problem; true where the
+      // cycle ends with it.
+      auto take = [&](uint32_t j, bool judge) {
+        check(hipEventSynchronize(D.column_read[j & 1u]), "Arnoldi step");
+        const double* col = D.host_columns + (j & 1u) * kColumnSlots;
+        if (judge) {
+          ResState state{};
+          std::memcpy(&state, col + kColumn, sizeof(state));
+          judge_momentum(D, state, out.inner);
+        }
         for (uint32_t i = 0; i <= j; ++i) {
           h[i][j] += col[1 + i];
           h[i][j] += col[1 + kRestart + i];
@@ -1079,9 +1389,6 @@ BlockSolve block_solve(Context& ctx, ResDevice& D, const std::vector<double>& rh
           throw Error(MSIM_RUNTIME_ERROR, "FGMRES non-finite Arnoldi vector");
         }
         const bool happy = h[j + 1][j] <= 1e-14;
-        double* next = basis + static_cast<size_t>(j + 1) * m;
-        k_res_scaled<<<grid_of(m), kResBlock, 0, ctx.stream>>>(
-            m, next, happy ? 0.0 : 1 / h[j + 1][j], D.w.data());
         for (uint32_t i = 0; i < j; ++i) {
           const double upper = cosine[i] * h[i][j] + sine[i] * h[i + 1][j];
           h[i + 1][j] = -sine[i] * h[i][j] + cosine[i] * h[i + 1][j];
@@ -1097,8 +1404,20 @@ BlockSolve block_solve(Context& ctx, ResDevice& D, const std::vector<double>& rh
         gv[j] *= cosine[j];
         ++iterations;
         used = j + 1;
-        if (happy || std::abs(gv[j + 1]) <= tolerance * rhs_norm) break;
+        return happy || std::abs(gv[j + 1]) <= tolerance * rhs_norm;
+      };
+      // A step's column is read while the next step runs: where the cycle ends
+      // with it, that step's vectors and counts are dropped (one of some 300
+      // us; waiting for each column left the device idle 45 us a step).
+      // Momentum solves whose state the host reads itself cannot run ahead.
+      bool ended = false;
+      for (uint32_t j = 0; j < count && !ended; ++j) {
+        const bool ahead = pending;
+        enqueue(j);
+        if (ahead) ended = take(j - 1, true);
+        if (!ended && !pending) ended = take(j, false);
       }
+      if (pending && !ended) take(count - 1, true);
       std::vector<double> weights(used);
       for (uint32_t i = used; i-- > 0;) {
         double value = gv[i];

@@ -1,5 +1,7 @@
 """Jacobi-PCG as one persistent launch (small and medium systems) against the
-same iteration as two launches each, which a profiled solve takes.
+same iteration as two launches each: the pressure's, which a profiled solve
+takes by launches, and the resolved flow's momentum solves, which take launches
+where more than 65536 iterations are allowed.
 
 Both stop on the same test of the same recurrence and differ in the order of
 their FP64 sums only, so the iteration counts agree within the reference's own
@@ -83,3 +85,33 @@ def test_persistent_resumes_and_stops_at_its_budget():
                     solve(hip, msa.SOLVER_JACOBI_FP64, 1e-8, profile, budget)
         rep2, faces2 = solve(hip, msa.SOLVER_JACOBI_FP64, 1e-8, False)
         assert rep2.iterations == rep.iterations and np.array_equal(faces2, faces)
+
+
+# Faces per workgroup are 512, 1024, 2048 or 4096 by the count; the halo is a
+# plane of the lattice either side, here also more than a workgroup's faces.
+@pytest.mark.parametrize("dims,tolerance", [
+    ((5, 4, 3), 1e-6), ((1, 6, 5), 1e-6), ((12, 9, 7), 1e-6), ((20, 15, 11), 1e-6),
+    ((7, 40, 30), 1e-6), ((40, 20, 18), 1e-5), ((3, 60, 61), 1e-6), ((72, 50, 49), 1e-2),
+])
+def test_momentum_persistent_matches_launches(dims, tolerance):
+    rng = np.random.default_rng(sum(dims))
+    solid = (rng.random(dims) < 0.06).astype(np.uint8)
+    solid[0] = solid[-1] = 0
+    grid = msa.Grid(*dims, 1.0, 0.9, 1.1, solid.reshape(-1))
+    drag = (rng.random(dims) * 2.0).astype(np.float32).reshape(-1)
+    out = []
+    with msa.HipBackend(0) as hip:
+        for most in (50_000, 100_000):
+            field, rep = hip.solve_resolved_flow(grid, drag, msa.ResolvedFlowParameters(
+                mean_inlet_speed=1.0, axis=0, relative_tolerance=tolerance,
+                max_outer_iterations=4000, max_inner_iterations=most))
+            out.append((field.concatenated(), rep))
+    (faces, rep), (expected, ref) = out
+    # The same FP64 recurrences with their sums in another order: an inner
+    # solve may stop one iteration apart, an outer cycle one step.
+    assert abs(rep.outer_iterations - ref.outer_iterations) <= 1
+    assert abs(rep.inner_iterations - ref.inner_iterations) <= 2 + ref.inner_iterations // 100
+    # 1e-6 for what the stopping test leaves at 1e-6, in proportion above it
+    # (at equal counts the two differ by rounding only, 1e-7 of FP32 faces).
+    bound = 1e-6 if rep.outer_iterations == ref.outer_iterations else 30 * tolerance
+    assert np.abs(faces - expected).max() <= bound * np.abs(expected).max()
