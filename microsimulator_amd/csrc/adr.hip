@@ -34,9 +34,9 @@ constexpr int kAdrBlock = 256;
 
 // The ledger of a step lives as per-block partial sums (mass after, boundary
 // supply rate, uptake rate, for each signal) in two generations by step
-// parity. Blocks j < 3S of the next step add partial j of the previous step
-// (in a fixed order) into its ledger row, so no grid-wide fence is needed; a
-// last small launch adds the final step's.
+// parity. 3S further blocks of the next step's launch each add one partial of
+// the previous step (in a fixed order) into its ledger row, so no grid-wide
+// fence is needed; a last small launch adds the final step's.
 struct LedgerParts {
   double* parts;   // [2][3 * kMaxSignals][blocks]
   double* ledger;  // [steps][S][4]
@@ -84,306 +84,314 @@ __device__ inline void block_sums(double (&v)[K], double* lds) {
   }
 }
 
-// What one thread holds of one x-row of its column: the S levels and the
-// mask; for sites the block updates also the faces, occupancy and (with
-// affine reactions) the rates.
+// What one lane holds of one x-row of its column: the S levels and what of
+// the site a face next to it needs (kOpen: a flux may cross it; kLimit: the
+// limited correction may read it); for sites the wave updates also the
+// velocities of the site's lower faces, the occupancy and (with affine
+// reactions) the rates. Beyond a fixed face stands a ghost site, open and
+// holding the reservoir's level; beyond a closed face a site that is neither.
+constexpr uint32_t kOpen = 1, kLimit = 2;
+
 template <typename T, int S, bool kAffine>
 struct AdrRow {
   T c[S];
   float src[kAffine ? S : 1], los[kAffine ? S : 1];
-  float xf, ylo, yhi, phi;
-  bool solid;
+  float ux, uy, phi;
+  uint32_t site;
 };
 
-// One forward-Euler step for S signals, marching: a block owns a strip of
-// TY - 2H columns and `rows` x-rows and walks x, so each level is read from
-// memory once and its x neighbours come from registers, its y neighbours from
-// a row in LDS. H = 1 for the upwind scheme, 2 under van Leer (whose
-// correction reads the site two away). The strip's first and last H threads
-// only load the columns just outside it (or, on a periodic y boundary, the
-// partner columns), so no thread holds more than its own column. The next
-// row's loads are issued one row ahead.
+// A value from the lane below or above (columns col - 1, col + 1); lanes 0
+// and 63 get zero from beyond the wave.
+__device__ inline float lane_below(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ inline float lane_above(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+template <int kControl>
+__device__ inline double lane_shift(double v) {
+  const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(v));
+  const uint32_t lo = static_cast<uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), kControl, 0xf, 0xf, true));
+  const uint32_t hi = static_cast<uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), kControl, 0xf, 0xf, true));
+  return __longlong_as_double(
+      static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+__device__ inline double lane_below(double v) { return lane_shift<0x138>(v); }
+__device__ inline double lane_above(double v) { return lane_shift<0x130>(v); }
+
+// One forward-Euler step for S signals, marching: each wave owns a strip of
+// 64 - 2H columns and `rows` x-rows and walks x on its own, one column per
+// lane, so each level is read from memory once; its x neighbours come from
+// registers and its y neighbours from the next lanes (H = 1 for the upwind
+// scheme, 2 under van Leer, whose correction reads the site two away: the
+// strip's first and last H lanes only hold the columns outside it, their
+// periodic partners or their ghosts). The next row's loads are issued a row
+// ahead.
+//  * Every face's flux (and limited correction) is computed once: the upper
+//    x face's is kept for the next row, the upper y face's comes from the
+//    lane above. The two sites of a face have the same expression for it, so
+//    this changes no bit.
 //  * T = float: the reference's per-site rate in its float order
-//    (fe_update_f32), so every site matches its CPU step bit for bit.
-//  * T = double: face-flux form, each face flux (with its limited
-//    correction) one expression of the sites around it, so what leaves one
-//    site enters the other bit for bit; the step's mass, boundary supply and
-//    uptake go to the ledger partials.
+//    (signals.cpp:1145-1291, 305-320, 1109-1134; transport_rate_f32 and
+//    fe_update_f32 spell it out), so every site matches its CPU step.
+//  * T = double: face-flux form; the step's mass, boundary supply and uptake
+//    go to the ledger partials.
 // A site whose update is non-finite, or negative under upwind, raises a flag
 // (the reference throws, signals.cpp:1119-1131); the step is then refused as
 // a whole. Under van Leer each block also leaves the largest level it wrote,
-// for the settle that follows.
-// Least waves per SIMD asked of the step kernel: four for the FP64 upwind
-// step without an affine reaction, which fits 128 VGPRs without spills once
-// its ledger sums live in LDS (three waves otherwise, at 131); 1 (no demand)
-// for the forms that would spill.
-template <typename T, int S, bool kAffine, bool kLimited>
-constexpr int step_waves() {
-  return sizeof(T) == 8 && !kAffine && !kLimited && S <= 3 ? 4 : 1;
-}
-
-template <typename T, int S, int TY, bool kAffine, bool kLimited, bool kPatched>
-__global__ __launch_bounds__(TY) __attribute__((amdgpu_waves_per_eu(step_waves<T, S, kAffine, kLimited>()))) void k_adr_step(
+// and flags[2] says whether any was negative, for the settle that follows.
+// The step was bound by instructions and barriers, not memory: every face
+// computed from both sides with a branch per case, an LDS row and a barrier
+// per x-row. 4096x2048, three signals with Monod, before and after: FP64
+// upwind 161 and 130 us (3.9 TB/s of its 61 B per site), FP32 upwind 86 and 74
+// us (4.2 TB/s), FP32 van Leer with its settle 207 and 109 us; 1531x769, two
+// signals, FP32 van Leer 40.5 and 20.8 us.
+template <typename T, int S, bool kAffine, bool kLimited, bool kPatched>
+__global__ __launch_bounds__(kAdrBlock) void k_adr_step(
     AdrParams P, const uint8_t* __restrict__ solid, const float* __restrict__ xf,
     const float* __restrict__ yf, const float* __restrict__ phi, const float* __restrict__ source,
     const float* __restrict__ loss, const T* __restrict__ in, T* __restrict__ out, float dt,
-    uint32_t* flags, uint32_t step, uint32_t rows, LedgerParts L, double* largest) {
+    uint32_t* flags, uint32_t step, uint32_t rows, uint32_t strips, LedgerParts L,
+    double* largest) {
   constexpr bool kF64 = sizeof(T) == 8;
   constexpr int kHalo = kLimited ? 2 : 1;
-  constexpr int kWidth = TY - 2 * kHalo;
+  constexpr int kWidth = kWave - 2 * kHalo;
+  constexpr int kWaves = kAdrBlock / kWave;
   using Row = AdrRow<T, S, kAffine>;
-  __shared__ T s_c[2][S][TY];
-  __shared__ uint8_t s_s[2][TY];
-  __shared__ double s_red[(kF64 ? 3 * S : 1) * (TY / kWave)];
+  __shared__ double s_red[(kF64 ? 3 * S : 1) * kWaves];
   // An earlier step failed: the run stops there. (flags[1] holds the first
   // failed step; a failure of this step may be seen here half-published, and
   // then the previous step's ledger row is still folded, as it is valid.)
   if (flags[0] != 0 && flags[1] < step) return;
   if constexpr (kF64) {
-    if (step > 0 && blockIdx.x < 3 * S) fold_ledger<S, TY>(P, L, step - 1, dt, blockIdx.x, s_red);
+    // The blocks past the walking ones add the previous step's ledger.
+    if (blockIdx.x >= L.blocks) {
+      if (step > 0)
+        fold_ledger<S, kAdrBlock>(P, L, step - 1, dt, blockIdx.x - L.blocks, s_red);
+      return;
+    }
   }
   if (flags[0] != 0) return;  // this step already failed elsewhere
   const uint32_t nx = P.nx, ny = P.ny;
   const size_t n = static_cast<size_t>(nx) * ny;
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const uint32_t strips = (ny + kWidth - 1) / kWidth;
-  const uint32_t x0 = (tile / strips) * rows, x1 = min(nx, x0 + rows);
-  const uint32_t t = threadIdx.x;
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t walk = __builtin_amdgcn_readfirstlane(
+      xcd_tile(blockIdx.x, L.blocks) * kWaves + threadIdx.x / kWave);
+  const int xa = static_cast<int>(min(nx, (walk / strips) * rows));
+  const int xb = static_cast<int>(min(nx, static_cast<uint32_t>(xa) + rows));
   const bool xper = P.kind[0] == MSIM_PERIODIC, yper = P.kind[2] == MSIM_PERIODIC;
-  // Column of this thread; columns off the grid stand for the periodic
-  // partner columns.
-  const int col = static_cast<int>((tile % strips) * kWidth + t) - kHalo;
-  int src_col = col;
-  if (col < 0) src_col = yper ? col + static_cast<int>(ny) : -1;
-  if (col >= static_cast<int>(ny)) src_col = yper ? col - static_cast<int>(ny) : -1;
-  if (src_col < 0 || src_col >= static_cast<int>(ny)) src_col = -1;
-  const bool loads = src_col >= 0;
-  const bool owns = t >= kHalo && t < kHalo + kWidth && col >= 0 && col < static_cast<int>(ny);
-  const uint32_t y = static_cast<uint32_t>(src_col);
   const bool field = P.has_field != 0, monod = P.has_monod != 0;
-  // Row xx of the walk (xx in [-H, nx + H - 1]); rows off the grid are the
-  // periodic partners when the x boundary is periodic and absent otherwise.
-  // `full` rows are the ones the block updates.
+  // This lane's column; off the grid the periodic partner's, a ghost of the
+  // fixed face next to it, or nothing.
+  const int col = static_cast<int>((walk % strips) * kWidth) + lane - kHalo;
+  const bool on_y = col >= 0 && col < static_cast<int>(ny);
+  int src_col = col;
+  if (!on_y && yper) src_col = col < 0 ? col + static_cast<int>(ny) : col - static_cast<int>(ny);
+  const bool loads =
+      src_col >= 0 && src_col < static_cast<int>(ny) && (on_y || (yper && ny > 1));
+  const int ghost_y = ny == 1 ? -1
+                      : col == -1 && P.kind[2] == MSIM_FIXED ? 2
+                      : col == static_cast<int>(ny) && P.kind[3] == MSIM_FIXED ? 3
+                                                                               : -1;
+  const bool limits_y = on_y || ny >= 3;  // a periodic partner, for the limiter
+  const bool owns = on_y && lane >= kHalo && lane < kHalo + kWidth;
+  const uint32_t y = static_cast<uint32_t>(src_col);
+  // Row xx of the walk, xx in [-H, nx + H - 1]; `full` rows are the ones the
+  // wave updates.
   auto load = [&](int xx, bool full) {
     Row w{};
+    const bool on_x = xx >= 0 && xx < static_cast<int>(nx);
+    if (field && owns && xx >= 0 && xx <= static_cast<int>(nx))
+      w.ux = xf[static_cast<size_t>(xx) * ny + y];
     int row = xx;
-    if (xx < 0) row = xper ? xx + static_cast<int>(nx) : -1;
-    if (xx >= static_cast<int>(nx)) row = xper ? xx - static_cast<int>(nx) : -1;
-    if (row >= static_cast<int>(nx)) row = -1;
-    if (owns && field && xx >= 0 && xx <= static_cast<int>(nx)) {
-      w.xf = xf[static_cast<size_t>(xx) * ny + y];  // lower x face of row xx
-    }
-    if (row < 0 || !loads) return w;
-    const size_t i = static_cast<size_t>(row) * ny + y;
-    w.solid = solid[i] != 0;
+    if (!on_x) {
+      if (xper && nx > 1) {
+        row = xx < 0 ? xx + static_cast<int>(nx) : xx - static_cast<int>(nx);
+      } else {
+        const int face = xx == -1 ? 0 : xx == static_cast<int>(nx) ? 1 : -1;
+        if (nx > 1 && on_y && face >= 0 && P.kind[face] == MSIM_FIXED) {
+          w.site = kOpen;
 #pragma unroll
-    for (int s = 0; s < S; ++s) w.c[s] = in[s * n + i];
-    if (!full || !owns) return w;
-    if (field) {
-      const size_t yfi = static_cast<size_t>(row) * (ny + 1) + y;
-      w.ylo = yf[yfi];
-      w.yhi = yf[yfi + 1];
-    }
-    if (monod) w.phi = phi[i];
-    if constexpr (kAffine) {
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        w.src[s] = source[s * n + i];
-        w.los[s] = loss[s * n + i];
+          for (int s = 0; s < S; ++s)
+            w.c[s] = static_cast<T>(reservoir<kPatched>(P, face, s, y));
+        }
+        return w;
       }
     }
+    if (row < 0 || row >= static_cast<int>(nx)) return w;
+    if (loads) {
+      const size_t i = static_cast<size_t>(row) * ny + y;
+      const uint32_t limit = limits_y && (on_x || nx >= 3) ? kOpen | kLimit : kOpen;
+      w.site = solid[i] != 0 ? 0u : limit;
+#pragma unroll
+      for (int s = 0; s < S; ++s) w.c[s] = in[s * n + i];
+      if (full && owns) {
+        if (monod) w.phi = phi[i];
+        if constexpr (kAffine) {
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            w.src[s] = source[s * n + i];
+            w.los[s] = loss[s * n + i];
+          }
+        }
+      }
+    } else if (ghost_y >= 0 && on_x) {
+      w.site = kOpen;
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        w.c[s] = static_cast<T>(reservoir<kPatched>(P, ghost_y, s, static_cast<uint32_t>(row)));
+    }
+    if (full && field && col >= 0 && col <= static_cast<int>(ny))
+      w.uy = yf[static_cast<size_t>(row) * (ny + 1) + static_cast<uint32_t>(col)];
     return w;
   };
-  // FP64 ledger sums (mass after, supply, uptake per signal), one slot per
-  // thread in LDS: kept in registers they would take 24 VGPRs and hold the
-  // step at three waves per SIMD instead of four.
-  __shared__ double s_acc[kF64 ? 3 * S : 1][TY];
-  if constexpr (kF64) {
-#pragma unroll
-    for (int k = 0; k < 3 * S; ++k) s_acc[k][threadIdx.x] = 0.0;
-  }
+  // What crosses a face from the lower site (level a) to the upper one (b):
+  // FP64 the flux, FP32 its advective part (the diffusive one is the site's)
+  // and, under van Leer, the correction; zero where the face is closed.
+  struct Face {
+    T flux;
+    T extra;  // FP32 van Leer
+  };
+  const T ihx = T(1) / static_cast<T>(P.dx), ihy = T(1) / static_cast<T>(P.dy);
+  auto face = [&](T a, T b, float velocity, int s, T ih, bool open, [[maybe_unused]] T far_a,
+                  [[maybe_unused]] T far_b, [[maybe_unused]] uint32_t lim,
+                  [[maybe_unused]] uint32_t lim_a, [[maybe_unused]] uint32_t lim_b) {
+    const T u = static_cast<T>(velocity);
+    const bool forward = u >= T(0);
+    T f = u * (forward ? a : b);
+    if constexpr (kF64) f -= static_cast<T>(P.diffusion[s]) * (b - a) * ih;
+    T extra = T(0);
+    if constexpr (kLimited) {
+      const T inc = van_leer_increment<T>(forward ? a : b, forward ? b : a,
+                                          forward ? far_a : far_b);
+      const bool corrected = (lim & (forward ? lim_a : lim_b) & kLimit) != 0;
+      if constexpr (kF64) {
+        if (corrected) f += u * inc;
+      } else {
+        if (corrected) extra = u * inc;
+      }
+    }
+    return Face{open ? f : T(0), extra};
+  };
+  double acc[kF64 ? 3 * S : 1] = {};
   T top = T(0);  // largest level written (van Leer)
-  bool bad = false;
-  if (x0 < x1) {
-    const int xa = static_cast<int>(x0), xb = static_cast<int>(x1);
-    // Window of rows xx - 2 .. xx + 2 (the outer two under van Leer only).
-    Row p2 = kLimited ? load(xa - 2, false) : Row{};
+  bool bad = false, negative = false;
+  if (xa < xb) {
+    // Rows xx - 1 .. xx + 1 (and xx + 2 under van Leer).
     Row prev = load(xa - 1, false);
     Row cur = load(xa, true);
     Row next = load(xa + 1, xa + 1 < xb);
     Row n2 = kLimited ? load(xa + 2, xa + 2 < xb) : Row{};
+    Face below[S];  // across the lower x face of the current row
+    {
+      const Row p2 = kLimited ? load(xa - 2, false) : Row{};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        below[s] = face(prev.c[s], cur.c[s], field ? cur.ux : P.advection[s][0], s, ihx,
+                        (prev.site & cur.site & kOpen) != 0, p2.c[s], next.c[s],
+                        prev.site & cur.site, p2.site, next.site);
+      }
+    }
     for (int xx = xa; xx < xb; ++xx) {
       constexpr int kAhead = kLimited ? 3 : 2;
-      const Row ahead =
-          xx + kAhead < xb + kHalo ? load(xx + kAhead, xx + kAhead < xb) : Row{};
-      const int buf = xx & 1;
+      const Row ahead = xx + kAhead < xb + kHalo ? load(xx + kAhead, xx + kAhead < xb) : Row{};
+      const size_t i = static_cast<size_t>(xx) * ny + y;
+      // The y neighbours' sites, and whether the four faces are open.
+      const uint32_t site_lo = __float_as_uint(lane_below(__uint_as_float(cur.site)));
+      const uint32_t site_hi = __float_as_uint(lane_above(__uint_as_float(cur.site)));
+      const bool open_xlo = (prev.site & cur.site & kOpen) != 0;
+      const bool open_xhi = (cur.site & next.site & kOpen) != 0;
+      const bool open_ylo = (site_lo & cur.site & kOpen) != 0;
+      const bool open_yhi = (cur.site & site_hi & kOpen) != 0;
+      [[maybe_unused]] uint32_t site_lo2 = 0;
+      if constexpr (kLimited) site_lo2 = __float_as_uint(lane_below(__uint_as_float(site_lo)));
+      const bool fluid = (cur.site & kOpen) != 0;
 #pragma unroll
-      for (int s = 0; s < S; ++s) s_c[buf][s][t] = cur.c[s];
-      s_s[buf][t] = cur.solid ? 1 : 0;
-      __syncthreads();
-      if (owns) {
-        const size_t i = static_cast<size_t>(xx) * ny + y;
-        if (cur.solid) {
-#pragma unroll
-          for (int s = 0; s < S; ++s) {
-            out[s * n + i] = cur.c[s];
-            if constexpr (kLimited) top = max(top, cur.c[s]);
+      for (int s = 0; s < S; ++s) {
+        const T c = cur.c[s];
+        const T ylo_v = lane_below(c), yhi_v = lane_above(c);
+        [[maybe_unused]] T far_lo = T(0);
+        if constexpr (kLimited) far_lo = lane_below(ylo_v);
+        const Face xlo = below[s];
+        const Face xhi = face(c, next.c[s], field ? next.ux : P.advection[s][0], s, ihx, open_xhi,
+                              prev.c[s], n2.c[s], cur.site & next.site, prev.site, n2.site);
+        below[s] = xhi;
+        const Face ylo = face(ylo_v, c, field ? cur.uy : P.advection[s][1], s, ihy, open_ylo,
+                              far_lo, yhi_v, site_lo & cur.site, site_lo2, site_hi);
+        Face yhi;
+        yhi.flux = lane_above(ylo.flux);
+        if constexpr (kLimited && !kF64) yhi.extra = lane_above(ylo.extra);
+        T v;
+        if constexpr (!kF64) {
+          const float D = P.diffusion[s];
+          float rate = 0.0f;
+          if (nx != 1) {
+            const float l = open_xlo ? prev.c[s] : c, u = open_xhi ? next.c[s] : c;
+            rate += D * (l - (2.0f * c) + u) * ihx * ihx;
+            rate -= (xhi.flux - xlo.flux) * ihx;
+            if constexpr (kLimited) rate -= (xhi.extra - xlo.extra) * ihx;
           }
+          if (ny != 1) {
+            const float l = open_ylo ? ylo_v : c, u = open_yhi ? yhi_v : c;
+            rate += D * (l - (2.0f * c) + u) * ihy * ihy;
+            rate -= (yhi.flux - ylo.flux) * ihy;
+            if constexpr (kLimited) rate -= (yhi.extra - ylo.extra) * ihy;
+          }
+          if constexpr (kAffine) rate += cur.src[s] - (cur.los[s] * c);
+          if (monod) {
+            const float uptake = P.vmax[s] * cur.phi / (P.monod_k[s] + c);
+            rate += 0.0f - (uptake * c);
+          }
+          v = c + (dt * rate);
         } else {
-          const bool xlo_edge = xx == 0, xhi_edge = xx + 1 == static_cast<int>(nx);
-          const bool ylo_edge = y == 0, yhi_edge = y + 1 == ny;
-          const bool ylo_solid = s_s[buf][t - 1] != 0, yhi_solid = s_s[buf][t + 1] != 0;
-          // face_closure (signals.cpp:213-261).
-          SiteGeometry g;
-          g.clo[0] = xlo_edge ? (P.kind[0] == MSIM_NO_FLUX ||
-                                 (P.kind[0] == MSIM_PERIODIC && prev.solid))
-                              : prev.solid;
-          g.cup[0] = xhi_edge ? (P.kind[1] == MSIM_NO_FLUX ||
-                                 (P.kind[1] == MSIM_PERIODIC && next.solid))
-                              : next.solid;
-          g.clo[1] = ylo_edge ? (P.kind[2] == MSIM_NO_FLUX ||
-                                 (P.kind[2] == MSIM_PERIODIC && ylo_solid))
-                              : ylo_solid;
-          g.cup[1] = yhi_edge ? (P.kind[3] == MSIM_NO_FLUX ||
-                                 (P.kind[3] == MSIM_PERIODIC && yhi_solid))
-                              : yhi_solid;
-          // Which sites the limited correction may use (signals.cpp:1235-1253).
-          [[maybe_unused]] bool lower_site[2], upper_site[2], far_lo_ok[2], far_hi_ok[2];
-          if constexpr (kLimited) {
-            const bool xp3 = xper && nx >= 3, yp3 = yper && ny >= 3;
-            lower_site[0] = !g.clo[0] && (!xlo_edge || xp3);
-            upper_site[0] = !g.cup[0] && (!xhi_edge || xp3);
-            lower_site[1] = !g.clo[1] && (!ylo_edge || yp3);
-            upper_site[1] = !g.cup[1] && (!yhi_edge || yp3);
-            far_lo_ok[0] = (xx >= 2 || xp3) && !p2.solid;
-            far_hi_ok[0] = (xx + 2 < static_cast<int>(nx) || xp3) && !n2.solid;
-            far_lo_ok[1] = (y >= 2 || yp3) && s_s[buf][t - 2] == 0;
-            far_hi_ok[1] = (y + 2 < ny || yp3) && s_s[buf][t + 2] == 0;
+          double rate = 0.0, supply = 0.0;
+          // A flux through an edge of the grid is supplied from outside.
+          if (nx != 1) {
+            if (xx == 0 && !xper) supply += xlo.flux * ihx;
+            if (xx + 1 == static_cast<int>(nx) && !xper) supply -= xhi.flux * ihx;
+            rate -= (xhi.flux - xlo.flux) * ihx;
           }
-#pragma unroll
-          for (int s = 0; s < S; ++s) {
-            if (field) {
-              g.ulo[0] = cur.xf;
-              g.uup[0] = next.xf;
-              g.ulo[1] = cur.ylo;
-              g.uup[1] = cur.yhi;
-            } else {
-              g.ulo[0] = g.uup[0] = P.advection[s][0];
-              g.ulo[1] = g.uup[1] = P.advection[s][1];
-            }
-            const T c = cur.c[s];
-            const T ylo_v = s_c[buf][s][t - 1];
-            const T yhi_v = s_c[buf][s][t + 1];
-            [[maybe_unused]] T far_lo[2] = {T(0), T(0)}, far_hi[2] = {T(0), T(0)};
-            if constexpr (kLimited) {
-              far_lo[0] = p2.c[s];
-              far_hi[0] = n2.c[s];
-              far_lo[1] = s_c[buf][s][t - 2];
-              far_hi[1] = s_c[buf][s][t + 2];
-            }
-            const float src = kAffine ? cur.src[kAffine ? s : 0] : 0.0f;
-            const float los = kAffine ? cur.los[kAffine ? s : 0] : 0.0f;
-            if constexpr (!kF64) {
-              const float l0 = xlo_edge ? exterior<kPatched>(P, 0, s, c, prev.c[s], y) : prev.c[s];
-              const float u0 = xhi_edge ? exterior<kPatched>(P, 1, s, c, next.c[s], y) : next.c[s];
-              const float l1 = ylo_edge ? exterior<kPatched>(P, 2, s, c, ylo_v, static_cast<uint32_t>(xx)) : ylo_v;
-              const float u1 = yhi_edge ? exterior<kPatched>(P, 3, s, c, yhi_v, static_cast<uint32_t>(xx)) : yhi_v;
-              float v;
-              if constexpr (kLimited) {
-                Limiter<float> lim;
-#pragma unroll
-                for (int a2 = 0; a2 < 2; ++a2) {
-                  lim.lower_site[a2] = lower_site[a2];
-                  lim.upper_site[a2] = upper_site[a2];
-                  lim.far_lo_ok[a2] = far_lo_ok[a2];
-                  lim.far_hi_ok[a2] = far_hi_ok[a2];
-                  lim.far_lo[a2] = far_lo[a2];
-                  lim.far_hi[a2] = far_hi[a2];
-                }
-                v = fe_update_f32<true>(P, g, c, l0, u0, l1, u1, s, dt, src, los, cur.phi, &lim);
-                if (!isfinite(v)) bad = true;
-                top = max(top, v);
-              } else {
-                v = fe_update_f32(P, g, c, l0, u0, l1, u1, s, dt, src, los, cur.phi);
-                if (!isfinite(v) || v < 0.0f) bad = true;
-              }
-              out[s * n + i] = v;
-            } else {
-              const double ih[2] = {1.0 / static_cast<double>(P.dx),
-                                    1.0 / static_cast<double>(P.dy)};
-              const uint32_t dims[2] = {nx, ny};
-              const bool lo_edge[2] = {xlo_edge, ylo_edge}, hi_edge[2] = {xhi_edge, yhi_edge};
-              const double nlo[2] = {prev.c[s], ylo_v}, nhi[2] = {next.c[s], yhi_v};
-              const double D = static_cast<double>(P.diffusion[s]);
-              double rate = 0.0, supply = 0.0;
-#pragma unroll
-              for (int a = 0; a < 2; ++a) {
-                if (dims[a] == 1) continue;
-                double fl = 0.0, fu = 0.0;
-                const double ul = static_cast<double>(g.ulo[a]);
-                const double uu = static_cast<double>(g.uup[a]);
-                if (lo_edge[a] && P.kind[2 * a] == MSIM_FIXED) {
-                  const double cb = static_cast<double>(
-                      reservoir<kPatched>(P, 2 * a, s, a == 0 ? y : static_cast<uint32_t>(xx)));
-                  fl = (ul >= 0.0 ? ul * cb : ul * c) - D * (c - cb) * ih[a];
-                  supply += fl * ih[a];
-                } else if (!g.clo[a]) {
-                  const double cl = nlo[a];
-                  fl = (ul >= 0.0 ? ul * cl : ul * c) - D * (c - cl) * ih[a];
-                  if constexpr (kLimited) {
-                    if (lower_site[a]) {
-                      if (ul >= 0.0) {
-                        if (far_lo_ok[a])
-                          fl += ul * van_leer_increment<double>(cl, c, far_lo[a]);
-                      } else if (upper_site[a]) {
-                        fl += ul * van_leer_increment<double>(c, cl, nhi[a]);
-                      }
-                    }
-                  }
-                }
-                if (hi_edge[a] && P.kind[2 * a + 1] == MSIM_FIXED) {
-                  const double cb = static_cast<double>(
-                      reservoir<kPatched>(P, 2 * a + 1, s, a == 0 ? y : static_cast<uint32_t>(xx)));
-                  fu = (uu >= 0.0 ? uu * c : uu * cb) - D * (cb - c) * ih[a];
-                  supply -= fu * ih[a];
-                } else if (!g.cup[a]) {
-                  const double cu = nhi[a];
-                  fu = (uu >= 0.0 ? uu * c : uu * cu) - D * (cu - c) * ih[a];
-                  if constexpr (kLimited) {
-                    if (upper_site[a]) {
-                      if (uu >= 0.0) {
-                        if (lower_site[a]) fu += uu * van_leer_increment<double>(c, cu, nlo[a]);
-                      } else if (far_hi_ok[a]) {
-                        fu += uu * van_leer_increment<double>(cu, c, far_hi[a]);
-                      }
-                    }
-                  }
-                }
-                rate -= (fu - fl) * ih[a];
-              }
-              double lossr = 0.0;
-              if constexpr (kAffine) {
-                rate += static_cast<double>(src);
-                supply += static_cast<double>(src);
-                lossr += static_cast<double>(los);
-              }
-              if (monod) {
-                lossr += static_cast<double>(P.vmax[s]) * static_cast<double>(cur.phi) /
-                         (static_cast<double>(P.monod_k[s]) + c);
-              }
-              rate -= lossr * c;
-              const double v = c + static_cast<double>(dt) * rate;
-              if (!isfinite(v) || (v < 0.0 && !kLimited)) bad = true;
-              if constexpr (kLimited) top = max(top, v);
-              out[s * n + i] = v;
-              s_acc[3 * s + 0][t] += v;
-              s_acc[3 * s + 1][t] += supply;
-              s_acc[3 * s + 2][t] += lossr * c;
-            }
+          if (ny != 1) {
+            if (col == 0 && !yper) supply += ylo.flux * ihy;
+            if (col + 1 == static_cast<int>(ny) && !yper) supply -= yhi.flux * ihy;
+            rate -= (yhi.flux - ylo.flux) * ihy;
+          }
+          double lossr = 0.0;
+          if constexpr (kAffine) {
+            rate += static_cast<double>(cur.src[s]);
+            supply += static_cast<double>(cur.src[s]);
+            lossr += static_cast<double>(cur.los[s]);
+          }
+          if (monod) {
+            lossr += static_cast<double>(P.vmax[s]) * static_cast<double>(cur.phi) /
+                     (static_cast<double>(P.monod_k[s]) + c);
+          }
+          rate -= lossr * c;
+          v = c + static_cast<double>(dt) * rate;
+          // Solid sites hold their (zero) level; the mass counts only what moved.
+          if (owns && fluid) {
+            acc[3 * s + 0] += v;
+            acc[3 * s + 1] += supply;
+            acc[3 * s + 2] += lossr * c;
           }
         }
+        if (owns) {
+          if (fluid) {
+            bad = bad || !isfinite(v) || (!kLimited && v < T(0));
+          } else {
+            v = c;
+          }
+          if constexpr (kLimited) {
+            top = max(top, v);
+            negative = negative || v < T(0);
+          }
+          out[s * n + i] = v;
+        }
       }
-      if constexpr (kLimited) p2 = prev;
       prev = cur;
       cur = next;
       if constexpr (kLimited) {
@@ -399,16 +407,12 @@ __global__ __launch_bounds__(TY) __attribute__((amdgpu_waves_per_eu(step_waves<T
     atomicMin(&flags[1], step);
   }
   if constexpr (kLimited) {
-    const double m = block_max<TY>(static_cast<double>(top), s_red);
+    if (negative) flags[2] = step + 1;
+    const double m = block_max<kAdrBlock>(static_cast<double>(top), s_red);
     if (threadIdx.x == 0) largest[blockIdx.x] = m;
-    __syncthreads();
   }
   if constexpr (kF64) {
-    // Solid sites hold their (zero) level; the mass counts only what moved.
-    double acc[3 * S];
-#pragma unroll
-    for (int k = 0; k < 3 * S; ++k) acc[k] = s_acc[k][threadIdx.x];
-    block_sums<TY, 3 * S>(acc, s_red);
+    block_sums<kAdrBlock, 3 * S>(acc, s_red);
     if (threadIdx.x == 0) {
 #pragma unroll
       for (int k = 0; k < 3 * S; ++k) {
@@ -424,15 +428,18 @@ __global__ __launch_bounds__(TY) __attribute__((amdgpu_waves_per_eu(step_waves<T
 // levels below zero by no more than 16 epsilon (of the level type) times the
 // largest level become zero; a level still negative or not finite refuses
 // the step. Every block takes the largest level from the step's block
-// maxima.
+// maxima. `marked`: the step said in flags[2] whether it wrote a negative
+// level (a level that is not finite has already refused it), and there is
+// nothing to do where it did not: 3 us in place of a pass over the levels.
 template <typename T>
 __global__ __launch_bounds__(kAdrBlock) void k_adr_settle(T* __restrict__ levels, size_t count,
                                                           const double* __restrict__ largest,
                                                           uint32_t parts, uint32_t* flags,
-                                                          uint32_t step) {
+                                                          uint32_t step, uint32_t marked) {
   __shared__ double s_red[kAdrBlock / kWave];
   __shared__ double s_top;
   if (flags[0] != 0) return;
+  if (marked != 0 && flags[2] != step + 1) return;
   double m = 0.0;
   for (uint32_t b = threadIdx.x; b < parts; b += kAdrBlock) m = fmax(m, largest[b]);
   m = block_max<kAdrBlock>(m, s_red);
@@ -527,44 +534,29 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_survey(
   }
 }
 
-// Launch shape of the marching step: TY threads per block (64, 128 or 256)
-// for strips of TY - 2 columns, and 16 x-rows per block (fewer on small grids,
-// for about 2048 blocks): on a 4096 x 2048 grid, 8 to 32 rows per block give
-// the same speed within 10%, 16 the best for FP64 levels.
+// Launch shape of the marching step: strips of one wave, four waves per block,
+// 12 x-rows per wave, or 8 or 4 on smaller grids for at least 4096 waves (one
+// round of 16 per compute unit). At 4096x2048 with three signals (FP64 upwind,
+// FP32 upwind, FP32 van Leer) 12 rows take 131, 74 and 109 us, 8 rows 135, 77
+// and 111, 16 rows 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows 151, 78
+// and 111: longer walks read fewer rows twice but leave a last round of waves
+// nearly empty. At 1531x769 (two signals) 4 rows instead of 8: 19.5 for 20.5
+// us FP64, 20.8 for 22.9 van Leer.
 struct AdrShape {
-  int ty;
-  uint32_t rows, blocks;
+  uint32_t strips, rows, blocks;
 };
 
-AdrShape adr_shape(uint32_t nx, uint32_t ny, int halo, bool patched) {
-  AdrShape s{};
-  // The strip width (TY - 2 halo columns) that covers the grid's width with
-  // the fewest threads, the wider on a tie; 128 columns with reservoir
-  // patches.
-  uint64_t best = ~0ull;
-  for (int ty : {256, 128, 64}) {
-    if (patched && ty != 128) continue;
-    const uint32_t width = static_cast<uint32_t>(ty - 2 * halo);
-    const uint64_t threads = static_cast<uint64_t>((ny + width - 1) / width) * ty;
-    if (threads < best) {
-      best = threads;
-      s.ty = ty;
-    }
-  }
-  const uint32_t width = static_cast<uint32_t>(s.ty - 2 * halo);
-  const uint32_t strips = (ny + width - 1) / width;
-  uint32_t rows = 16;
-  while (rows > 4 && static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows) < 2048) rows /= 2;
-  s.rows = rows;
-  s.blocks = strips * ((nx + rows - 1) / rows);
-  return s;
+AdrShape adr_shape(uint32_t strips, uint32_t nx, uint32_t rows) {
+  constexpr uint32_t kWaves = kAdrBlock / kWave;
+  return AdrShape{strips, rows, (strips * ((nx + rows - 1) / rows) + kWaves - 1) / kWaves};
 }
 
-// Blocks of a step launch: at least 3S, since blocks j < 3S fold the
-// previous step's ledger partial j (blocks past the grid's strips only add
-// zeros).
-uint32_t step_blocks(const AdrShape& sh) {
-  return std::max<uint32_t>(sh.blocks, 3 * kMaxSignals);
+AdrShape adr_shape(uint32_t nx, uint32_t ny, bool limited) {
+  const uint32_t width = static_cast<uint32_t>(kWave) - (limited ? 4 : 2);
+  const uint32_t strips = (ny + width - 1) / width;
+  uint32_t rows = 12;
+  while (rows > 4 && static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows) < 4096) rows -= 4;
+  return adr_shape(strips, nx, rows);
 }
 
 uint32_t site_blocks(size_t n) { return static_cast<uint32_t>((n + kAdrBlock - 1) / kAdrBlock); }
@@ -630,13 +622,12 @@ void adr_upload(Context& ctx, const msim_signal_grid& grid, const void* levels,
   a.levels_a.reserve(bytes);
   a.levels_b.reserve(bytes);
   a.current = 0;
-  a.flags.reserve(2);
+  a.flags.reserve(3);
   a.state.reserve(1);
   a.mass.reserve(kMaxSignals);
   // Ledger partials [2][3 * kMaxSignals][blocks], then the van Leer block
   // maxima [blocks]; the survey's partials reuse the front.
-  const uint32_t step_parts =
-      step_blocks(adr_shape(P.nx, P.ny, P.limited != 0 ? 2 : 1, patched));
+  const uint32_t step_parts = adr_shape(P.nx, P.ny, P.limited != 0).blocks;
   a.partials.reserve(std::max<size_t>(
       static_cast<size_t>(3 * kMaxSignals * 2 + 1) * step_parts,
       static_cast<size_t>(kMaxSignals + 1) * 2048));
@@ -801,26 +792,22 @@ AdrView view_of(Context& ctx) {
                  a.flags.data()};
 }
 
-template <typename T, int S, int TY, bool kLimited, bool kPatched>
+template <typename T, int S, bool kAffine, bool kLimited>
 void launch_step(hipStream_t stream, const AdrView& v, const AdrShape& sh, const float* xf,
                  const float* yf, const uint8_t* src, uint8_t* dst, float dt, uint32_t k,
-                 LedgerParts L, double* largest, bool settle) {
+                 LedgerParts L, double* largest) {
   const AdrParams& P = *v.P;
-  if (P.has_affine != 0) {
-    k_adr_step<T, S, TY, true, kLimited, kPatched><<<sh.blocks, TY, 0, stream>>>(
-        P, v.solid, xf, yf, v.phi, v.source, v.loss, reinterpret_cast<const T*>(src),
-        reinterpret_cast<T*>(dst), dt, v.flags, k, sh.rows, L, largest);
+  const T* in = reinterpret_cast<const T*>(src);
+  T* out = reinterpret_cast<T*>(dst);
+  const uint32_t blocks = sh.blocks + (sizeof(T) == 8 ? 3 * S : 0);
+  if (P.edge != nullptr) {
+    k_adr_step<T, S, kAffine, kLimited, true><<<blocks, kAdrBlock, 0, stream>>>(
+        P, v.solid, xf, yf, v.phi, v.source, v.loss, in, out, dt, v.flags, k, sh.rows, sh.strips,
+        L, largest);
   } else {
-    k_adr_step<T, S, TY, false, kLimited, kPatched><<<sh.blocks, TY, 0, stream>>>(
-        P, v.solid, xf, yf, v.phi, v.source, v.loss, reinterpret_cast<const T*>(src),
-        reinterpret_cast<T*>(dst), dt, v.flags, k, sh.rows, L, largest);
-  }
-  if (kLimited && settle) {
-    const size_t count = static_cast<size_t>(S) * P.nx * P.ny;
-    const uint32_t blocks = static_cast<uint32_t>(
-        std::min<size_t>((count + kAdrBlock - 1) / kAdrBlock, 2048));
-    k_adr_settle<T><<<blocks, kAdrBlock, 0, stream>>>(reinterpret_cast<T*>(dst), count, largest,
-                                                      sh.blocks, v.flags, k);
+    k_adr_step<T, S, kAffine, kLimited, false><<<blocks, kAdrBlock, 0, stream>>>(
+        P, v.solid, xf, yf, v.phi, v.source, v.loss, in, out, dt, v.flags, k, sh.rows, sh.strips,
+        L, largest);
   }
 }
 
@@ -828,24 +815,18 @@ template <typename T, int S, bool kLimited>
 void launch_typed(hipStream_t stream, const AdrView& v, const AdrShape& sh, const float* xf,
                   const float* yf, const uint8_t* src, uint8_t* dst, float dt, uint32_t k,
                   LedgerParts L, double* largest, bool settle = true) {
-  // Specs with reservoir patches take one strip width (128 columns).
-  if (v.P->edge != nullptr) {
-    launch_step<T, S, 128, kLimited, true>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest,
-                                           settle);
-    return;
+  const AdrParams& P = *v.P;
+  if (P.has_affine != 0) {
+    launch_step<T, S, true, kLimited>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest);
+  } else {
+    launch_step<T, S, false, kLimited>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest);
   }
-  switch (sh.ty) {
-    case 64:
-      launch_step<T, S, 64, kLimited, false>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest,
-                                             settle);
-      break;
-    case 128:
-      launch_step<T, S, 128, kLimited, false>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest,
-                                              settle);
-      break;
-    default:
-      launch_step<T, S, 256, kLimited, false>(stream, v, sh, xf, yf, src, dst, dt, k, L, largest,
-                                              settle);
+  if (kLimited && settle) {
+    const size_t count = static_cast<size_t>(S) * P.nx * P.ny;
+    const uint32_t blocks = static_cast<uint32_t>(
+        std::min<size_t>((count + kAdrBlock - 1) / kAdrBlock, 2048));
+    k_adr_settle<T><<<blocks, kAdrBlock, 0, stream>>>(reinterpret_cast<T*>(dst), count, largest,
+                                                      sh.blocks, v.flags, k, 1);
   }
 }
 
@@ -855,8 +836,7 @@ void launch_candidate(Context& ctx, float dt, const float* in, float* out, uint3
                       const float* xf, const float* yf) {
   auto& a = ctx.adr;
   const bool limited = a.params.limited != 0;
-  AdrShape sh = adr_shape(a.params.nx, a.params.ny, limited ? 2 : 1, a.params.edge != nullptr);
-  sh.blocks = step_blocks(sh);
+  AdrShape sh = adr_shape(a.params.nx, a.params.ny, limited);
   LedgerParts L{a.partials.data(), a.ledger.data(), sh.blocks};
   double* largest = a.partials.data() + static_cast<size_t>(3 * kMaxSignals * 2) * sh.blocks;
   const auto* src = reinterpret_cast<const uint8_t*>(in);
@@ -875,8 +855,7 @@ void launch_steps(Context& ctx, float dt, uint32_t steps, const float* xf, const
   auto& a = ctx.adr;
   const auto& P = a.params;
   const bool limited = P.limited != 0;
-  AdrShape sh = adr_shape(P.nx, P.ny, limited ? 2 : 1, P.edge != nullptr);
-  sh.blocks = step_blocks(sh);
+  AdrShape sh = adr_shape(P.nx, P.ny, limited);
   LedgerParts L{a.partials.data(), a.ledger.data(), sh.blocks};
   double* largest = a.partials.data() + static_cast<size_t>(3 * kMaxSignals * 2) * sh.blocks;
   const AdrView v = view_of(ctx);
@@ -926,7 +905,7 @@ void launch_settle_f32(Context& ctx, float* levels, size_t count, const double* 
   const uint32_t blocks =
       static_cast<uint32_t>(std::min<size_t>((count + kAdrBlock - 1) / kAdrBlock, 2048));
   k_adr_settle<float><<<blocks, kAdrBlock, 0, ctx.stream>>>(levels, count, largest, parts,
-                                                            ctx.adr.flags.data(), step);
+                                                            ctx.adr.flags.data(), step, 0);
   check(hipGetLastError(), "launch k_adr_settle");
 }
 
@@ -935,7 +914,7 @@ void adr_run(Context& ctx, float dt, uint32_t steps, double* ledger) {
   const auto& P = a.params;
   const float* xf = a.flow_field ? ctx.flow.faces.data() : a.xf.data();
   const float* yf = a.flow_field ? ctx.flow.faces.data() + ctx.flow.x_faces() : a.yf.data();
-  const uint32_t init_flags[2] = {0u, 0xffffffffu};
+  const uint32_t init_flags[3] = {0u, 0xffffffffu, 0u};
   check(hipMemcpyAsync(a.flags.data(), init_flags, sizeof(init_flags), hipMemcpyHostToDevice,
                        ctx.stream),
         "clear flags");
@@ -1087,6 +1066,26 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 void* g_scratch[kStaticDevices] = {};
 std::mutex g_scratch_lock[kStaticDevices];
 
+// Blocks whose partials the scratch holds room for: strips of 62, 126 or 254
+// columns (60, 124 or 252 under van Leer; whichever takes the fewest threads)
+// by 16 x-rows, or fewer down to 4 for 2048 blocks. A formula of its own, so
+// that the grids that fit the scratch stay the same whatever shape a step is
+// launched in.
+uint32_t static_blocks(const AdrParams& P) {
+  uint64_t best = ~0ull, strips = 1;
+  for (uint32_t threads : {256u, 128u, 64u}) {
+    const uint64_t width = threads - (P.limited != 0 ? 4 : 2);
+    const uint64_t count = (P.ny + width - 1) / width;
+    if (count * threads < best) {
+      best = count * threads;
+      strips = count;
+    }
+  }
+  uint32_t rows = 16;
+  while (rows > 4 && strips * ((P.nx + rows - 1) / rows) < 2048) rows /= 2;
+  return std::max(static_cast<uint32_t>(strips * ((P.nx + rows - 1) / rows)), 3u * kMaxSignals);
+}
+
 // Carves 256-byte aligned regions out of the scratch array, in order.
 struct ScratchLayout {
   size_t used = 0;
@@ -1145,16 +1144,17 @@ void adr_step_static(Context& ctx, const msim_signal_grid& grid, float dt, float
   AdrParams P = transport_params(grid);
   const uint32_t S = P.signals;
   const size_t n = static_cast<size_t>(P.nx) * P.ny;
-  const AdrShape base = adr_shape(P.nx, P.ny, P.limited != 0 ? 2 : 1, false);
-  AdrShape sh = base;
-  sh.blocks = step_blocks(sh);
+  AdrShape sh = adr_shape(P.nx, P.ny, P.limited != 0);
+  // Longer walks where the shape has more blocks than that.
+  const uint32_t room = static_blocks(P);
+  while (sh.blocks > room && sh.rows < P.nx) sh = adr_shape(sh.strips, P.nx, sh.rows + 4);
   const uint32_t survey_blocks = std::min<uint32_t>(site_blocks(n), 2048);
   ScratchLayout at;
   const size_t o_state = at.take(sizeof(CgState));
-  const size_t o_flags = at.take(2 * sizeof(uint32_t));
+  const size_t o_flags = at.take(3 * sizeof(uint32_t));
   const size_t o_mass = at.take(kMaxSignals * sizeof(double));
   const size_t o_parts = at.take(
-      std::max<size_t>(static_cast<size_t>(3 * kMaxSignals * 2 + 1) * sh.blocks,
+      std::max<size_t>(static_cast<size_t>(3 * kMaxSignals * 2 + 1) * std::max(room, sh.blocks),
                        static_cast<size_t>(kMaxSignals + 1) * survey_blocks) *
       sizeof(double));
   const size_t o_solid = at.take(n);
@@ -1192,7 +1192,7 @@ void adr_step_static(Context& ctx, const msim_signal_grid& grid, float dt, float
   // The array keeps the last call's contents: the state (with its tickets),
   // the flags and every staged array are written afresh.
   const CgState zero_state{};
-  const uint32_t init_flags[2] = {0u, 0xffffffffu};
+  const uint32_t init_flags[3] = {0u, 0xffffffffu, 0u};
   check(hipMemcpyAsync(state, &zero_state, sizeof(CgState), hipMemcpyHostToDevice, stream),
         "clear state");
   check(hipMemcpyAsync(flags, init_flags, sizeof(init_flags), hipMemcpyHostToDevice, stream),
