@@ -891,9 +891,11 @@ class HipBackend:
         zf = np.zeros(nfz, np.float32)
         p = parameters._c(keep)
         rep = _FlowReport()
+        # One layer's z faces are zero, as zf is already.
         self._check(self.lib.msim_hip_solve_depth_averaged_flow(
             self.ctx, C.byref(g), None if mob is None else mob.ctypes.data, C.byref(p),
-            xf.ctypes.data, yf.ctypes.data, zf.ctypes.data, C.byref(rep)))
+            xf.ctypes.data, yf.ctypes.data, None if grid.nz == 1 else zf.ctypes.data,
+            C.byref(rep)))
         return DepthAveragedFlowResult(VelocityField(xf, yf, zf),
                                        DepthAveragedFlowReport._from(rep))
 
@@ -1189,7 +1191,7 @@ class HipBackend:
         xf, yf, zf = (np.zeros(k, np.float32) for k in (nfx, nfy, nfz))
         self._check(self.lib.msim_hip_flow_download(self.ctx, pressure.ctypes.data,
                                                     xf.ctypes.data, yf.ctypes.data,
-                                                    zf.ctypes.data))
+                                                    None if g.nz == 1 else zf.ctypes.data))
         return pressure, VelocityField(xf, yf, zf)
 
     def flow_apply(self, x) -> np.ndarray:

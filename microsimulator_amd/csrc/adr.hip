@@ -1041,8 +1041,7 @@ void adr_download(Context& ctx, void* levels) {
   const size_t bytes =
       a.params.signals * a.sites() * (a.precision == 64 ? sizeof(double) : sizeof(float));
   const uint8_t* src = a.current == 0 ? a.levels_a.data() : a.levels_b.data();
-  check(hipMemcpyAsync(levels, src, bytes, hipMemcpyDeviceToHost, ctx.stream), "download levels");
-  check(hipStreamSynchronize(ctx.stream), "download levels");
+  download(ctx, levels, src, bytes, "download levels");
 }
 
 // ---------------------------------------------------------------------------

@@ -1206,6 +1206,7 @@ int msim_hip_create(int device, msim_ctx** out) {
   }
   auto* ctx = new (std::nothrow) msim_ctx;
   if (ctx == nullptr) return MSIM_RUNTIME_ERROR;
+  msim::download_enter();
   ctx->impl.device = device;
   if (hipSetDevice(device) != hipSuccess ||
       hipStreamCreateWithFlags(&ctx->impl.stream, hipStreamNonBlocking) != hipSuccess ||
@@ -1243,6 +1244,7 @@ void msim_hip_destroy(msim_ctx* ctx) {
   if (ctx->impl.stop != nullptr) static_cast<void>(hipEventDestroy(ctx->impl.stop));
   if (ctx->impl.stream != nullptr) static_cast<void>(hipStreamDestroy(ctx->impl.stream));
   delete ctx;
+  msim::download_leave();
 }
 
 const char* msim_hip_last_error(const msim_ctx* ctx) {
@@ -1323,13 +1325,10 @@ int msim_hip_flow_download(msim_ctx* ctx, double* pressure, float* x_faces, floa
     auto& f = c.flow;
     if (!f.solved) msim::invalid("no flow solve to download");
     if (pressure != nullptr) {
-      msim::check(hipMemcpyAsync(pressure, f.x.data(), f.sites() * sizeof(double),
-                                 hipMemcpyDeviceToHost, c.stream),
-                  "download pressure");
+      msim::download(c, pressure, f.x.data(), f.sites() * sizeof(double), "download pressure");
     }
     if (f.layers.nz > 1) {
       // The lifted voxel faces of a grid of several layers.
-      msim::check(hipStreamSynchronize(c.stream), "download");
       const auto& v = f.layers.faces;
       const size_t nz = f.layers.nz;
       const size_t nxf = f.x_faces() * nz, nyf = f.y_faces() * nz;
@@ -1341,16 +1340,13 @@ int msim_hip_flow_download(msim_ctx* ctx, double* pressure, float* x_faces, floa
       return;
     }
     if (x_faces != nullptr) {
-      msim::check(hipMemcpyAsync(x_faces, f.faces.data(), f.x_faces() * sizeof(float),
-                                 hipMemcpyDeviceToHost, c.stream),
-                  "download x faces");
+      msim::download(c, x_faces, f.faces.data(), f.x_faces() * sizeof(float),
+                     "download x faces");
     }
     if (y_faces != nullptr) {
-      msim::check(hipMemcpyAsync(y_faces, f.faces.data() + f.x_faces(),
-                                 f.y_faces() * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-                  "download y faces");
+      msim::download(c, y_faces, f.faces.data() + f.x_faces(), f.y_faces() * sizeof(float),
+                     "download y faces");
     }
-    msim::check(hipStreamSynchronize(c.stream), "download");
     if (z_faces != nullptr) std::memset(z_faces, 0, 2 * f.sites() * sizeof(float));
   });
 }

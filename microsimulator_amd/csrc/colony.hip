@@ -395,15 +395,12 @@ uint32_t colony_deposit(Context& ctx, const msim_grid& grid, const float* origin
     throw Error(MSIM_RUNTIME_ERROR, "a deposit support exceeded the bound its launch was sized for");
   }
   if (failed[0] == 0xffffffffu) {
-    check(hipMemcpyAsync(want_mobility ? mobility_host : density_host, d.out.data(),
-                         n * sizeof(double), hipMemcpyDeviceToHost, ctx.stream),
-          "download colony field");
+    download(ctx, want_mobility ? mobility_host : density_host, d.out.data(), n * sizeof(double),
+             "download colony field");
     if (coupling) {
-      check(hipMemcpyAsync(force_host, d.force.data(), 2 * columns * sizeof(double),
-                           hipMemcpyDeviceToHost, ctx.stream),
-            "download colony force");
+      download(ctx, force_host, d.force.data(), 2 * columns * sizeof(double),
+               "download colony force");
     }
-    check(hipStreamSynchronize(ctx.stream), "download colony field");
   }
   return failed[0];
 }

@@ -883,11 +883,8 @@ void coupled_download(Context& ctx, float* levels, float* species) {
         c.order.data(), c.cells, c.species, true, reinterpret_cast<const uint32_t*>(src),
         reinterpret_cast<uint32_t*>(c.staging.data()));
     check(hipGetLastError(), "launch k_permute");
-    check(hipMemcpyAsync(species, c.staging.data(),
-                         static_cast<size_t>(c.cells) * c.species * sizeof(float),
-                         hipMemcpyDeviceToHost, ctx.stream),
-          "download species");
-    check(hipStreamSynchronize(ctx.stream), "download species");
+    download(ctx, species, c.staging.data(),
+             static_cast<size_t>(c.cells) * c.species * sizeof(float), "download species");
   }
 }
 

@@ -1,0 +1,134 @@
+// Large results to the caller's memory. A pageable destination goes through
+// the runtime's single staging thread at about 10 GB/s (a fresh array's pages
+// are touched there too); here several threads each bring chunks over into a
+// pinned slot of their own and copy them out, so the transfers run back to
+// back while the pages are touched in parallel.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "internal.hpp"
+
+namespace msim {
+namespace {
+
+constexpr size_t kSlotBytes = size_t(2) << 20;
+constexpr size_t kMostSlots = 16;     // 32 MiB pinned in the process, at most
+constexpr size_t kMostThreads = 8;
+// Below this the threads cost more than they save.
+constexpr size_t kThreadedBytes = size_t(4) << 20;
+
+// The process's pinned slots: handed out to one download at a time, kept for
+// the next, freed with the last context.
+class SlotPool {
+ public:
+  std::vector<void*> take(size_t wanted) {
+    std::lock_guard<std::mutex> hold(lock_);
+    std::vector<void*> out;
+    while (out.size() < wanted) {
+      if (!free_.empty()) {
+        out.push_back(free_.back());
+        free_.pop_back();
+        continue;
+      }
+      if (made_ == kMostSlots) break;
+      void* ptr = nullptr;
+      if (hipHostMalloc(&ptr, kSlotBytes, hipHostMallocPortable) != hipSuccess) {
+        static_cast<void>(hipGetLastError());
+        break;
+      }
+      ++made_;
+      out.push_back(ptr);
+    }
+    return out;
+  }
+  void give(const std::vector<void*>& slots) {
+    std::lock_guard<std::mutex> hold(lock_);
+    free_.insert(free_.end(), slots.begin(), slots.end());
+    if (users_ == 0) release();
+  }
+  void enter() {
+    std::lock_guard<std::mutex> hold(lock_);
+    ++users_;
+  }
+  void leave() {
+    std::lock_guard<std::mutex> hold(lock_);
+    if (--users_ == 0) release();
+  }
+
+ private:
+  void release() {
+    for (void* p : free_) static_cast<void>(hipHostFree(p));
+    made_ -= free_.size();
+    free_.clear();
+  }
+  std::mutex lock_;
+  std::vector<void*> free_;
+  size_t made_ = 0, users_ = 0;
+};
+
+SlotPool g_slots;
+
+}  // namespace
+
+void download_enter() { g_slots.enter(); }
+void download_leave() { g_slots.leave(); }
+
+void download(Context& ctx, void* dst, const void* src, size_t bytes, const char* what) {
+  const size_t chunks = (bytes + kSlotBytes - 1) / kSlotBytes;
+  const size_t cores = std::max<size_t>(std::thread::hardware_concurrency(), 1);
+  std::vector<void*> slots;
+  if (bytes >= kThreadedBytes && cores > 1)
+    slots = g_slots.take(std::min({kMostThreads, cores, chunks}));
+  if (slots.size() < 2) {
+    g_slots.give(slots);
+    check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx.stream), what);
+    check(hipStreamSynchronize(ctx.stream), what);
+    return;
+  }
+  // Every chunk is taken by exactly one thread; whatever fails, all are joined
+  // and the slots go back only after the stream has drained.
+  std::atomic<size_t> next{0};
+  std::atomic<int> failed{hipSuccess};
+  auto work = [&](void* slot) {
+    hipEvent_t ready = nullptr;
+    hipError_t e = hipSetDevice(ctx.device);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
+    while (e == hipSuccess && failed.load() == hipSuccess) {
+      const size_t c = next.fetch_add(1);
+      if (c >= chunks) break;
+      const size_t at = c * kSlotBytes, size = std::min(kSlotBytes, bytes - at);
+      e = hipMemcpyAsync(slot, static_cast<const char*>(src) + at, size, hipMemcpyDeviceToHost,
+                         ctx.stream);
+      if (e == hipSuccess) e = hipEventRecord(ready, ctx.stream);
+      if (e == hipSuccess) e = hipEventSynchronize(ready);
+      if (e == hipSuccess) std::memcpy(static_cast<char*>(dst) + at, slot, size);
+    }
+    if (ready != nullptr) static_cast<void>(hipEventDestroy(ready));
+    if (e != hipSuccess) {
+      int none = hipSuccess;
+      failed.compare_exchange_strong(none, e);
+    }
+  };
+  std::vector<std::thread> threads;
+  threads.reserve(slots.size());
+  try {
+    for (size_t k = 1; k < slots.size(); ++k) threads.emplace_back(work, slots[k]);
+  } catch (const std::system_error&) {
+    // Fewer threads then: the others take every chunk.
+  }
+  work(slots[0]);
+  for (auto& t : threads) t.join();
+  const hipError_t drained = hipStreamSynchronize(ctx.stream);
+  g_slots.give(slots);
+  check(static_cast<hipError_t>(failed.load()), what);
+  check(drained, what);
+}
+
+}  // namespace msim

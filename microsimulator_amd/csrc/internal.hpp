@@ -390,6 +390,12 @@ struct KernelTimes {
   uint32_t cycles = 0;
 };
 
+// download.cpp: device memory to the caller's, complete on return; the pinned
+// slots it keeps live as long as any context.
+void download(Context& ctx, void* dst, const void* src, size_t bytes, const char* what);
+void download_enter();
+void download_leave();
+
 // flow.hip
 void flow_assemble(Context& ctx, const uint8_t* solid_host, const float* mobility_host);
 // Conductance and assembly of one grid already on the device, with the

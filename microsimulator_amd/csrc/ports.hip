@@ -385,22 +385,16 @@ void port_flow_solve(Context& ctx, const PortPlan& plan, const msim_port_flow_pa
   const size_t nxf = f.x_faces() * nz, nyf = f.y_faces() * nz;
   const float* out = f.lifted.data();
   if (x_faces != nullptr) {
-    check(hipMemcpyAsync(x_faces, out, nxf * sizeof(float), hipMemcpyDeviceToHost, ctx.stream),
-          "download x faces");
+    download(ctx, x_faces, out, nxf * sizeof(float), "download x faces");
   }
   if (y_faces != nullptr) {
-    check(hipMemcpyAsync(y_faces, out + nxf, nyf * sizeof(float), hipMemcpyDeviceToHost,
-                         ctx.stream),
-          "download y faces");
+    download(ctx, y_faces, out + nxf, nyf * sizeof(float), "download y faces");
   }
   if (z_faces != nullptr && nz == 1) {
     std::memset(z_faces, 0, 2 * f.sites() * sizeof(float));
   } else if (z_faces != nullptr) {
-    check(hipMemcpyAsync(z_faces, out + nxf + nyf, (F - nxf - nyf) * sizeof(float),
-                         hipMemcpyDeviceToHost, ctx.stream),
-          "download z faces");
+    download(ctx, z_faces, out + nxf + nyf, (F - nxf - nyf) * sizeof(float), "download z faces");
   }
-  check(hipStreamSynchronize(ctx.stream), "download port flow");
   if (states != nullptr) {
     for (uint32_t q = 0; q < count; ++q) {
       const double flux = combined_flux(q);
