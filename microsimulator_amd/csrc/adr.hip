@@ -24,13 +24,14 @@
 #include <vector>
 
 #include "adr_site.hpp"
+#include "adr_strip.hpp"
 #include "common.hpp"
 #include "internal.hpp"
 
 namespace msim {
 namespace {
 
-constexpr int kAdrBlock = 256;
+constexpr int kAdrBlock = kStripBlock;
 
 // The ledger of a step lives as per-block partial sums (mass after, boundary
 // supply rate, uptake rate, for each signal) in two generations by step
@@ -84,45 +85,6 @@ __device__ inline void block_sums(double (&v)[K], double* lds) {
   }
 }
 
-// What one lane holds of one x-row of its column: the S levels and what of
-// the site a face next to it needs (kOpen: a flux may cross it; kLimit: the
-// limited correction may read it); for sites the wave updates also the
-// velocities of the site's lower faces, the occupancy and (with affine
-// reactions) the rates. Beyond a fixed face stands a ghost site, open and
-// holding the reservoir's level; beyond a closed face a site that is neither.
-constexpr uint32_t kOpen = 1, kLimit = 2;
-
-template <typename T, int S, bool kAffine>
-struct AdrRow {
-  T c[S];
-  float src[kAffine ? S : 1], los[kAffine ? S : 1];
-  float ux, uy, phi;
-  uint32_t site;
-};
-
-// A value from the lane below or above (columns col - 1, col + 1); lanes 0
-// and 63 get zero from beyond the wave.
-__device__ inline float lane_below(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ inline float lane_above(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-template <int kControl>
-__device__ inline double lane_shift(double v) {
-  const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(v));
-  const uint32_t lo = static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), kControl, 0xf, 0xf, true));
-  const uint32_t hi = static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), kControl, 0xf, 0xf, true));
-  return __longlong_as_double(
-      static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
-}
-__device__ inline double lane_below(double v) { return lane_shift<0x138>(v); }
-__device__ inline double lane_above(double v) { return lane_shift<0x130>(v); }
-
 // One forward-Euler step for S signals, marching: each wave owns a strip of
 // 64 - 2H columns and `rows` x-rows and walks x on its own, one column per
 // lane, so each level is read from memory once; its x neighbours come from
@@ -158,11 +120,10 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
     uint32_t* flags, uint32_t step, uint32_t rows, uint32_t strips, LedgerParts L,
     double* largest) {
   constexpr bool kF64 = sizeof(T) == 8;
-  constexpr int kHalo = kLimited ? 2 : 1;
-  constexpr int kWidth = kWave - 2 * kHalo;
-  constexpr int kWaves = kAdrBlock / kWave;
-  using Row = AdrRow<T, S, kAffine>;
-  __shared__ double s_red[(kF64 ? 3 * S : 1) * kWaves];
+  using Lane = Strip<kLimited, kPatched>;
+  using Row = StripRow<T, S>;
+  using Face = StripFace<T>;
+  __shared__ double s_red[(kF64 ? 3 * S : 1) * kStripWaves];
   // An earlier step failed: the run stops there. (flags[1] holds the first
   // failed step; a failure of this step may be seen here half-published, and
   // then the previous step's ledger row is still folded, as it is valid.)
@@ -176,106 +137,38 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
     }
   }
   if (flags[0] != 0) return;  // this step already failed elsewhere
-  const uint32_t nx = P.nx, ny = P.ny;
-  const size_t n = static_cast<size_t>(nx) * ny;
-  const int lane = threadIdx.x & (kWave - 1);
-  const uint32_t walk = __builtin_amdgcn_readfirstlane(
-      xcd_tile(blockIdx.x, L.blocks) * kWaves + threadIdx.x / kWave);
-  const int xa = static_cast<int>(min(nx, (walk / strips) * rows));
-  const int xb = static_cast<int>(min(nx, static_cast<uint32_t>(xa) + rows));
-  const bool xper = P.kind[0] == MSIM_PERIODIC, yper = P.kind[2] == MSIM_PERIODIC;
-  const bool field = P.has_field != 0, monod = P.has_monod != 0;
-  // This lane's column; off the grid the periodic partner's, a ghost of the
-  // fixed face next to it, or nothing.
-  const int col = static_cast<int>((walk % strips) * kWidth) + lane - kHalo;
-  const bool on_y = col >= 0 && col < static_cast<int>(ny);
-  int src_col = col;
-  if (!on_y && yper) src_col = col < 0 ? col + static_cast<int>(ny) : col - static_cast<int>(ny);
-  const bool loads =
-      src_col >= 0 && src_col < static_cast<int>(ny) && (on_y || (yper && ny > 1));
-  const int ghost_y = ny == 1 ? -1
-                      : col == -1 && P.kind[2] == MSIM_FIXED ? 2
-                      : col == static_cast<int>(ny) && P.kind[3] == MSIM_FIXED ? 3
-                                                                               : -1;
-  const bool limits_y = on_y || ny >= 3;  // a periodic partner, for the limiter
-  const bool owns = on_y && lane >= kHalo && lane < kHalo + kWidth;
-  const uint32_t y = static_cast<uint32_t>(src_col);
-  // Row xx of the walk, xx in [-H, nx + H - 1]; `full` rows are the ones the
-  // wave updates.
+  const Lane at(P, xcd_tile(blockIdx.x, L.blocks) * kStripWaves + threadIdx.x / kWave, strips,
+                rows);
+  const int xa = at.xa, xb = at.xb, col = at.col;
+  const uint32_t nx = at.nx, ny = at.ny, y = at.y;
+  const size_t n = at.n;
+  const bool owns = at.owns, field = at.field, monod = P.has_monod != 0;
   auto load = [&](int xx, bool full) {
-    Row w{};
-    const bool on_x = xx >= 0 && xx < static_cast<int>(nx);
-    if (field && owns && xx >= 0 && xx <= static_cast<int>(nx))
-      w.ux = xf[static_cast<size_t>(xx) * ny + y];
-    int row = xx;
-    if (!on_x) {
-      if (xper && nx > 1) {
-        row = xx < 0 ? xx + static_cast<int>(nx) : xx - static_cast<int>(nx);
-      } else {
-        const int face = xx == -1 ? 0 : xx == static_cast<int>(nx) ? 1 : -1;
-        if (nx > 1 && on_y && face >= 0 && P.kind[face] == MSIM_FIXED) {
-          w.site = kOpen;
+    return at.template load<T, S>(xx, full, solid, xf, yf, in);
+  };
+  // What a site's own update reads besides, for rows the wave updates.
+  struct Extra {
+    float src[kAffine ? S : 1], los[kAffine ? S : 1], phi;
+  };
+  auto load_extra = [&](int xx) {
+    Extra w{};
+    if (xx >= xb || !owns) return w;
+    const size_t i = static_cast<size_t>(xx) * ny + y;
+    if (monod) w.phi = phi[i];
+    if constexpr (kAffine) {
 #pragma unroll
-          for (int s = 0; s < S; ++s)
-            w.c[s] = static_cast<T>(reservoir<kPatched>(P, face, s, y));
-        }
-        return w;
+      for (int s = 0; s < S; ++s) {
+        w.src[s] = source[s * n + i];
+        w.los[s] = loss[s * n + i];
       }
     }
-    if (row < 0 || row >= static_cast<int>(nx)) return w;
-    if (loads) {
-      const size_t i = static_cast<size_t>(row) * ny + y;
-      const uint32_t limit = limits_y && (on_x || nx >= 3) ? kOpen | kLimit : kOpen;
-      w.site = solid[i] != 0 ? 0u : limit;
-#pragma unroll
-      for (int s = 0; s < S; ++s) w.c[s] = in[s * n + i];
-      if (full && owns) {
-        if (monod) w.phi = phi[i];
-        if constexpr (kAffine) {
-#pragma unroll
-          for (int s = 0; s < S; ++s) {
-            w.src[s] = source[s * n + i];
-            w.los[s] = loss[s * n + i];
-          }
-        }
-      }
-    } else if (ghost_y >= 0 && on_x) {
-      w.site = kOpen;
-#pragma unroll
-      for (int s = 0; s < S; ++s)
-        w.c[s] = static_cast<T>(reservoir<kPatched>(P, ghost_y, s, static_cast<uint32_t>(row)));
-    }
-    if (full && field && col >= 0 && col <= static_cast<int>(ny))
-      w.uy = yf[static_cast<size_t>(row) * (ny + 1) + static_cast<uint32_t>(col)];
     return w;
   };
-  // What crosses a face from the lower site (level a) to the upper one (b):
-  // FP64 the flux, FP32 its advective part (the diffusive one is the site's)
-  // and, under van Leer, the correction; zero where the face is closed.
-  struct Face {
-    T flux;
-    T extra;  // FP32 van Leer
-  };
   const T ihx = T(1) / static_cast<T>(P.dx), ihy = T(1) / static_cast<T>(P.dy);
-  auto face = [&](T a, T b, float velocity, int s, T ih, bool open, [[maybe_unused]] T far_a,
-                  [[maybe_unused]] T far_b, [[maybe_unused]] uint32_t lim,
-                  [[maybe_unused]] uint32_t lim_a, [[maybe_unused]] uint32_t lim_b) {
-    const T u = static_cast<T>(velocity);
-    const bool forward = u >= T(0);
-    T f = u * (forward ? a : b);
-    if constexpr (kF64) f -= static_cast<T>(P.diffusion[s]) * (b - a) * ih;
-    T extra = T(0);
-    if constexpr (kLimited) {
-      const T inc = van_leer_increment<T>(forward ? a : b, forward ? b : a,
-                                          forward ? far_a : far_b);
-      const bool corrected = (lim & (forward ? lim_a : lim_b) & kLimit) != 0;
-      if constexpr (kF64) {
-        if (corrected) f += u * inc;
-      } else {
-        if (corrected) extra = u * inc;
-      }
-    }
-    return Face{open ? f : T(0), extra};
+  auto face = [&](T a, T b, float velocity, int s, T ih, bool open, T far_a, T far_b, uint32_t lim,
+                  uint32_t lim_a, uint32_t lim_b) {
+    return strip_face<kLimited, T>(a, b, velocity, P.diffusion[s], ih, open, far_a, far_b, lim,
+                                   lim_a, lim_b);
   };
   double acc[kF64 ? 3 * S : 1] = {};
   T top = T(0);  // largest level written (van Leer)
@@ -286,6 +179,7 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
     Row cur = load(xa, true);
     Row next = load(xa + 1, xa + 1 < xb);
     Row n2 = kLimited ? load(xa + 2, xa + 2 < xb) : Row{};
+    Extra own = load_extra(xa), own_next = load_extra(xa + 1);
     Face below[S];  // across the lower x face of the current row
     {
       const Row p2 = kLimited ? load(xa - 2, false) : Row{};
@@ -298,17 +192,18 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
     }
     for (int xx = xa; xx < xb; ++xx) {
       constexpr int kAhead = kLimited ? 3 : 2;
-      const Row ahead = xx + kAhead < xb + kHalo ? load(xx + kAhead, xx + kAhead < xb) : Row{};
+      const Row ahead =
+          xx + kAhead < xb + Lane::kHalo ? load(xx + kAhead, xx + kAhead < xb) : Row{};
+      const Extra own_ahead = load_extra(xx + 2);
       const size_t i = static_cast<size_t>(xx) * ny + y;
       // The y neighbours' sites, and whether the four faces are open.
-      const uint32_t site_lo = __float_as_uint(lane_below(__uint_as_float(cur.site)));
-      const uint32_t site_hi = __float_as_uint(lane_above(__uint_as_float(cur.site)));
+      const uint32_t site_lo = site_below(cur.site), site_hi = site_above(cur.site);
       const bool open_xlo = (prev.site & cur.site & kOpen) != 0;
       const bool open_xhi = (cur.site & next.site & kOpen) != 0;
       const bool open_ylo = (site_lo & cur.site & kOpen) != 0;
       const bool open_yhi = (cur.site & site_hi & kOpen) != 0;
       [[maybe_unused]] uint32_t site_lo2 = 0;
-      if constexpr (kLimited) site_lo2 = __float_as_uint(lane_below(__uint_as_float(site_lo)));
+      if constexpr (kLimited) site_lo2 = site_below(site_lo);
       const bool fluid = (cur.site & kOpen) != 0;
 #pragma unroll
       for (int s = 0; s < S; ++s) {
@@ -327,23 +222,12 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
         if constexpr (kLimited && !kF64) yhi.extra = lane_above(ylo.extra);
         T v;
         if constexpr (!kF64) {
-          const float D = P.diffusion[s];
-          float rate = 0.0f;
-          if (nx != 1) {
-            const float l = open_xlo ? prev.c[s] : c, u = open_xhi ? next.c[s] : c;
-            rate += D * (l - (2.0f * c) + u) * ihx * ihx;
-            rate -= (xhi.flux - xlo.flux) * ihx;
-            if constexpr (kLimited) rate -= (xhi.extra - xlo.extra) * ihx;
-          }
-          if (ny != 1) {
-            const float l = open_ylo ? ylo_v : c, u = open_yhi ? yhi_v : c;
-            rate += D * (l - (2.0f * c) + u) * ihy * ihy;
-            rate -= (yhi.flux - ylo.flux) * ihy;
-            if constexpr (kLimited) rate -= (yhi.extra - ylo.extra) * ihy;
-          }
-          if constexpr (kAffine) rate += cur.src[s] - (cur.los[s] * c);
+          float rate = strip_rate<kLimited>(P, P.diffusion[s], c, prev.c[s], next.c[s], ylo_v,
+                                            yhi_v, xlo, xhi, ylo, yhi, open_xlo, open_xhi,
+                                            open_ylo, open_yhi, ihx, ihy);
+          if constexpr (kAffine) rate += own.src[s] - (own.los[s] * c);
           if (monod) {
-            const float uptake = P.vmax[s] * cur.phi / (P.monod_k[s] + c);
+            const float uptake = P.vmax[s] * own.phi / (P.monod_k[s] + c);
             rate += 0.0f - (uptake * c);
           }
           v = c + (dt * rate);
@@ -351,23 +235,23 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
           double rate = 0.0, supply = 0.0;
           // A flux through an edge of the grid is supplied from outside.
           if (nx != 1) {
-            if (xx == 0 && !xper) supply += xlo.flux * ihx;
-            if (xx + 1 == static_cast<int>(nx) && !xper) supply -= xhi.flux * ihx;
+            if (xx == 0 && !at.xper) supply += xlo.flux * ihx;
+            if (xx + 1 == static_cast<int>(nx) && !at.xper) supply -= xhi.flux * ihx;
             rate -= (xhi.flux - xlo.flux) * ihx;
           }
           if (ny != 1) {
-            if (col == 0 && !yper) supply += ylo.flux * ihy;
-            if (col + 1 == static_cast<int>(ny) && !yper) supply -= yhi.flux * ihy;
+            if (col == 0 && !at.yper) supply += ylo.flux * ihy;
+            if (col + 1 == static_cast<int>(ny) && !at.yper) supply -= yhi.flux * ihy;
             rate -= (yhi.flux - ylo.flux) * ihy;
           }
           double lossr = 0.0;
           if constexpr (kAffine) {
-            rate += static_cast<double>(cur.src[s]);
-            supply += static_cast<double>(cur.src[s]);
-            lossr += static_cast<double>(cur.los[s]);
+            rate += static_cast<double>(own.src[s]);
+            supply += static_cast<double>(own.src[s]);
+            lossr += static_cast<double>(own.los[s]);
           }
           if (monod) {
-            lossr += static_cast<double>(P.vmax[s]) * static_cast<double>(cur.phi) /
+            lossr += static_cast<double>(P.vmax[s]) * static_cast<double>(own.phi) /
                      (static_cast<double>(P.monod_k[s]) + c);
           }
           rate -= lossr * c;
@@ -392,6 +276,8 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_step(
           out[s * n + i] = v;
         }
       }
+      own = own_next;
+      own_next = own_ahead;
       prev = cur;
       cur = next;
       if constexpr (kLimited) {
@@ -532,31 +418,6 @@ __global__ __launch_bounds__(kAdrBlock) void k_adr_survey(
       st->peak = outflow[0];
     }
   }
-}
-
-// Launch shape of the marching step: strips of one wave, four waves per block,
-// 12 x-rows per wave, or 8 or 4 on smaller grids for at least 4096 waves (one
-// round of 16 per compute unit). At 4096x2048 with three signals (FP64 upwind,
-// FP32 upwind, FP32 van Leer) 12 rows take 131, 74 and 109 us, 8 rows 135, 77
-// and 111, 16 rows 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows 151, 78
-// and 111: longer walks read fewer rows twice but leave a last round of waves
-// nearly empty. At 1531x769 (two signals) 4 rows instead of 8: 19.5 for 20.5
-// us FP64, 20.8 for 22.9 van Leer.
-struct AdrShape {
-  uint32_t strips, rows, blocks;
-};
-
-AdrShape adr_shape(uint32_t strips, uint32_t nx, uint32_t rows) {
-  constexpr uint32_t kWaves = kAdrBlock / kWave;
-  return AdrShape{strips, rows, (strips * ((nx + rows - 1) / rows) + kWaves - 1) / kWaves};
-}
-
-AdrShape adr_shape(uint32_t nx, uint32_t ny, bool limited) {
-  const uint32_t width = static_cast<uint32_t>(kWave) - (limited ? 4 : 2);
-  const uint32_t strips = (ny + width - 1) / width;
-  uint32_t rows = 12;
-  while (rows > 4 && static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows) < 4096) rows -= 4;
-  return adr_shape(strips, nx, rows);
 }
 
 uint32_t site_blocks(size_t n) { return static_cast<uint32_t>((n + kAdrBlock - 1) / kAdrBlock); }

@@ -81,16 +81,17 @@ void download_enter() { g_slots.enter(); }
 void download_leave() { g_slots.leave(); }
 
 void download(Context& ctx, void* dst, const void* src, size_t bytes, const char* what) {
-  const size_t chunks = (bytes + kSlotBytes - 1) / kSlotBytes;
-  const size_t cores = std::max<size_t>(std::thread::hardware_concurrency(), 1);
-  std::vector<void*> slots;
-  if (bytes >= kThreadedBytes && cores > 1)
-    slots = g_slots.take(std::min({kMostThreads, cores, chunks}));
-  if (slots.size() < 2) {
-    g_slots.give(slots);
+  auto plain = [&] {
     check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx.stream), what);
     check(hipStreamSynchronize(ctx.stream), what);
-    return;
+  };
+  if (bytes < kThreadedBytes) return plain();
+  const size_t chunks = (bytes + kSlotBytes - 1) / kSlotBytes;
+  const size_t cores = std::max<size_t>(std::thread::hardware_concurrency(), 1);
+  const std::vector<void*> slots = g_slots.take(std::min({kMostThreads, cores, chunks}));
+  if (slots.size() < 2) {
+    g_slots.give(slots);
+    return plain();
   }
   // Every chunk is taken by exactly one thread; whatever fails, all are joined
   // and the slots go back only after the stream has drained.

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "adr_site.hpp"
+#include "adr_strip.hpp"
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -31,6 +32,7 @@ namespace msim {
 namespace {
 
 constexpr int kImplicitBlock = 256;
+constexpr int kJudgeBlock = 1024;        // of the two single-block kernels
 constexpr uint32_t kImplicitBatch = 16;  // iterations between host checks
 
 // The iteration's site work shared by the setup and the sweep: the site's
@@ -185,146 +187,153 @@ __global__ __launch_bounds__(kImplicitBlock) void k_implicit_setup(
 
 // One Jacobi iteration (signals.cpp:1348-1373) from iterate `cur`: per fluid
 // level the operator rate, the residual rhs - c + half_dt * rate (its square
-// summed per block) and the damped update into `nxt`. Levels at obstacle
-// sites are never written. A non-finite level of the iterate is recorded: the
-// reference refuses to take the rates of such levels.
+// summed per block) and the damped update into `nxt`, which at obstacle sites
+// takes cur's level, so every iterate is whole. A non-finite level of the
+// iterate is recorded (the reference refuses to take the rates of such
+// levels), and per block whether it holds a negative one, for the step's
+// validation. Each wave walks a strip (adr_strip.hpp), as the explicit step:
+// at 2048x1024 with three signals 32.7 us (3.65 TB/s of 57 B per site) and
+// 1088 partials for the decision (4.8 us); one thread per site with every
+// neighbour loaded took 35.0 us and left 8192 (9.6 us).
 template <int S, bool kLimited, bool kPatched>
-__global__ __launch_bounds__(kImplicitBlock) void k_implicit_sweep(
+__global__ __launch_bounds__(kStripBlock) void k_implicit_sweep(
     AdrParams P, const uint8_t* __restrict__ solid, const float* __restrict__ xf,
     const float* __restrict__ yf, const float* __restrict__ source, const float* __restrict__ loss,
-    const float* __restrict__ rhs, const float* __restrict__ cur, float* __restrict__ nxt,
-    float half_dt, float relaxation, ImplicitState* state, double* __restrict__ sums) {
-  __shared__ double s_red[kImplicitBlock / kWave];
+    const float* __restrict__ rhs, const float* __restrict__ cur_levels, float* __restrict__ nxt,
+    float half_dt, float relaxation, uint32_t rows, uint32_t strips, ImplicitState* state,
+    double* __restrict__ sums, float* __restrict__ negatives) {
+  using Lane = Strip<kLimited, kPatched>;
+  using Row = StripRow<float, S>;
+  using Face = StripFace<float>;
+  __shared__ double s_red[kStripWaves];
+  __shared__ uint32_t s_negative;
   if (state->halted != 0) return;
-  const uint32_t nx = P.nx, ny = P.ny;
-  const size_t n = static_cast<size_t>(nx) * ny;
-  const size_t i = static_cast<size_t>(blockIdx.x) * kImplicitBlock + threadIdx.x;
+  if (threadIdx.x == 0) s_negative = 0;
+  const Lane at(P, xcd_tile(blockIdx.x, gridDim.x) * kStripWaves + threadIdx.x / kWave, strips,
+                rows);
+  const int xa = at.xa, xb = at.xb;
+  const uint32_t nx = at.nx, ny = at.ny, y = at.y;
+  const size_t n = at.n;
+  const bool owns = at.owns, field = at.field;
   const bool affine = P.has_affine != 0, reaction = affine || P.has_monod != 0;
+  auto load = [&](int xx, bool full) {
+    return at.template load<float, S>(xx, full, solid, xf, yf, cur_levels);
+  };
+  struct Extra {
+    float b[S], L[S], q[S];
+  };
+  auto load_extra = [&](int xx) {
+    Extra w{};
+    if (xx >= xb || !owns) return w;
+    const size_t i = static_cast<size_t>(xx) * ny + y;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      w.b[s] = rhs[s * n + i];
+      if (reaction) w.L[s] = loss[s * n + i];
+      if (affine) w.q[s] = source[s * n + i];
+    }
+    return w;
+  };
+  const float ihx = 1.0f / P.dx, ihy = 1.0f / P.dy;
+  auto face = [&](float a, float b, float velocity, float ih, bool open, float far_a, float far_b,
+                  uint32_t lim, uint32_t lim_a, uint32_t lim_b) {
+    return strip_face<kLimited, float>(a, b, velocity, 0.0f, ih, open, far_a, far_b, lim, lim_a,
+                                       lim_b);
+  };
   double acc = 0.0;
-  bool bad = false;
-  if constexpr (!kLimited) {
-    // Upwind: every level this site reads is loaded before any is used, so a
-    // wave has all of its loads in flight at once; then the same arithmetic
-    // as the general path below.
-    if (i < n && solid[i] == 0) {
-      const uint32_t x = static_cast<uint32_t>(i / ny), y = static_cast<uint32_t>(i % ny);
-      const size_t row = static_cast<size_t>(x) * ny;
-      const size_t at[4] = {x == 0 ? static_cast<size_t>(nx - 1) * ny + y : i - ny,
-                            x + 1 == nx ? static_cast<size_t>(y) : i + ny,
-                            y == 0 ? row + ny - 1 : i - 1, y + 1 == ny ? row : i + 1};
-      float c[S], nb[S][4], b[S], L[S], q[S];
+  bool bad = false, negative = false;
+  if (xa < xb) {
+    Row prev = load(xa - 1, false);
+    Row cur = load(xa, true);
+    Row next = load(xa + 1, xa + 1 < xb);
+    Row n2 = kLimited ? load(xa + 2, xa + 2 < xb) : Row{};
+    Extra own = load_extra(xa), own_next = load_extra(xa + 1);
+    Face below[S];
+    {
+      const Row p2 = kLimited ? load(xa - 2, false) : Row{};
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        const float* lv = cur + s * n;
-        c[s] = lv[i];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) nb[s][k] = lv[at[k]];
-        b[s] = rhs[s * n + i];
-        L[s] = reaction ? loss[s * n + i] : 0.0f;
-        q[s] = affine ? source[s * n + i] : 0.0f;
+        below[s] = face(prev.c[s], cur.c[s], field ? cur.ux : P.advection[s][0], ihx,
+                        (prev.site & cur.site & kOpen) != 0, p2.c[s], next.c[s],
+                        prev.site & cur.site, p2.site, next.site);
       }
-      const SiteGeometry base = geometry(P, solid, xf, yf, x, y, 0);
+    }
+    for (int xx = xa; xx < xb; ++xx) {
+      constexpr int kAhead = kLimited ? 3 : 2;
+      const Row ahead =
+          xx + kAhead < xb + Lane::kHalo ? load(xx + kAhead, xx + kAhead < xb) : Row{};
+      const Extra own_ahead = load_extra(xx + 2);
+      const size_t i = static_cast<size_t>(xx) * ny + y;
+      const uint32_t site_lo = site_below(cur.site), site_hi = site_above(cur.site);
+      const bool open_xlo = (prev.site & cur.site & kOpen) != 0;
+      const bool open_xhi = (cur.site & next.site & kOpen) != 0;
+      const bool open_ylo = (site_lo & cur.site & kOpen) != 0;
+      const bool open_yhi = (cur.site & site_hi & kOpen) != 0;
+      [[maybe_unused]] uint32_t site_lo2 = 0;
+      if constexpr (kLimited) site_lo2 = site_below(site_lo);
+      const bool fluid = (cur.site & kOpen) != 0;
+      const float uy_hi = lane_above(cur.uy);
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        SiteGeometry g = base;
-        if (P.has_field == 0) {
-          g.ulo[0] = g.uup[0] = P.advection[s][0];
-          g.ulo[1] = g.uup[1] = P.advection[s][1];
-        }
-        const float v = c[s];
-        if (!isfinite(v)) bad = true;
-        const float l0 = x == 0 ? exterior<kPatched>(P, 0, s, v, nb[s][0], y) : nb[s][0];
-        const float u0 = x + 1 == nx ? exterior<kPatched>(P, 1, s, v, nb[s][1], y) : nb[s][1];
-        const float l1 = y == 0 ? exterior<kPatched>(P, 2, s, v, nb[s][2], x) : nb[s][2];
-        const float u1 = y + 1 == ny ? exterior<kPatched>(P, 3, s, v, nb[s][3], x) : nb[s][3];
-        float rate = transport_rate_f32<false>(P, g, v, l0, u0, l1, u1, s);
-        if (reaction) rate += q[s] - (L[s] * v);
-        const float r = (b[s] - v) + (half_dt * rate);
-        acc += static_cast<double>(r) * static_cast<double>(r);
-        const float diagonal = operator_diagonal_f32(P, g, s, reaction, L[s]);
+        const float v = cur.c[s];
+        const float ylo_v = lane_below(v), yhi_v = lane_above(v);
+        [[maybe_unused]] float far_lo = 0.0f;
+        if constexpr (kLimited) far_lo = lane_below(ylo_v);
+        SiteGeometry g;
+        g.clo[0] = !open_xlo;
+        g.cup[0] = !open_xhi;
+        g.clo[1] = !open_ylo;
+        g.cup[1] = !open_yhi;
+        g.ulo[0] = field ? cur.ux : P.advection[s][0];
+        g.uup[0] = field ? next.ux : P.advection[s][0];
+        g.ulo[1] = field ? cur.uy : P.advection[s][1];
+        g.uup[1] = field ? uy_hi : P.advection[s][1];
+        const Face xlo = below[s];
+        const Face xhi = face(v, next.c[s], g.uup[0], ihx, open_xhi, prev.c[s], n2.c[s],
+                              cur.site & next.site, prev.site, n2.site);
+        below[s] = xhi;
+        const Face ylo = face(ylo_v, v, g.ulo[1], ihy, open_ylo, far_lo, yhi_v,
+                              site_lo & cur.site, site_lo2, site_hi);
+        Face yhi;
+        yhi.flux = lane_above(ylo.flux);
+        yhi.extra = kLimited ? lane_above(ylo.extra) : 0.0f;
+        float rate = strip_rate<kLimited>(P, P.diffusion[s], v, prev.c[s], next.c[s], ylo_v,
+                                          yhi_v, xlo, xhi, ylo, yhi, open_xlo, open_xhi, open_ylo,
+                                          open_yhi, ihx, ihy);
+        if (reaction) rate += own.q[s] - (own.L[s] * v);
+        const float r = (own.b[s] - v) + (half_dt * rate);
+        const float diagonal = operator_diagonal_f32(P, g, s, reaction, own.L[s]);
         const float remainder = rate - (diagonal * v);
-        const float update = (b[s] + (half_dt * remainder)) / (1.0f - (half_dt * diagonal));
-        nxt[s * n + i] = v + (relaxation * (update - v));
+        const float update =
+            (own.b[s] + (half_dt * remainder)) / (1.0f - (half_dt * diagonal));
+        if (owns) {
+          if (fluid) {
+            acc += static_cast<double>(r) * static_cast<double>(r);
+            bad = bad || !isfinite(v);
+            negative = negative || v < 0.0f;
+          }
+          nxt[s * n + i] = fluid ? v + (relaxation * (update - v)) : v;
+        }
       }
-    }
-  } else if (i < n && solid[i] == 0) {
-    // van Leer: the same, with the four sites two away (site_limiter's, in
-    // adr_site.hpp) loaded up front as well.
-    const uint32_t x = static_cast<uint32_t>(i / ny), y = static_cast<uint32_t>(i % ny);
-    const size_t row = static_cast<size_t>(x) * ny;
-    const size_t at[4] = {x == 0 ? static_cast<size_t>(nx - 1) * ny + y : i - ny,
-                          x + 1 == nx ? static_cast<size_t>(y) : i + ny,
-                          y == 0 ? row + ny - 1 : i - 1, y + 1 == ny ? row : i + 1};
-    const bool xp3 = P.kind[0] == MSIM_PERIODIC && nx >= 3;
-    const bool yp3 = P.kind[2] == MSIM_PERIODIC && ny >= 3;
-    // Far sites: x - 2, x + 2, y - 2, y + 2 (wrapped on a periodic axis of at
-    // least three sites, absent past a boundary otherwise).
-    size_t far_at[4];
-    bool far_in[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int axis = k >> 1;
-      const int64_t count = axis == 0 ? nx : ny;
-      const int64_t along = static_cast<int64_t>(axis == 0 ? x : y) + ((k & 1) ? 2 : -2);
-      far_in[k] = (axis == 0 ? xp3 : yp3) || (along >= 0 && along < count);
-      const uint32_t wrapped = static_cast<uint32_t>(((along % count) + count) % count);
-      far_at[k] = axis == 0 ? static_cast<size_t>(wrapped) * ny + y : row + wrapped;
-    }
-    bool far_open[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) far_open[k] = far_in[k] && solid[far_at[k]] == 0;
-    float c[S], nb[S][4], fv[S][4], b[S], L[S], q[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const float* lv = cur + s * n;
-      c[s] = lv[i];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        nb[s][k] = lv[at[k]];
-        fv[s][k] = far_in[k] ? lv[far_at[k]] : 0.0f;
+      own = own_next;
+      own_next = own_ahead;
+      prev = cur;
+      cur = next;
+      if constexpr (kLimited) {
+        next = n2;
+        n2 = ahead;
+      } else {
+        next = ahead;
       }
-      b[s] = rhs[s * n + i];
-      L[s] = reaction ? loss[s * n + i] : 0.0f;
-      q[s] = affine ? source[s * n + i] : 0.0f;
-    }
-    const SiteGeometry base = geometry(P, solid, xf, yf, x, y, 0);
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      SiteGeometry g = base;
-      if (P.has_field == 0) {
-        g.ulo[0] = g.uup[0] = P.advection[s][0];
-        g.ulo[1] = g.uup[1] = P.advection[s][1];
-      }
-      const float v = c[s];
-      if (!isfinite(v)) bad = true;
-      const float l0 = x == 0 ? exterior<kPatched>(P, 0, s, v, nb[s][0], y) : nb[s][0];
-      const float u0 = x + 1 == nx ? exterior<kPatched>(P, 1, s, v, nb[s][1], y) : nb[s][1];
-      const float l1 = y == 0 ? exterior<kPatched>(P, 2, s, v, nb[s][2], x) : nb[s][2];
-      const float u1 = y + 1 == ny ? exterior<kPatched>(P, 3, s, v, nb[s][3], x) : nb[s][3];
-      Limiter<float> lim;
-      lim.lower_site[0] = !g.clo[0] && (x > 0 || xp3);
-      lim.upper_site[0] = !g.cup[0] && (x + 1 < nx || xp3);
-      lim.lower_site[1] = !g.clo[1] && (y > 0 || yp3);
-      lim.upper_site[1] = !g.cup[1] && (y + 1 < ny || yp3);
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        lim.far_lo_ok[a] = far_open[2 * a];
-        lim.far_hi_ok[a] = far_open[2 * a + 1];
-        lim.far_lo[a] = far_open[2 * a] ? fv[s][2 * a] : 0.0f;
-        lim.far_hi[a] = far_open[2 * a + 1] ? fv[s][2 * a + 1] : 0.0f;
-      }
-      float rate = transport_rate_f32<true>(P, g, v, l0, u0, l1, u1, s, &lim);
-      if (reaction) rate += q[s] - (L[s] * v);
-      const float r = (b[s] - v) + (half_dt * rate);
-      acc += static_cast<double>(r) * static_cast<double>(r);
-      const float diagonal = operator_diagonal_f32(P, g, s, reaction, L[s]);
-      const float remainder = rate - (diagonal * v);
-      const float update = (b[s] + (half_dt * remainder)) / (1.0f - (half_dt * diagonal));
-      nxt[s * n + i] = v + (relaxation * (update - v));
     }
   }
-  const double total = block_sum<kImplicitBlock>(acc, s_red);
-  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+  __syncthreads();
+  if (negative) s_negative = 1;
+  const double total = block_sum<kStripBlock>(acc, s_red);
+  if (threadIdx.x == 0) {
+    sums[blockIdx.x] = total;
+    negatives[blockIdx.x] = s_negative != 0 ? 1.0f : 0.0f;
+  }
   if (bad) atomicOr(&state->nonfinite, 1u);
 }
 
@@ -332,24 +341,24 @@ __global__ __launch_bounds__(kImplicitBlock) void k_implicit_sweep(
 // max(1, 1 - half_dt * least diagonal) (SignalGridLayout::
 // implicit_operator_scale, signals.cpp:823-825) from the setup's partials;
 // resets the solve's state.
-__global__ __launch_bounds__(kImplicitBlock) void k_implicit_begin(
+__global__ __launch_bounds__(kJudgeBlock) void k_implicit_begin(
     const double* __restrict__ sums, const float* __restrict__ least, uint32_t blocks,
     double levels, float half_dt, ImplicitState* state) {
-  __shared__ double s_red[kImplicitBlock / kWave];
-  __shared__ float s_min[kImplicitBlock / kWave];
+  __shared__ double s_red[kJudgeBlock / kWave];
+  __shared__ float s_min[kJudgeBlock / kWave];
   double v = 0.0;
   float m = 0.0f;
-  for (uint32_t b = threadIdx.x; b < blocks; b += kImplicitBlock) {
+  for (uint32_t b = threadIdx.x; b < blocks; b += kJudgeBlock) {
     v += sums[b];
     m = fminf(m, least[b]);
   }
-  v = block_sum<kImplicitBlock>(v, s_red);
+  v = block_sum<kJudgeBlock>(v, s_red);
 #pragma unroll
   for (int offset = 32; offset > 0; offset >>= 1) m = fminf(m, __shfl_xor(m, offset, kWave));
   if ((threadIdx.x & (kWave - 1)) == 0) s_min[threadIdx.x / kWave] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 0; w < kImplicitBlock / kWave; ++w) m = fminf(m, s_min[w]);
+    for (int w = 0; w < kJudgeBlock / kWave; ++w) m = fminf(m, s_min[w]);
     state->rhs_rms = static_cast<float>(sqrt(v / levels));
     const float scaled = 1.0f - (half_dt * m);
     state->scale = scaled > 1.0f ? scaled : 1.0f;
@@ -359,6 +368,7 @@ __global__ __launch_bounds__(kImplicitBlock) void k_implicit_begin(
     state->converged = 0;
     state->iteration = 0;
     state->nonfinite = 0;
+    state->negative = 0;
   }
 }
 
@@ -366,15 +376,26 @@ __global__ __launch_bounds__(kImplicitBlock) void k_implicit_begin(
 // the residual RMS from the sweep's partials; at k = 0 the threshold
 // max(absolute, eps * rhs RMS * scale) + relative * RMS; stop converged when
 // the RMS meets it, unconverged when it (or the threshold) is not finite.
-__global__ __launch_bounds__(kImplicitBlock) void k_implicit_decide(
-    const double* __restrict__ sums, uint32_t blocks, double levels, uint32_t k,
-    float absolute_tolerance, float relative_tolerance, ImplicitState* state) {
-  __shared__ double s_red[kImplicitBlock / kWave];
+// negatives: per block whether the iterate holds a negative level, or null.
+__global__ __launch_bounds__(kJudgeBlock) void k_implicit_decide(
+    const double* __restrict__ sums, const float* __restrict__ negatives, uint32_t blocks,
+    double levels, uint32_t k, float absolute_tolerance, float relative_tolerance,
+    ImplicitState* state) {
+  __shared__ double s_red[kJudgeBlock / kWave];
+  __shared__ uint32_t s_negative;
   if (state->halted != 0) return;
+  if (threadIdx.x == 0) s_negative = 0;
+  __syncthreads();
   double v = 0.0;
-  for (uint32_t b = threadIdx.x; b < blocks; b += kImplicitBlock) v += sums[b];
-  v = block_sum<kImplicitBlock>(v, s_red);
+  bool negative = false;
+  for (uint32_t b = threadIdx.x; b < blocks; b += kJudgeBlock) {
+    v += sums[b];
+    negative = negative || (negatives != nullptr && negatives[b] != 0.0f);
+  }
+  if (negative) s_negative = 1;
+  v = block_sum<kJudgeBlock>(v, s_red);
   if (threadIdx.x != 0) return;
+  state->negative = s_negative;
   const float rms = static_cast<float>(sqrt(v / levels));
   state->rms = rms;
   state->iteration = k;
@@ -431,7 +452,7 @@ void launch_setup(Context& ctx, uint32_t blocks, const float* xf, const float* y
 }
 
 template <int S, bool kLimited, bool kPatched>
-void launch_sweep(Context& ctx, uint32_t blocks, const float* xf, const float* yf,
+void launch_sweep(Context& ctx, uint32_t blocks, const AdrShape& shape, const float* xf, const float* yf,
                   const float* cur, float* nxt, float half_dt, float relaxation) {
   auto& a = ctx.adr;
   if (a.params.nz > 1) {
@@ -439,9 +460,10 @@ void launch_sweep(Context& ctx, uint32_t blocks, const float* xf, const float* y
     return;
   }
   const float* loss = a.params.has_monod != 0 ? a.lagged.data() : a.loss.data();
-  k_implicit_sweep<S, kLimited, kPatched><<<blocks, kImplicitBlock, 0, ctx.stream>>>(
+  k_implicit_sweep<S, kLimited, kPatched><<<shape.blocks, kStripBlock, 0, ctx.stream>>>(
       a.params, a.solid.data(), xf, yf, a.source.data(), loss, a.rhs.data(), cur, nxt, half_dt,
-      relaxation, a.implicit_state.data(), a.implicit_sums.data());
+      relaxation, shape.rows, shape.strips, a.implicit_state.data(), a.implicit_sums.data(),
+      a.implicit_least.data());
 }
 
 template <int S, bool kLimited, bool kPatched>
@@ -456,24 +478,31 @@ void implicit_steps(Context& ctx, float dt, uint32_t steps, const float* xf, con
   const float half_dt = (backward ? 1.0f : 0.5f) * dt;
   const float explicit_dt = backward ? 0.0f : half_dt;
   const float relaxation = kLimited ? 0.5f : 1.0f;
-  float* base[2] = {reinterpret_cast<float*>(a.levels_a.data()),
-                    reinterpret_cast<float*>(a.levels_b.data())};
-  float* third = reinterpret_cast<float*>(a.levels_c.data());
+  // The sweeps of several layers (adr3.hip) leave a partial per `blocks` and
+  // neither write obstacle sites nor look for negative levels.
+  const bool layered = a.params.nz > 1;
+  const AdrShape shape = adr_shape(a.params.nx, a.params.ny, kLimited);
+  const uint32_t parts_swept = layered ? blocks : shape.blocks;
   for (uint32_t step = 0; step < steps; ++step) {
     // The step's levels stay untouched in `old` until it is accepted: the
     // iterates alternate between the two other buffers, iterate k (k >= 1)
-    // in work[k & 1]. Both start as copies, so they hold the levels of the
-    // obstacle sites, which no kernel writes.
+    // in work[k & 1].
+    float* base[2] = {reinterpret_cast<float*>(a.levels_a.data()),
+                      reinterpret_cast<float*>(a.levels_b.data())};
+    float* third = reinterpret_cast<float*>(a.levels_c.data());
     float* old = base[a.current];
     float* work[2] = {third, base[a.current ^ 1]};
-    for (float* w : work) {
-      check(hipMemcpyAsync(w, old, count * sizeof(float), hipMemcpyDeviceToDevice, ctx.stream),
-            "copy levels");
+    if (layered) {
+      // Both start as copies: they hold the levels of the obstacle sites.
+      for (float* w : work) {
+        check(hipMemcpyAsync(w, old, count * sizeof(float), hipMemcpyDeviceToDevice, ctx.stream),
+              "copy levels");
+      }
     }
     auto iterate = [&](uint32_t k) { return k == 0 ? old : work[k & 1u]; };
     launch_setup<S, kLimited, kPatched>(ctx, blocks, xf, yf, sources, old, explicit_dt, dt);
     check(hipGetLastError(), "launch k_implicit_setup");
-    k_implicit_begin<<<1, kImplicitBlock, 0, ctx.stream>>>(
+    k_implicit_begin<<<1, kJudgeBlock, 0, ctx.stream>>>(
         a.implicit_sums.data(), a.implicit_least.data(), blocks, levels, half_dt,
         a.implicit_state.data());
     check(hipGetLastError(), "launch k_implicit_begin");
@@ -489,12 +518,12 @@ void implicit_steps(Context& ctx, float dt, uint32_t steps, const float* xf, con
           std::min<uint64_t>(static_cast<uint64_t>(k) + batch - 1, a.max_iterations));
       batch = kImplicitBatch;
       for (; k <= last; ++k) {
-        launch_sweep<S, kLimited, kPatched>(ctx, blocks, xf, yf, iterate(k), work[(k + 1) & 1u],
-                                            half_dt, relaxation);
+        launch_sweep<S, kLimited, kPatched>(ctx, blocks, shape, xf, yf, iterate(k),
+                                            work[(k + 1) & 1u], half_dt, relaxation);
         check(hipGetLastError(), "launch k_implicit_sweep");
-        k_implicit_decide<<<1, kImplicitBlock, 0, ctx.stream>>>(
-            a.implicit_sums.data(), blocks, levels, k, a.absolute_tolerance,
-            a.relative_tolerance, a.implicit_state.data());
+        k_implicit_decide<<<1, kJudgeBlock, 0, ctx.stream>>>(
+            a.implicit_sums.data(), layered ? nullptr : a.implicit_least.data(), parts_swept,
+            levels, k, a.absolute_tolerance, a.relative_tolerance, a.implicit_state.data());
         check(hipGetLastError(), "launch k_implicit_decide");
       }
       check(hipMemcpyAsync(&host, a.implicit_state.data(), sizeof(host), hipMemcpyDeviceToHost,
@@ -522,26 +551,29 @@ void implicit_steps(Context& ctx, float dt, uint32_t steps, const float* xf, con
     }
     if (host.iteration == 0) continue;  // the levels already met the rule
     // accept_step (signals.cpp:1003-1011): the settle under van Leer, then
-    // the levels' validation, in place on the accepted iterate.
+    // the levels' validation, in place on the accepted iterate. The sweep that
+    // judged it has seen every level: finite ones with none below zero stand
+    // as they are, and upwind has nothing to settle.
     float* accepted = work[host.iteration & 1u];
-    const uint32_t parts = static_cast<uint32_t>(std::min<size_t>((count + 255) / 256, 1024));
-    if (kLimited) {
-      k_level_max<<<parts, kImplicitBlock, 0, ctx.stream>>>(accepted, count, a.partials.data());
-      check(hipGetLastError(), "launch k_level_max");
+    if (layered || (kLimited && host.negative != 0)) {
+      const uint32_t parts = static_cast<uint32_t>(std::min<size_t>((count + 255) / 256, 1024));
+      if (kLimited) {
+        k_level_max<<<parts, kImplicitBlock, 0, ctx.stream>>>(accepted, count, a.partials.data());
+        check(hipGetLastError(), "launch k_level_max");
+      }
+      launch_settle_f32(ctx, accepted, count, a.partials.data(), kLimited ? parts : 0, step);
+      uint32_t flags[2] = {0, 0};
+      check(hipMemcpyAsync(flags, a.flags.data(), sizeof(flags), hipMemcpyDeviceToHost,
+                           ctx.stream),
+            "read flags");
+      check(hipStreamSynchronize(ctx.stream), "settle");
+      host.negative = flags[0];
     }
-    launch_settle_f32(ctx, accepted, count, a.partials.data(), kLimited ? parts : 0, step);
-    uint32_t flags[2] = {0, 0};
-    check(hipMemcpyAsync(flags, a.flags.data(), sizeof(flags), hipMemcpyDeviceToHost, ctx.stream),
-          "read flags");
-    check(hipStreamSynchronize(ctx.stream), "settle");
-    if (flags[0] != 0) {
+    if (host.negative != 0) {
       throw Error(MSIM_INVALID_ARGUMENT, "signal grid levels must be finite and non-negative");
     }
-    if (accepted == third) {
-      check(hipMemcpyAsync(base[a.current ^ 1], third, count * sizeof(float),
-                           hipMemcpyDeviceToDevice, ctx.stream),
-            "copy accepted levels");
-    }
+    // The accepted iterate becomes the other level buffer.
+    if (accepted == third) a.levels_c.swap(a.current == 0 ? a.levels_b : a.levels_a);
     a.current ^= 1;
   }
 }
@@ -570,8 +602,9 @@ void implicit_run(Context& ctx, float dt, uint32_t steps, const float* xf, const
   a.rhs.reserve(static_cast<size_t>(a.params.signals) * n);
   a.levels_c.reserve(static_cast<size_t>(a.params.signals) * n * sizeof(float));
   if (a.params.has_monod != 0) a.lagged.reserve(static_cast<size_t>(a.params.signals) * n);
-  a.implicit_sums.reserve(blocks);
-  a.implicit_least.reserve(blocks);
+  const uint32_t swept = adr_shape(a.params.nx, a.params.ny, a.params.limited != 0).blocks;
+  a.implicit_sums.reserve(std::max(blocks, swept));
+  a.implicit_least.reserve(std::max(blocks, swept));
   a.implicit_state.reserve(1);
   switch (a.params.signals) {
     case 1: implicit_typed<1>(ctx, dt, steps, xf, yf, sources, label); break;

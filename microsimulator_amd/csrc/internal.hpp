@@ -12,6 +12,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "msim_hip.h"
@@ -59,6 +60,11 @@ class DeviceBuffer {
     data_ = nullptr;
     capacity_ = 0;
     count_ = 0;
+  }
+  void swap(DeviceBuffer& other) noexcept {
+    std::swap(data_, other.data_);
+    std::swap(capacity_, other.capacity_);
+    std::swap(count_, other.count_);
   }
   [[nodiscard]] T* data() const noexcept { return data_; }
   [[nodiscard]] std::size_t size() const noexcept { return count_; }
@@ -266,6 +272,7 @@ struct ImplicitState {
   uint32_t converged;
   uint32_t iteration;  // the last iterate judged
   uint32_t nonfinite;  // an iterate held a non-finite level
+  uint32_t negative;   // the last iterate judged holds a negative level (one layer)
 };
 
 struct AdrDevice {

@@ -8,6 +8,7 @@ import microsimulator_amd as msa
 from oracle import VAN_LEER
 from oracle import Grid as OGrid
 from tests.helpers import FIXED, NO_FLUX, PERIODIC, random_transport_case
+from tests.test_gpu_implicit import oracle_kw, same_report, spec_of
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +81,26 @@ def test_settle_of_a_marked_step(hip, oracle):
                                   faces=np.concatenate([xf.reshape(-1), zero_y, zero_z]))
         assert np.array_equal(hip.adr_download(), ref)
     assert ref.min() >= 0.0
+
+
+@pytest.mark.parametrize("limited", [False, True])
+@pytest.mark.parametrize("shape,kinds", [((13, 62), KINDS[0]), ((5, 61), KINDS[1]),
+                                         ((30, 125), KINDS[2]), ((1400, 63), KINDS[0])])
+def test_implicit_steps_at_strip_edges(hip, oracle, shape, kinds, limited):
+    """Several implicit steps on the device (the accepted iterate changes
+    buffers from step to step by its parity) bit for bit with the oracle's,
+    obstacle levels included."""
+    nx, ny = shape
+    c = random_transport_case(nx, ny, 2, kinds, seed=3 * nx + ny)
+    scheme = msa.VAN_LEER if limited else msa.UPWIND
+    og = OGrid(nx, ny, 1, 1.0, 0.5, 1.0, c["solid"], kinds)
+    spec = spec_of(msa.Grid(nx, ny, 1, 1.0, 0.5, 1.0, c["solid"], kinds), c, scheme,
+                   msa.CRANK_NICOLSON)
+    ref = c["levels"].astype(np.float32)
+    hip.adr_upload(spec, ref, precision=32)
+    for dt in (0.02, 0.3, 0.1, 0.01):
+        hip.adr_run(dt, 1, ledger=False)
+        ref, rep = oracle.adr_step_implicit(og, ref, dt,
+                                            **oracle_kw(c, scheme, msa.CRANK_NICOLSON))
+        assert np.array_equal(hip.adr_download(), ref)
+        same_report(hip.adr_report(), rep)
