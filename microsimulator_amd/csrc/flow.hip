@@ -38,21 +38,6 @@ __global__ void k_conductance(const uint8_t* __restrict__ solid, const float* __
   cond[i] = solid[i] != 0 ? 0.0f : dz * mobility[i];
 }
 
-// Whether the exterior face `side` (0 x lower, 1 x upper, 2 y lower, 3 y
-// upper) at in-plane index `along` is open, and the pressure held half a
-// spacing outside it.
-__device__ __forceinline__ bool open_edge(const FlowEdges& e, uint32_t side, uint32_t along,
-                                          uint32_t nx, uint32_t ny, float& pressure) {
-  if (e.open == nullptr) {
-    pressure = (side & 1u) != 0 || e.held_zero != 0 ? 0.0f : 1.0f;
-    return (side >> 1) == e.axis;
-  }
-  const uint32_t slot =
-      along + (side == 0 ? 0u : side == 1 ? ny : side == 2 ? 2u * ny : 2u * ny + nx);
-  pressure = e.held_zero != 0 ? 0.0f : e.pressure[slot];
-  return e.open[slot] != 0;
-}
-
 // ShallowFlowReduction::body_flux (flow_system.hpp:395-420) per face of the
 // grid of columns (x faces, then y faces): the body force integrated across
 // each half cell in series, harm(m_l, m_u) (f_l/2 + f_u/2) on an interior
@@ -117,66 +102,13 @@ __global__ __launch_bounds__(256) void k_forced_rhs(const float* __restrict__ co
   rhs[i] = r;
 }
 
-// Assembly (flow_system.hpp:549-599): diagonal, right-hand side and boundary
-// conductance in the reference's float order (x lower, x upper, y lower,
-// y upper), and the lower-face conductances the operator uses. Each open
-// exterior face adds 2m/h^2 toward the pressure held outside it.
 __global__ void k_assemble(const float* __restrict__ cond, float* __restrict__ diag,
                            float* __restrict__ rhs, float* __restrict__ bc,
                            float* __restrict__ cxl, float* __restrict__ cyl, uint32_t nx,
                            uint32_t ny, float dx, float dy, FlowEdges edges) {
   const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= static_cast<size_t>(nx) * ny) return;
-  const uint32_t x = static_cast<uint32_t>(i / ny);
-  const uint32_t y = static_cast<uint32_t>(i % ny);
-  const float m = cond[i];
-  cxl[i] = x > 0 ? harmonic(m, cond[i - ny]) : 0.0f;
-  cyl[i] = y > 0 ? harmonic(m, cond[i - 1]) : 0.0f;
-  float d = 0.0f, r = 0.0f, b = 0.0f;
-  if (m != 0.0f) {
-    const float isx = 1.0f / (dx * dx);
-    const float isy = 1.0f / (dy * dy);
-    float held = 0.0f;
-    // x lower
-    if (x > 0) {
-      d += harmonic(m, cond[i - ny]) * isx;
-    } else if (open_edge(edges, 0, y, nx, ny, held)) {
-      const float c = 2.0f * m * isx;
-      d += c;
-      b += c;
-      r += c * held;
-    }
-    // x upper
-    if (x + 1 < nx) {
-      d += harmonic(m, cond[i + ny]) * isx;
-    } else if (open_edge(edges, 1, y, nx, ny, held)) {
-      const float c = 2.0f * m * isx;
-      d += c;
-      b += c;
-      r += c * held;
-    }
-    // y lower
-    if (y > 0) {
-      d += harmonic(m, cond[i - 1]) * isy;
-    } else if (open_edge(edges, 2, x, nx, ny, held)) {
-      const float c = 2.0f * m * isy;
-      d += c;
-      b += c;
-      r += c * held;
-    }
-    // y upper
-    if (y + 1 < ny) {
-      d += harmonic(m, cond[i + 1]) * isy;
-    } else if (open_edge(edges, 3, x, nx, ny, held)) {
-      const float c = 2.0f * m * isy;
-      d += c;
-      b += c;
-      r += c * held;
-    }
-  }
-  diag[i] = d;
-  rhs[i] = r;
-  bc[i] = b;
+  assemble_site(cond, diag, rhs, bc, cxl, cyl, i, nx, ny, dx, dy, edges);
 }
 
 // ---------------------------------------------------------------------------

@@ -77,33 +77,14 @@ __global__ void k_mg_dinv(const float* __restrict__ wx, const float* __restrict_
                           const float* __restrict__ bc, float* __restrict__ dinv, uint32_t nx,
                           uint32_t ny) {
   const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= static_cast<size_t>(nx) * ny) return;
-  const uint32_t x = static_cast<uint32_t>(i / ny), y = static_cast<uint32_t>(i % ny);
-  float d = bc[i] + wx[i] + wy[i];
-  if (x + 1 < nx) d += wx[i + ny];
-  if (y + 1 < ny) d += wy[i + 1];
-  dinv[i] = d > 0.0f ? 1.0f / d : 0.0f;
+  if (i < static_cast<size_t>(nx) * ny) dinv[i] = level_dinv(wx, wy, bc, i, nx, ny);
 }
 
-// Galerkin coarse operator of 2x2 aggregation.
 __global__ void k_mg_coarsen(LevelView f, float* __restrict__ wx, float* __restrict__ wy,
                              float* __restrict__ bc, uint32_t nxc, uint32_t nyc) {
   const size_t c = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c >= static_cast<size_t>(nxc) * nyc) return;
-  const uint32_t X = static_cast<uint32_t>(c / nyc), Y = static_cast<uint32_t>(c % nyc);
-  const uint32_t fx = 2 * X, fy = 2 * Y;
-  const bool x1 = fx + 1 < f.nx, y1 = fy + 1 < f.ny;
-  const size_t i = static_cast<size_t>(fx) * f.ny + fy;
-  float cx = 0.0f, cy = 0.0f;
-  if (X > 0) cx = f.wx[i] + (y1 ? f.wx[i + 1] : 0.0f);
-  if (Y > 0) cy = f.wy[i] + (x1 ? f.wy[i + f.ny] : 0.0f);
-  float b = f.bc[i];
-  if (y1) b += f.bc[i + 1];
-  if (x1) b += f.bc[i + f.ny];
-  if (x1 && y1) b += f.bc[i + f.ny + 1];
-  wx[c] = cx;
-  wy[c] = cy;
-  bc[c] = b;
+  if (c < static_cast<size_t>(nxc) * nyc)
+    coarsen_cell(f.wx, f.wy, f.bc, f.nx, f.ny, wx, wy, bc, c, nyc);
 }
 
 // A tile grown by 2 in LDS (kHX2 x kHY2, pitch kHY2): r, the inverse
@@ -1056,34 +1037,6 @@ uint32_t run_fcg(Context& ctx, double rnorm, double tolerance, uint32_t budget, 
 }
 
 }  // namespace
-
-std::vector<float> mg_coarse_inverse(const std::vector<float>& wx, const std::vector<float>& wy,
-                                     const std::vector<float>& bc, uint32_t nx, uint32_t ny) {
-  return coarse_inverse(wx, wy, bc, nx, ny);
-}
-
-void mg_level0_operator(hipStream_t stream, const float* cxl, const float* cyl, const float* bc,
-                        float* wx, float* wy, float* bcl, float* dinv, uint32_t nx, uint32_t ny,
-                        float isx, float isy) {
-  const size_t n = static_cast<size_t>(nx) * ny;
-  const uint32_t blocks = static_cast<uint32_t>((n + 255) / 256);
-  k_mg_level0<<<blocks, 256, 0, stream>>>(cxl, cyl, bc, wx, wy, bcl, n, isx, isy);
-  check(hipGetLastError(), "launch k_mg_level0");
-  k_mg_dinv<<<blocks, 256, 0, stream>>>(wx, wy, bcl, dinv, nx, ny);
-  check(hipGetLastError(), "launch k_mg_dinv");
-}
-
-void mg_coarse_operator(hipStream_t stream, const float* fwx, const float* fwy, const float* fbc,
-                        uint32_t fnx, uint32_t fny, float* wx, float* wy, float* bc, float* dinv,
-                        uint32_t nx, uint32_t ny) {
-  const size_t n = static_cast<size_t>(nx) * ny;
-  const uint32_t blocks = static_cast<uint32_t>((n + 255) / 256);
-  const LevelView f{fwx, fwy, fbc, nullptr, fnx, fny};
-  k_mg_coarsen<<<blocks, 256, 0, stream>>>(f, wx, wy, bc, nx, ny);
-  check(hipGetLastError(), "launch k_mg_coarsen");
-  k_mg_dinv<<<blocks, 256, 0, stream>>>(wx, wy, bc, dinv, nx, ny);
-  check(hipGetLastError(), "launch k_mg_dinv");
-}
 
 void mg_prepare(Context& ctx) {
   auto& f = ctx.flow;
