@@ -77,6 +77,42 @@ def test_batch_flow_matches_the_oracle(hip, oracle):
     assert np.all(it2 <= 2)
 
 
+def odd_instance(nx, ny, pocket):
+    rng = np.random.default_rng([SEED, nx, ny])
+    solid = np.zeros((nx, ny), np.uint8)
+    if nx >= 16 and ny >= 16:
+        solid[5:9, 2:ny // 2] = 1
+    if pocket:  # fluid without an open boundary: zero rows and a vanishing pivot
+        solid[nx // 2:nx // 2 + 7, 8:15] = 1
+        solid[nx // 2 + 2:nx // 2 + 5, 10:13] = 0
+    return msa.BatchInstance(nx=nx, ny=ny, mobility=rng.uniform(0.2, 2.0, nx * ny).astype(np.float32),
+                             obstacles=solid.reshape(-1), inlet_pressure=1.3, dx=1.5, dy=0.75)
+
+
+@pytest.mark.parametrize("sizes", [
+    [(3, 3), (8, 8), (2, 31)],            # one level: the dense inverse alone
+    [(13, 5), (65, 3), (3, 65), (9, 8)],  # one coarsening, odd remainders
+    [(33, 31), (129, 17), (64, 64), (37, 111)],
+])
+@pytest.mark.parametrize("pocket", [False, True])
+def test_batch_system_at_odd_sizes(hip, oracle, sizes, pocket):
+    """The device's setup and cycle at level edges: every instance converges to
+    1e-10 of the oracle's own right-hand side and operator (FP64), in no more
+    iterations than a multilevel cycle needs (a wrong coarse operator or
+    inverse costs hundreds or fails)."""
+    inst = [odd_instance(nx, ny, pocket and nx >= 24 and ny >= 17) for nx, ny in sizes]
+    hip.batch_upload(inst, relative_tolerance=1e-10, max_iterations=4000)
+    it, res, fl = hip.batch_solve_flow()
+    print(sizes, "iterations", it.tolist(), "residuals", res.tolist(), flush=True)
+    assert np.all(fl == 0)
+    for k, i in enumerate(inst):
+        g = ogrid(i)
+        b = oracle.assemble(g, i.mobility, 0)["rhs"].astype(np.float64) * np.float64(np.float32(i.inlet_pressure))
+        true = np.linalg.norm(b - oracle.apply(g, i.mobility, hip.batch_download(k)["pressure"])) / np.linalg.norm(b)
+        assert true <= 1e-10
+        assert it[k] <= 120
+
+
 def test_batch_step_is_the_single_grid_step(hip, oracle):
     inst = small_batch()
     rng = np.random.default_rng(4)
