@@ -25,13 +25,13 @@
 // per instance in a fixed order on the host. A run of steps is captured once
 // into a HIP graph and replayed.
 //
-// The pressure solve itself is one launch with one workgroup per instance
-// (largest first): the refinement loop needs the instance's dot products,
-// and a workgroup reduces them with barriers only. Each FP32 correction is
-// conjugate gradient preconditioned by the instance's own multilevel cycle
-// (2x2 aggregation, V(1,1) damped Jacobi, the coarse correction weighted by
-// 1.8, the coarsest level of <= 64 cells inverted densely): the cycle of the
-// single-grid multilevel form, run level by level inside the workgroup. It is
+// The pressure solve takes one of two forms: one launch with one workgroup per
+// instance (largest first), or launches in which every instance's iteration
+// advances together over the whole chip. Each FP32 correction is conjugate
+// gradient preconditioned by the instance's own multilevel cycle (2x2
+// aggregation, V(1,1) damped Jacobi, the coarse correction weighted by 1.8, the
+// coarsest level of <= 64 cells inverted densely): the cycle of the
+// single-grid multilevel form. It is
 // linear and symmetric positive definite, so plain CG applies.
 //
 // The launch shapes (sites per item; workgroup size and sweep row width of
@@ -94,6 +94,7 @@ struct BatchData {
   float* x;     // FP32 correction of one refinement
   float* r;
   float* p;
+  float* p2;  // the direction before or after p, by turns
   float* q;
   float* xf;
   float* yf;
@@ -133,20 +134,6 @@ __device__ inline void block_sums(double (&v)[K], double* lds) {
 #pragma unroll
   for (int k = 0; k < K; ++k) v[k] = s_out[k];
   __syncthreads();
-}
-
-// The operator (flow_system.hpp:670-695) on an FP32 vector at site i.
-__device__ inline float apply_f32(const float* __restrict__ v, const float* __restrict__ cxl,
-                                  const float* __restrict__ cyl, const float* __restrict__ bc,
-                                  uint32_t x, uint32_t y, uint32_t nx, uint32_t ny, size_t i,
-                                  float isx, float isy) {
-  const float c = v[i];
-  float a = bc[i] * c;
-  if (x > 0) a += (cxl[i] * isx) * (c - v[i - ny]);
-  if (x + 1 < nx) a += (cxl[i + ny] * isx) * (c - v[i + ny]);
-  if (y > 0) a += (cyl[i] * isy) * (c - v[i - 1]);
-  if (y + 1 < ny) a += (cyl[i + 1] * isy) * (c - v[i + 1]);
-  return a;
 }
 
 // b - A x in FP64 at site i, b = inlet * (the assembled Dirichlet-1 rhs).
@@ -239,47 +226,160 @@ __device__ inline LevelRef level_ref(const BatchData& D, const BatchLevels& V, u
 constexpr float kCycleOmega = 0.8f;
 constexpr float kCycleCorrection = 1.8f;
 
-// (A x)_i on a level, x at cell (gx, gy) given by xat, xc its value at i.
-template <class X>
-__device__ inline float level_ax(const LevelRef& L, size_t i, uint32_t x, uint32_t y, float xc,
-                                 X&& xat) {
-  float a = L.bc[i] * xc;
-  if (x > 0) a += L.wx[i] * (xc - xat(x - 1, y));
-  if (x + 1 < L.nx) a += L.wx[i + L.ny] * (xc - xat(x + 1, y));
-  if (y > 0) a += L.wy[i] * (xc - xat(x, y - 1));
-  if (y + 1 < L.ny) a += L.wy[i + 1] * (xc - xat(x, y + 1));
+// A workgroup's pass over the cells [lo, hi): each thread takes U of them, NT
+// apart, and issues all their loads before it uses any, so a pass of few cells
+// per thread is one memory latency and not U of them.
+template <int NT, int U, class Load, class Use>
+__device__ inline void sweep_cells(uint32_t lo, uint32_t hi, Load&& load, Use&& use) {
+  for (uint32_t i0 = lo + threadIdx.x; i0 < hi; i0 += U * NT) {
+    decltype(load(0u)) v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = i0 + static_cast<uint32_t>(u * NT);
+      if (i < hi) v[u] = load(i);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = i0 + static_cast<uint32_t>(u * NT);
+      if (i < hi) use(i, v[u]);
+    }
+  }
+}
+
+// The operator at a cell of a level: its couplings to the four neighbours and
+// its boundary term. The lower couplings are zero on the first row and column
+// (and the first column's are the last column's upper ones), so the neighbours
+// are taken by index alone, clamped to the grid.
+struct CellOp {
+  float xl, xu, yl, yu, b;
+  uint32_t ixl, ixu, iyl, iyu;
+};
+
+__device__ inline CellOp cell_op(const float* wx, const float* wy, const float* bc, uint32_t i,
+                                 uint32_t cells, uint32_t ny) {
+  CellOp o;
+  o.ixl = i >= ny ? i - ny : i;
+  o.ixu = i + ny < cells ? i + ny : i;
+  o.iyl = i >= 1 ? i - 1 : i;
+  o.iyu = i + 1 < cells ? i + 1 : i;
+  o.xl = wx[i];
+  o.xu = i + ny < cells ? wx[i + ny] : 0.0f;
+  o.yl = wy[i];
+  o.yu = i + 1 < cells ? wy[i + 1] : 0.0f;
+  o.b = bc[i];
+  return o;
+}
+
+__device__ inline float cell_apply(const CellOp& o, float c, float xl, float xu, float yl,
+                                   float yu) {
+  float a = o.b * c;
+  a += o.xl * (c - xl);
+  a += o.xu * (c - xu);
+  a += o.yl * (c - yl);
+  a += o.yu * (c - yu);
   return a;
 }
 
-// z = M r on one instance, by the whole workgroup: per level a down pass
-// (pre-smoothing from zero, x = omega D^-1 r, its residual restricted to the
-// next level), the coarsest level's dense inverse, then per level an up pass
-// (x + 1.8 P e_c, post-smoothed). Returns r.z (FP64) in every thread.
+// The cycle's passes over a range of a level's cells. The finest level's
+// x = omega D^-1 r stands in x0 (the pass that leaves r leaves it too); a
+// coarser level's (x0 null) is formed where it is read.
+//
+// Down: the residual of x, restricted to the cells [lo, hi) of the next level.
 template <int NT>
-__device__ double batch_cycle(const BatchData& D, const BatchLevels& V, size_t site, double* lds) {
-  const uint32_t K = V.count - 1;
-  for (uint32_t l = 0; l < K; ++l) {
-    const LevelRef F = level_ref(D, V, l, site);
-    const LevelRef C = level_ref(D, V, l + 1, site);
-    auto pre = [&](uint32_t gx, uint32_t gy) {
-      const size_t j = static_cast<size_t>(gx) * F.ny + gy;
-      return kCycleOmega * F.dinv[j] * F.r[j];
-    };
-    const size_t cells = static_cast<size_t>(C.nx) * C.ny;
-    for (size_t c = threadIdx.x; c < cells; c += NT) {
-      const uint32_t X = static_cast<uint32_t>(c / C.ny), Y = static_cast<uint32_t>(c % C.ny);
-      float sum = 0.0f;
-      for (uint32_t a = 0; a < 2; ++a) {
-        for (uint32_t b = 0; b < 2; ++b) {
-          const uint32_t fx = 2 * X + a, fy = 2 * Y + b;
-          if (fx >= F.nx || fy >= F.ny) continue;
-          const size_t i = static_cast<size_t>(fx) * F.ny + fy;
-          const float xc = kCycleOmega * F.dinv[i] * F.r[i];
-          sum += F.r[i] - level_ax(F, i, fx, fy, xc, pre);
+__device__ inline void cycle_down(const LevelRef& F, const LevelRef& C, const float* x0,
+                                  uint32_t lo, uint32_t hi) {
+  const uint32_t fine = F.nx * F.ny;
+  auto pre = [&](uint32_t j) { return x0 != nullptr ? x0[j] : kCycleOmega * F.dinv[j] * F.r[j]; };
+  struct Quad {
+    float r[4], c[4], n[4][4];
+    CellOp o[4];
+    uint32_t in;
+  };
+  sweep_cells<NT, 1>(
+      lo, hi,
+      [&](uint32_t c) {
+        Quad q;
+        const uint32_t X = c / C.ny, Y = c - X * C.ny;
+        q.in = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+          const uint32_t fx = 2 * X + (k >> 1), fy = 2 * Y + (k & 1);
+          if (fx < F.nx && fy < F.ny) {
+            const uint32_t i = fx * F.ny + fy;
+            q.in |= 1u << k;
+            q.o[k] = cell_op(F.wx, F.wy, F.bc, i, fine, F.ny);
+            q.r[k] = F.r[i];
+            q.c[k] = pre(i);
+            q.n[k][0] = pre(q.o[k].ixl);
+            q.n[k][1] = pre(q.o[k].ixu);
+            q.n[k][2] = pre(q.o[k].iyl);
+            q.n[k][3] = pre(q.o[k].iyu);
+          }
         }
-      }
-      C.r[c] = sum;
-    }
+        return q;
+      },
+      [&](uint32_t c, const Quad& q) {
+        float sum = 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+          if ((q.in >> k) & 1u)
+            sum += q.r[k] - cell_apply(q.o[k], q.c[k], q.n[k][0], q.n[k][1], q.n[k][2], q.n[k][3]);
+        }
+        C.r[c] = sum;
+      });
+}
+
+// Up: x + 1.8 P e_c, post-smoothed, on the cells [lo, hi); their share of z.r
+// joins rz.
+template <int NT>
+__device__ inline void cycle_up(const LevelRef& F, const LevelRef& C, const float* x0, uint32_t lo,
+                                uint32_t hi, double& rz) {
+  const uint32_t cells = F.nx * F.ny;
+  struct Cell {
+    CellOp o;
+    float r, d, c, xl, xu, yl, yu;
+  };
+  sweep_cells<NT, 2>(
+      lo, hi,
+      [&](uint32_t i) {
+        Cell v;
+        const uint32_t x = i / F.ny, y = i - x * F.ny;
+        // The cells over a clamped neighbour: its coupling is zero there.
+        const uint32_t xl = (x > 0 ? x - 1 : 0) / 2, xu = min(x + 1, F.nx - 1) / 2;
+        const uint32_t yl = (y > 0 ? y - 1 : 0) / 2, yu = min(y + 1, F.ny - 1) / 2;
+        auto corrected = [&](uint32_t j, uint32_t X, uint32_t Y) {
+          return (x0 != nullptr ? x0[j] : kCycleOmega * F.dinv[j] * F.r[j]) +
+                 kCycleCorrection * C.e[X * C.ny + Y];
+        };
+        v.o = cell_op(F.wx, F.wy, F.bc, i, cells, F.ny);
+        v.r = F.r[i];
+        v.d = F.dinv[i];
+        v.c = corrected(i, x / 2, y / 2);
+        v.xl = corrected(v.o.ixl, xl, y / 2);
+        v.xu = corrected(v.o.ixu, xu, y / 2);
+        v.yl = corrected(v.o.iyl, x / 2, yl);
+        v.yu = corrected(v.o.iyu, x / 2, yu);
+        return v;
+      },
+      [&](uint32_t i, const Cell& v) {
+        const float z =
+            v.c + kCycleOmega * v.d * (v.r - cell_apply(v.o, v.c, v.xl, v.xu, v.yl, v.yu));
+        F.e[i] = z;
+        rz += static_cast<double>(z) * static_cast<double>(v.r);
+      });
+}
+
+// The cycle from level `from` down to the coarsest level's dense inverse and
+// back, by the whole workgroup: from level 0 it is z = M r and returns r.z
+// (this thread's share of it).
+template <int NT>
+__device__ double batch_cycle(const BatchData& D, const BatchLevels& V, size_t site,
+                              uint32_t from) {
+  const uint32_t K = V.count - 1;
+  const float* x0 = D.q + site;
+  for (uint32_t l = from; l < K; ++l) {
+    const LevelRef F = level_ref(D, V, l, site), C = level_ref(D, V, l + 1, site);
+    cycle_down<NT>(F, C, l == 0 ? x0 : nullptr, 0, C.nx * C.ny);
     __syncthreads();
   }
   double rz = 0.0;
@@ -313,28 +413,13 @@ __device__ double batch_cycle(const BatchData& D, const BatchLevels& V, size_t s
     }
     __syncthreads();
   }
-  for (int l = static_cast<int>(K) - 1; l >= 0; --l) {
-    const LevelRef F = level_ref(D, V, static_cast<uint32_t>(l), site);
-    const LevelRef C = level_ref(D, V, static_cast<uint32_t>(l) + 1, site);
-    auto corrected = [&](uint32_t gx, uint32_t gy) {
-      const size_t j = static_cast<size_t>(gx) * F.ny + gy;
-      return kCycleOmega * F.dinv[j] * F.r[j] +
-             kCycleCorrection * C.e[static_cast<size_t>(gx / 2) * C.ny + gy / 2];
-    };
-    const size_t cells = static_cast<size_t>(F.nx) * F.ny;
-    for (size_t i = threadIdx.x; i < cells; i += NT) {
-      const uint32_t fx = static_cast<uint32_t>(i / F.ny), fy = static_cast<uint32_t>(i % F.ny);
-      const float ri = F.r[i];
-      const float xc = corrected(fx, fy);
-      const float z = xc + kCycleOmega * F.dinv[i] * (ri - level_ax(F, i, fx, fy, xc, corrected));
-      F.e[i] = z;
-      if (l == 0) rz += static_cast<double>(z) * static_cast<double>(ri);
-    }
+  for (uint32_t l = K; l-- > from;) {
+    const LevelRef F = level_ref(D, V, l, site), C = level_ref(D, V, l + 1, site);
+    rz = 0.0;
+    cycle_up<NT>(F, C, l == 0 ? x0 : nullptr, 0, F.nx * F.ny, rz);
     __syncthreads();
   }
-  double out[1] = {rz};
-  block_sums<NT, 1>(out, lds);
-  return out[0];
+  return rz;
 }
 
 // What the setup writes of an instance.
@@ -464,122 +549,410 @@ __global__ __launch_bounds__(NT) void k_batch_setup(const BatchDesc* __restrict_
   }
 }
 
-// The pressure solve: one workgroup per instance (order[b], largest first),
-// FP64 refinement around FP32 corrections by conjugate gradient with the
-// instance's multilevel cycle, then every face velocity of the instance.
-template <int NT, int TY>
+// The pressure solve's passes over a range of an instance's sites, and what
+// decides between them. A solve is FP64 refinement around FP32 corrections by
+// conjugate gradient with the instance's multilevel cycle.
+constexpr uint32_t kRefinements = 16;
+constexpr double kInner = 1.0e-4;  // relative tolerance of each FP32 correction
+
+// An instance's vectors.
+struct FlowRef {
+  const float *cxl, *cyl, *bc, *rhs, *wx, *wy, *dinv;
+  double* x64;
+  float *x, *r, *q, *z;
+  float inlet;
+  uint32_t nx, ny, sites;
+  double isx, isy;
+};
+
+__device__ inline FlowRef flow_ref(const BatchData& D, const BatchDesc& I) {
+  const size_t o = I.site;
+  // The finest level's couplings (over the spacing squared), boundary term and
+  // inverse diagonal are the operator's own.
+  return FlowRef{D.cxl + o,  D.cyl + o, D.bc + o, D.rhs + o, D.lwx + o,
+                 D.lwy + o,  D.ldinv + o, D.x64 + o, D.x + o, D.r + o,
+                 D.q + o,    D.z + o,   I.inlet,  I.nx,      I.ny,
+                 I.nx * I.ny, 1.0 / (static_cast<double>(I.dx) * I.dx),
+                 1.0 / (static_cast<double>(I.dy) * I.dy)};
+}
+
+// FP64 true residual; its FP32 copy starts the correction x = 0, with the
+// cycle's first sweep beside it. s[0], s[1]: r.r (FP64) and b.b.
+template <int NT>
+__device__ inline void flow_residual(const FlowRef& A, uint32_t lo, uint32_t hi, double (&s)[2]) {
+  struct Cell {
+    double res, b;
+    float d;
+  };
+  sweep_cells<NT, 2>(
+      lo, hi,
+      [&](uint32_t i) {
+        const uint32_t x = i / A.ny, y = i - x * A.ny;
+        return Cell{residual_f64(A.x64, A.cxl, A.cyl, A.bc, A.rhs, A.inlet, x, y, A.nx, A.ny, i,
+                                 A.isx, A.isy),
+                    static_cast<double>(A.inlet) * static_cast<double>(A.rhs[i]), A.dinv[i]};
+      },
+      [&](uint32_t i, const Cell& v) {
+        const float ri = static_cast<float>(v.res);
+        A.r[i] = ri;
+        A.q[i] = kCycleOmega * v.d * ri;
+        A.x[i] = 0.0f;
+        s[0] += v.res * v.res;
+        s[1] += v.b * v.b;
+      });
+}
+
+// p = z + beta p (beta = 0 and no old p at the first), q = A p; p.q joins pq.
+// Neighbours' new directions are formed where they are read, so the old and
+// the new direction are two vectors.
+template <int NT, int U, bool kFirst>
+__device__ inline void flow_direction(const FlowRef& A, const float* p, float* pn, float beta,
+                                      uint32_t lo, uint32_t hi, double& pq) {
+  struct Cell {
+    CellOp o;
+    float c, xl, xu, yl, yu;
+  };
+  auto at = [&](uint32_t j) { return kFirst ? A.z[j] : A.z[j] + beta * p[j]; };
+  sweep_cells<NT, U>(
+      lo, hi,
+      [&](uint32_t i) {
+        Cell v;
+        v.o = cell_op(A.wx, A.wy, A.bc, i, A.sites, A.ny);
+        v.c = at(i);
+        v.xl = at(v.o.ixl);
+        v.xu = at(v.o.ixu);
+        v.yl = at(v.o.iyl);
+        v.yu = at(v.o.iyu);
+        return v;
+      },
+      [&](uint32_t i, const Cell& v) {
+        const float qi = cell_apply(v.o, v.c, v.xl, v.xu, v.yl, v.yu);
+        pn[i] = v.c;
+        A.q[i] = qi;
+        pq += static_cast<double>(v.c) * static_cast<double>(qi);
+      });
+}
+
+// x += alpha p, r -= alpha q, the cycle's first sweep; r.r joins rr.
+template <int NT>
+__device__ inline void flow_update(const FlowRef& A, const float* p, float alpha, uint32_t lo,
+                                   uint32_t hi, double& rr) {
+  struct Cell {
+    float x, p, r, q, d;
+  };
+  sweep_cells<NT, 4>(
+      lo, hi, [&](uint32_t i) { return Cell{A.x[i], p[i], A.r[i], A.q[i], A.dinv[i]}; },
+      [&](uint32_t i, const Cell& v) {
+        A.x[i] = v.x + alpha * v.p;
+        const float ri = v.r - alpha * v.q;
+        A.r[i] = ri;
+        A.q[i] = kCycleOmega * v.d * ri;
+        rr += static_cast<double>(ri) * static_cast<double>(ri);
+      });
+}
+
+template <int NT>
+__device__ inline void flow_correct(const FlowRef& A, uint32_t lo, uint32_t hi) {
+  struct Cell {
+    double x;
+    float e;
+  };
+  sweep_cells<NT, 4>(
+      lo, hi, [&](uint32_t i) { return Cell{A.x64[i], A.x[i]}; },
+      [&](uint32_t i, const Cell& v) { A.x64[i] = v.x + static_cast<double>(v.e); });
+}
+
+// The face velocities of the sites [lo, hi): their lower faces, and the last
+// row's and column's upper ones.
+template <int NT>
+__device__ inline void flow_faces(const BatchData& D, const BatchDesc& I, uint32_t lo,
+                                  uint32_t hi) {
+  const size_t o = I.site;
+  const double* x64 = D.x64 + o;
+  const float* cond = D.cond + o;
+  const uint8_t* solid = D.solid + o;
+  float* xf = D.xf + I.xface;
+  float* yf = D.yf + I.yface;
+  for (uint32_t i = lo + threadIdx.x; i < hi; i += NT) {
+    const uint32_t x = i / I.ny, y = i - x * I.ny;
+    xf[i] = face_x(I, x64, cond, solid, x, y);
+    if (x + 1 == I.nx) xf[i + I.ny] = face_x(I, x64, cond, solid, x + 1, y);
+    yf[i + x] = face_y(I, x64, cond, solid, x, y);
+    if (y + 1 == I.ny) yf[i + x + 1] = face_y(I, x64, cond, solid, x, y + 1);
+  }
+}
+
+__device__ inline bool flow_breaks(double product) {
+  return !(product > 0.0) || !isfinite(product);
+}
+
+__device__ inline double flow_threshold(const BatchParams& P, double bb) {
+  const double bound = static_cast<double>(P.tolerance) * sqrt(bb);
+  return bound * bound;
+}
+
+__device__ inline void flow_result(const BatchData& D, uint32_t inst, uint32_t it, double rr64,
+                                   double bb, bool failed, bool short_of) {
+  D.iterations[inst] = it;
+  D.residual[inst] = bb > 0.0 ? static_cast<float>(sqrt(rr64 / bb)) : 0.0f;
+  D.bnorm2[inst] = bb;
+  if (failed) D.flags[inst] |= 1u;
+  if (short_of && !failed) D.flags[inst] |= 2u;
+}
+
+// One workgroup per instance (order[b]) solves it alone: one launch, barriers
+// in place of launches. A compute unit moves about 20 GB/s of a 512x256
+// instance (its 6 MB are past its L2's share), so this is the form of small
+// instances, and of batches that keep every unit busy (solve_alone).
+template <int NT>
 __global__ __launch_bounds__(NT) void k_batch_flow(BatchData D, BatchParams P) {
   __shared__ double s_red[NT / kWave];
-  constexpr int RX = NT / TY;
   const uint32_t inst = D.order[blockIdx.x];
   const BatchDesc I = D.desc[inst];
-  const uint32_t nx = I.nx, ny = I.ny;
-  const size_t o = I.site;
-  const uint32_t tx = threadIdx.x / TY, ty = threadIdx.x % TY;
-  const uint8_t* solid = D.solid + o;
-  const float* cond = D.cond + o;
-  const float* cxl = D.cxl + o;
-  const float* cyl = D.cyl + o;
-  const float* bc = D.bc + o;
-  const float* rhs = D.rhs + o;
-  double* x64 = D.x64 + o;
-  float* xv = D.x + o;
-  float* r = D.r + o;
-  float* p = D.p + o;
-  float* q = D.q + o;
-  const float isx = 1.0f / (I.dx * I.dx), isy = 1.0f / (I.dy * I.dy);
-  auto sweep = [&](auto&& f) {
-    for (uint32_t x0 = 0; x0 < nx; x0 += RX) {
-      const uint32_t x = x0 + tx;
-      if (x >= nx) continue;
-      for (uint32_t y = ty; y < ny; y += TY) f(x, y, static_cast<size_t>(x) * ny + y);
-    }
-  };
-  constexpr uint32_t kRefinements = 16;
-  constexpr double kInner = 1.0e-4;  // relative tolerance of each FP32 correction
   const BatchLevels& V = D.levels[inst];
-  float* z = D.z + o;
-  uint32_t it = 0, failed = 0;
+  const FlowRef A = flow_ref(D, I);
+  const uint32_t n = A.sites;
+  uint32_t it = 0;
+  bool failed = false;
   double rr64 = 0.0, bb = 0.0, threshold = 0.0;
-  for (uint32_t ref = 0; ref <= kRefinements; ++ref) {
-    // FP64 true residual; its FP32 copy starts the correction e = 0.
-    double s2[2] = {0.0, 0.0};  // r.r (FP64), b.b
-    sweep([&](uint32_t x, uint32_t y, size_t i) {
-      const double res = residual_f64(x64, cxl, cyl, bc, rhs, I.inlet, x, y, nx, ny, i, isx, isy);
-      const double b = static_cast<double>(I.inlet) * static_cast<double>(rhs[i]);
-      r[i] = static_cast<float>(res);
-      xv[i] = 0.0f;
-      s2[0] += res * res;
-      s2[1] += b * b;
-    });
+  for (uint32_t ref = 0;; ++ref) {
+    double s2[2] = {0.0, 0.0};
+    flow_residual<NT>(A, 0, n, s2);
     block_sums<NT, 2>(s2, s_red);
     rr64 = s2[0];
     bb = s2[1];
-    const double bound = static_cast<double>(P.tolerance) * sqrt(bb);
-    threshold = bound * bound;
+    threshold = flow_threshold(P, bb);
     if (rr64 <= threshold || ref == kRefinements || it >= P.max_iterations) break;
-    double rz = batch_cycle<NT>(D, V, o, s_red);
-    if (!(rz > 0.0) || !isfinite(rz)) {
-      failed = 1;
-      break;
-    }
-    sweep([&](uint32_t x, uint32_t y, size_t i) { p[i] = z[i]; });
-    __syncthreads();
-    double rr = rr64;
+    double rr = rr64, rz_old = 0.0;
     const double inner = kInner * kInner * rr64;
-    while (rr > inner && it < P.max_iterations) {
-      double s1[1] = {0.0};
-      sweep([&](uint32_t x, uint32_t y, size_t i) {
-        const float qi = apply_f32(p, cxl, cyl, bc, x, y, nx, ny, i, isx, isy);
-        q[i] = qi;
-        s1[0] += static_cast<double>(p[i]) * static_cast<double>(qi);
-      });
-      block_sums<NT, 1>(s1, s_red);
-      if (!(s1[0] > 0.0) || !isfinite(s1[0])) {
-        failed = 1;
-        break;
+    for (uint32_t k = 0; rr > inner && it < P.max_iterations; ++k, ++it) {
+      float* p = (k & 1u) != 0 ? D.p2 + I.site : D.p + I.site;
+      float* pn = (k & 1u) != 0 ? D.p + I.site : D.p2 + I.site;
+      double rz[1] = {batch_cycle<NT>(D, V, I.site, 0)};
+      block_sums<NT, 1>(rz, s_red);
+      failed = flow_breaks(rz[0]);
+      if (failed) break;
+      double pq[1] = {0.0};
+      if (k == 0) {
+        flow_direction<NT, 2, true>(A, p, pn, 0.0f, 0, n, pq[0]);
+      } else {
+        flow_direction<NT, 2, false>(A, p, pn, static_cast<float>(rz[0] / rz_old), 0, n, pq[0]);
       }
-      const float alpha = static_cast<float>(rz / s1[0]);
-      double s3[1] = {0.0};
-      sweep([&](uint32_t x, uint32_t y, size_t i) {
-        xv[i] = xv[i] + alpha * p[i];
-        const float ri = r[i] - alpha * q[i];
-        r[i] = ri;
-        s3[0] += static_cast<double>(ri) * static_cast<double>(ri);
-      });
-      block_sums<NT, 1>(s3, s_red);
-      rr = s3[0];
-      ++it;
-      if (rr <= inner) break;
-      const double rz_next = batch_cycle<NT>(D, V, o, s_red);
-      if (!(rz_next > 0.0) || !isfinite(rz_next)) {
-        failed = 1;
-        break;
-      }
-      const float beta = static_cast<float>(rz_next / rz);
-      rz = rz_next;
-      sweep([&](uint32_t x, uint32_t y, size_t i) { p[i] = z[i] + beta * p[i]; });
-      __syncthreads();
+      block_sums<NT, 1>(pq, s_red);
+      failed = flow_breaks(pq[0]);
+      if (failed) break;
+      rz_old = rz[0];
+      double s[1] = {0.0};
+      flow_update<NT>(A, pn, static_cast<float>(rz[0] / pq[0]), 0, n, s[0]);
+      block_sums<NT, 1>(s, s_red);
+      rr = s[0];
     }
-    if (failed != 0) break;
-    sweep([&](uint32_t x, uint32_t y, size_t i) { x64[i] += static_cast<double>(xv[i]); });
+    if (failed) break;
+    flow_correct<NT>(A, 0, n);
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    D.iterations[inst] = it;
-    D.residual[inst] = bb > 0.0 ? static_cast<float>(sqrt(rr64 / bb)) : 0.0f;
-    D.bnorm2[inst] = bb;
-    if (failed != 0) D.flags[inst] |= 1u;
-    if (rr64 > threshold && failed == 0) D.flags[inst] |= 2u;
+  if (threadIdx.x == 0) flow_result(D, inst, it, rr64, bb, failed, rr64 > threshold);
+  flow_faces<NT>(D, I, 0, n);
+}
+
+// The same solve over the whole chip: every instance's iteration advances
+// together, each pass one launch over tiles of all instances,
+//   down (finest levels) - tail (one workgroup per instance: its levels of at
+//   most kTailCells, and the decision of what comes next) - up - direction -
+//   update,
+// and an instance whose correction is done adds it and takes its FP64 residual
+// in the up and direction launches of the same body. Each tile leaves its share
+// of a product; whoever needs the product adds the instance's shares in tile
+// order. Nothing waits inside a launch, and the host looks at the number of
+// finished instances a few bodies behind.
+enum FlowPhase : uint32_t { kFlowCorrect, kFlowIterate, kFlowDone };
+
+struct FlowState {
+  double rz, rr64, bb, inner;
+  uint32_t phase, first, it, ref;
+};
+
+// A range of an instance's cells of one level, and the instance's tiles of the
+// finest level.
+struct FlowTile {
+  uint32_t inst, lo, hi, slot;
+};
+struct FlowSpan {
+  uint32_t first, count, tail, pad;  // tail: the level the tail starts at
+};
+
+struct FlowWork {
+  BatchData D;
+  BatchParams P;
+  const FlowSpan* span;
+  FlowState* state;
+  double* share;  // [3][tiles]: r.z | p.q, FP64 r.r | r.r, b.b
+  uint32_t tiles;
+  uint32_t* done;
+};
+
+constexpr int kFlowTileThreads = 256;
+constexpr uint32_t kFlowTile = 1024;  // sites of a tile (512: 20.6 ms, 2048: 18.6)
+
+// The instance's shares of product k in tile order, the same in every wave.
+__device__ inline double flow_sum(const FlowWork& W, const FlowSpan& s, uint32_t k) {
+  const double* at = W.share + static_cast<size_t>(k) * W.tiles + s.first;
+  double v = 0.0;
+  for (uint32_t j = threadIdx.x % kWave; j < s.count; j += kWave) v += at[j];
+  return wave_sum(v);
+}
+
+__device__ inline void flow_share(const FlowWork& W, uint32_t slot, uint32_t k, double v,
+                                  double* lds) {
+  const double t = block_sum<kFlowTileThreads>(v, lds);
+  if (threadIdx.x == 0) W.share[static_cast<size_t>(k) * W.tiles + slot] = t;
+}
+
+// What follows the last body: the state after it, from its shares.
+__device__ inline FlowState flow_next(const FlowWork& W, const FlowSpan& s, FlowState S,
+                                      bool& failed) {
+  failed = false;
+  S.first = 0;
+  if (S.phase == kFlowIterate) {
+    const double rz = flow_sum(W, s, 0), pq = flow_sum(W, s, 1), rr = flow_sum(W, s, 2);
+    failed = flow_breaks(rz) || flow_breaks(pq);
+    S.rz = rz;
+    if (failed) {
+      S.phase = kFlowDone;
+    } else {
+      ++S.it;
+      if (!(rr > S.inner) || S.it >= W.P.max_iterations) S.phase = kFlowCorrect;
+    }
+  } else if (S.phase == kFlowCorrect) {
+    S.rr64 = flow_sum(W, s, 1);
+    S.bb = flow_sum(W, s, 2);
+    if (S.rr64 <= flow_threshold(W.P, S.bb) || S.ref == kRefinements ||
+        S.it >= W.P.max_iterations) {
+      S.phase = kFlowDone;
+    } else {
+      S.phase = kFlowIterate;
+      S.first = 1;
+      S.inner = kInner * kInner * S.rr64;
+      ++S.ref;
+    }
   }
-  // Face velocities.
-  float* xf = D.xf + I.xface;
-  float* yf = D.yf + I.yface;
-  for (size_t f = threadIdx.x; f < static_cast<size_t>(nx + 1) * ny; f += NT)
-    xf[f] = face_x(I, x64, cond, solid, static_cast<uint32_t>(f / ny), static_cast<uint32_t>(f % ny));
-  for (size_t f = threadIdx.x; f < static_cast<size_t>(nx) * (ny + 1); f += NT)
-    yf[f] = face_y(I, x64, cond, solid, static_cast<uint32_t>(f / (ny + 1)),
-                   static_cast<uint32_t>(f % (ny + 1)));
+  return S;
+}
+
+__global__ __launch_bounds__(kFlowTileThreads) void k_flow_down(FlowWork W, const FlowTile* tiles,
+                                                                uint32_t level) {
+  const FlowTile t = tiles[blockIdx.x];
+  const FlowState S = W.state[t.inst];
+  if (S.phase == kFlowDone) return;
+  bool failed;
+  if (flow_next(W, W.span[t.inst], S, failed).phase != kFlowIterate) return;
+  const BatchLevels& V = W.D.levels[t.inst];
+  const size_t site = W.D.desc[t.inst].site;
+  cycle_down<kFlowTileThreads>(level_ref(W.D, V, level, site), level_ref(W.D, V, level + 1, site),
+                               level == 0 ? W.D.q + site : nullptr, t.lo, t.hi);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_flow_tail(FlowWork W) {
+  const uint32_t inst = W.D.order[blockIdx.x];
+  const FlowState S = W.state[inst];
+  if (S.phase == kFlowDone) return;
+  const FlowSpan s = W.span[inst];
+  bool failed;
+  const FlowState next = flow_next(W, s, S, failed);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    W.state[inst] = next;
+    if (next.phase == kFlowDone) {
+      flow_result(W.D, inst, next.it, next.rr64, next.bb, failed,
+                  next.rr64 > flow_threshold(W.P, next.bb));
+      atomicAdd(W.done, 1u);
+    }
+  }
+  if (next.phase == kFlowIterate)
+    batch_cycle<NT>(W.D, W.D.levels[inst], W.D.desc[inst].site, s.tail);
+}
+
+__global__ __launch_bounds__(kFlowTileThreads) void k_flow_up(FlowWork W, const FlowTile* tiles,
+                                                              uint32_t level) {
+  __shared__ double s_red[kFlowTileThreads / kWave];
+  const FlowTile t = tiles[blockIdx.x];
+  const FlowState S = W.state[t.inst];
+  if (S.phase == kFlowDone) return;
+  const BatchDesc I = W.D.desc[t.inst];
+  if (S.phase == kFlowCorrect) {
+    if (level == 0) flow_correct<kFlowTileThreads>(flow_ref(W.D, I), t.lo, t.hi);
+    return;
+  }
+  const BatchLevels& V = W.D.levels[t.inst];
+  double rz = 0.0;
+  if (V.count > 1) {
+    cycle_up<kFlowTileThreads>(level_ref(W.D, V, level, I.site),
+                               level_ref(W.D, V, level + 1, I.site),
+                               level == 0 ? W.D.q + I.site : nullptr, t.lo, t.hi, rz);
+  } else {  // one level: the tail's dense inverse left z
+    const FlowRef A = flow_ref(W.D, I);
+    for (uint32_t i = t.lo + threadIdx.x; i < t.hi; i += kFlowTileThreads)
+      rz += static_cast<double>(A.z[i]) * static_cast<double>(A.r[i]);
+  }
+  if (level == 0) flow_share(W, t.slot, 0, rz, s_red);
+}
+
+__global__ __launch_bounds__(kFlowTileThreads) void k_flow_direction(FlowWork W,
+                                                                     const FlowTile* tiles) {
+  __shared__ double s_red[kFlowTileThreads / kWave];
+  const FlowTile t = tiles[blockIdx.x];
+  const FlowState S = W.state[t.inst];
+  if (S.phase == kFlowDone) return;
+  const BatchDesc I = W.D.desc[t.inst];
+  const FlowRef A = flow_ref(W.D, I);
+  if (S.phase == kFlowCorrect) {
+    double s[2] = {0.0, 0.0};
+    flow_residual<kFlowTileThreads>(A, t.lo, t.hi, s);
+    flow_share(W, t.slot, 1, s[0], s_red);
+    flow_share(W, t.slot, 2, s[1], s_red);
+    return;
+  }
+  const double rz = flow_sum(W, W.span[t.inst], 0);
+  if (flow_breaks(rz)) return;
+  float* p = ((S.it & 1u) != 0 ? W.D.p2 : W.D.p) + I.site;
+  float* pn = ((S.it & 1u) != 0 ? W.D.p : W.D.p2) + I.site;
+  double pq = 0.0;
+  if (S.first != 0) {
+    flow_direction<kFlowTileThreads, 4, true>(A, p, pn, 0.0f, t.lo, t.hi, pq);
+  } else {
+    flow_direction<kFlowTileThreads, 4, false>(A, p, pn, static_cast<float>(rz / S.rz), t.lo,
+                                               t.hi, pq);
+  }
+  flow_share(W, t.slot, 1, pq, s_red);
+}
+
+__global__ __launch_bounds__(kFlowTileThreads) void k_flow_update(FlowWork W,
+                                                                  const FlowTile* tiles) {
+  __shared__ double s_red[kFlowTileThreads / kWave];
+  const FlowTile t = tiles[blockIdx.x];
+  const FlowState S = W.state[t.inst];
+  if (S.phase != kFlowIterate) return;
+  const FlowSpan span = W.span[t.inst];
+  const double rz = flow_sum(W, span, 0), pq = flow_sum(W, span, 1);
+  if (flow_breaks(rz) || flow_breaks(pq)) return;
+  const BatchDesc I = W.D.desc[t.inst];
+  const float* pn = ((S.it & 1u) != 0 ? W.D.p : W.D.p2) + I.site;
+  double rr = 0.0;
+  flow_update<kFlowTileThreads>(flow_ref(W.D, I), pn, static_cast<float>(rz / pq), t.lo, t.hi, rr);
+  flow_share(W, t.slot, 2, rr, s_red);
+}
+
+__global__ __launch_bounds__(kFlowTileThreads) void k_flow_faces(BatchData D,
+                                                                 const FlowTile* tiles) {
+  const FlowTile t = tiles[blockIdx.x];
+  flow_faces<kFlowTileThreads>(D, D.desc[t.inst], t.lo, t.hi);
+}
+
+__global__ void k_flow_begin(FlowState* state, uint32_t count, uint32_t* done) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < count) state[k] = FlowState{0.0, 0.0, 0.0, 0.0, kFlowCorrect, 0, 0, 0};
+  if (k == 0) *done = 0;
 }
 
 // One step for work item blockIdx.x (rows [x0, x1) of an instance): the FP64
@@ -894,7 +1267,6 @@ __global__ __launch_bounds__(kMarchThreads) void k_batch_march(
   }
 }
 
-using FlowKernel = void (*)(BatchData, BatchParams);
 using StepKernel = void (*)(BatchData, BatchParams, const BatchItem*, double*, uint32_t, float,
                             uint32_t, uint32_t);
 
@@ -925,8 +1297,22 @@ int class_of(uint32_t ny) {
   return kClasses - 1;
 }
 constexpr int kSetupThreads = 1024;
-constexpr FlowKernel kFlowKernel = k_batch_flow<1024, 128>;
-constexpr int kFlowThreads = 1024;
+constexpr int kFlowThreads = 1024;  // of k_batch_flow and k_flow_tail
+// Levels of at most this many cells are the tail's: a 256-instance sweep solves
+// in 17.6 ms with 2048, 17.9 with 4096, 18.0 with 8192.
+constexpr uint64_t kTailCells = 2048;
+constexpr uint32_t kFlowBodies = 4;  // bodies between two looks at the finished instances
+
+// Whether a batch is solved one workgroup per instance. An iteration then takes
+// what the largest instance takes one compute unit; over the whole chip it
+// takes some 45 us of launches and dependent reads, and the sites of all. In us
+// per iteration, alone and together: 1 x 64x64 31 and 46, 1 x 96x80 52 and 54,
+// 1 x 128x96 67 and 58, 64 x 128x96 78 and 81, 256 x 128x96 92 and 144,
+// 64 x 256x128 187 and 121, 256 x 256x128 291 and 328, 64 x 512x256 903 and 344.
+constexpr uint64_t kAloneSites = 8192;
+bool solve_alone(uint64_t sites, uint64_t largest) {
+  return largest <= kAloneSites || 256 * sites >= largest * largest;
+}
 
 }  // namespace
 
@@ -944,12 +1330,21 @@ struct BatchDevice {
   DeviceBuffer<BatchDesc> d_desc;
   DeviceBuffer<uint32_t> d_order, iterations, flags;
   DeviceBuffer<uint8_t> solid;
-  DeviceBuffer<float> mobility, cond, cxl, cyl, bc, diag, rhs, phi, x, r, p, q, z, xf, yf, la, lb,
+  DeviceBuffer<float> mobility, cond, cxl, cyl, bc, diag, rhs, phi, x, r, p, p2, q, z, xf, yf, la, lb,
       residual, saved;
   std::vector<BatchLevels> levels;  // per instance
   DeviceBuffer<BatchLevels> d_levels;
   DeviceBuffer<float> lwx, lwy, lbc, ldinv, lr, le, cinv;
   DeviceBuffer<double> x64, bnorm2, partials;
+  // The solve over the whole chip: tiles per level (down: of the level below),
+  // shares of the products, the host's view of the finished instances.
+  std::vector<std::unique_ptr<DeviceBuffer<FlowTile>>> flow_down, flow_up;
+  DeviceBuffer<FlowSpan> flow_span;
+  DeviceBuffer<FlowState> flow_state;
+  DeviceBuffer<double> flow_share;
+  DeviceBuffer<uint32_t> flow_done;
+  uint32_t* host_done = nullptr;  // pinned, two by turns
+  hipEvent_t looked[2] = {};
   BatchParams params{};
   bool has_phi = false;
   bool solved = false;
@@ -962,6 +1357,10 @@ struct BatchDevice {
   BatchData graph_data{};
   const double* graph_partials = nullptr;
   ~BatchDevice() {
+    for (hipEvent_t e : looked) {
+      if (e != nullptr) static_cast<void>(hipEventDestroy(e));
+    }
+    if (host_done != nullptr) static_cast<void>(hipHostFree(host_done));
     if (graph != nullptr) static_cast<void>(hipGraphExecDestroy(graph));
   }
 };
@@ -983,6 +1382,7 @@ BatchData batch_data(BatchDevice& B) {
   D.x = B.x.data();
   D.r = B.r.data();
   D.p = B.p.data();
+  D.p2 = B.p2.data();
   D.q = B.q.data();
   D.xf = B.xf.data();
   D.yf = B.yf.data();
@@ -1116,6 +1516,105 @@ void build_systems(Context& ctx, BatchDevice& B) {
   check(hipGetLastError(), "launch k_batch_setup");
 }
 
+// Tiles of the solve over the whole chip; none for a batch of small instances.
+void plan_flow(Context& ctx, BatchDevice& B) {
+  B.flow_down.clear();
+  B.flow_up.clear();
+  const BatchDesc& largest = B.desc[B.order[0]];
+  if (solve_alone(B.sites, static_cast<uint64_t>(largest.nx) * largest.ny)) return;
+  std::vector<FlowSpan> span(B.count);
+  std::vector<std::vector<FlowTile>> down, up;
+  auto cut = [](std::vector<FlowTile>& to, uint32_t inst, uint32_t cells, uint32_t tile) {
+    for (uint32_t lo = 0; lo < cells; lo += tile)
+      to.push_back(FlowTile{inst, lo, std::min(cells, lo + tile), static_cast<uint32_t>(to.size())});
+  };
+  for (uint32_t k : B.order) {
+    const BatchLevels& L = B.levels[k];
+    uint32_t tail = 0;
+    do {
+      if (up.size() <= tail) {
+        up.emplace_back();
+        down.emplace_back();
+      }
+      const uint32_t first = static_cast<uint32_t>(up[tail].size());
+      cut(up[tail], k, L.nx[tail] * L.ny[tail], kFlowTile);
+      if (tail == 0) span[k] = FlowSpan{first, static_cast<uint32_t>(up[0].size()) - first, 0, 0};
+      if (L.count == 1) break;
+      cut(down[tail], k, L.nx[tail + 1] * L.ny[tail + 1], kFlowTile / 4);
+      ++tail;
+    } while (tail + 1 < L.count && static_cast<uint64_t>(L.nx[tail]) * L.ny[tail] > kTailCells);
+    span[k].tail = tail;
+  }
+  auto upload = [&](const std::vector<FlowTile>& tiles) {
+    auto buf = std::make_unique<DeviceBuffer<FlowTile>>();
+    buf->reserve(tiles.size());
+    check(hipMemcpyAsync(buf->data(), tiles.data(), tiles.size() * sizeof(FlowTile),
+                         hipMemcpyHostToDevice, ctx.stream),
+          "upload flow tiles");
+    return buf;
+  };
+  for (const auto& t : up) B.flow_up.push_back(upload(t));
+  for (const auto& t : down) B.flow_down.push_back(upload(t));
+  B.flow_span.reserve(B.count);
+  check(hipMemcpyAsync(B.flow_span.data(), span.data(), B.count * sizeof(FlowSpan),
+                       hipMemcpyHostToDevice, ctx.stream),
+        "upload flow spans");
+  B.flow_state.reserve(B.count);
+  B.flow_share.reserve(3 * up[0].size());
+  B.flow_done.reserve(1);
+  if (B.host_done == nullptr) {
+    void* ptr = nullptr;
+    check(hipHostMalloc(&ptr, 2 * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
+    B.host_done = static_cast<uint32_t*>(ptr);
+    for (hipEvent_t& e : B.looked)
+      check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+  }
+  // The host vectors end here.
+  check(hipStreamSynchronize(ctx.stream), "flow tiles");
+}
+
+void solve_together(Context& ctx, BatchDevice& B) {
+  const uint32_t levels = static_cast<uint32_t>(B.flow_up.size());
+  const uint32_t tiles = static_cast<uint32_t>(B.flow_up[0]->size());
+  const FlowWork W{batch_data(B),        B.params, B.flow_span.data(), B.flow_state.data(),
+                   B.flow_share.data(), tiles,    B.flow_done.data()};
+  k_flow_begin<<<(B.count + 255) / 256, 256, 0, ctx.stream>>>(W.state, B.count, W.done);
+  k_flow_direction<<<tiles, kFlowTileThreads, 0, ctx.stream>>>(W, B.flow_up[0]->data());
+  auto body = [&]() {
+    for (uint32_t l = 0; l < levels; ++l) {
+      const uint32_t n = static_cast<uint32_t>(B.flow_down[l]->size());
+      if (n > 0)
+        k_flow_down<<<n, kFlowTileThreads, 0, ctx.stream>>>(W, B.flow_down[l]->data(), l);
+    }
+    k_flow_tail<kFlowThreads><<<B.count, kFlowThreads, 0, ctx.stream>>>(W);
+    for (uint32_t l = levels; l-- > 0;) {
+      k_flow_up<<<static_cast<uint32_t>(B.flow_up[l]->size()), kFlowTileThreads, 0, ctx.stream>>>(
+          W, B.flow_up[l]->data(), l);
+    }
+    k_flow_direction<<<tiles, kFlowTileThreads, 0, ctx.stream>>>(W, B.flow_up[0]->data());
+    k_flow_update<<<tiles, kFlowTileThreads, 0, ctx.stream>>>(W, B.flow_up[0]->data());
+    check(hipGetLastError(), "launch batch flow");
+  };
+  // An instance takes one body per iteration and per refinement, and one to
+  // find that it is done.
+  const uint64_t most = static_cast<uint64_t>(B.params.max_iterations) + kRefinements + 2;
+  const uint64_t looks = (most + kFlowBodies - 1) / kFlowBodies;
+  for (uint64_t k = 0; k <= looks; ++k) {
+    if (k < looks) {
+      for (uint32_t j = 0; j < kFlowBodies; ++j) body();
+      check(hipMemcpyAsync(B.host_done + (k & 1), B.flow_done.data(), sizeof(uint32_t),
+                           hipMemcpyDeviceToHost, ctx.stream),
+            "look at finished instances");
+      check(hipEventRecord(B.looked[k & 1], ctx.stream), "event");
+    }
+    if (k == 0) continue;
+    check(hipEventSynchronize(B.looked[(k - 1) & 1]), "batch flow");
+    if (B.host_done[(k - 1) & 1] == B.count) break;
+  }
+  k_flow_faces<<<tiles, kFlowTileThreads, 0, ctx.stream>>>(W.D, B.flow_up[0]->data());
+  check(hipGetLastError(), "launch k_flow_faces");
+}
+
 }  // namespace
 
 BatchDevice& batch_of(Context& ctx) {
@@ -1218,7 +1717,7 @@ void batch_upload(Context& ctx, uint32_t count, const msim_batch_instance* inst,
   const size_t n = site;
   B.solid.reserve(n);
   for (auto* b : {&B.mobility, &B.cond, &B.cxl, &B.cyl, &B.bc, &B.diag, &B.rhs, &B.phi, &B.x,
-                  &B.r, &B.p, &B.q, &B.z, &B.la, &B.lb, &B.saved})
+                  &B.r, &B.p, &B.p2, &B.q, &B.z, &B.la, &B.lb, &B.saved})
     b->reserve(n);
   B.x64.reserve(n);
   B.xf.reserve(xface);
@@ -1271,6 +1770,7 @@ void batch_upload(Context& ctx, uint32_t count, const msim_batch_instance* inst,
     }
   }
   build_systems(ctx, B);
+  plan_flow(ctx, B);
   B.params.tolerance = params.relative_tolerance;
   B.params.max_iterations = params.max_iterations;
   B.params.vmax = params.monod_vmax;
@@ -1281,13 +1781,17 @@ void batch_upload(Context& ctx, uint32_t count, const msim_batch_instance* inst,
 }
 
 // Solves every instance's pressure from its current one and rebuilds its
-// velocities (one launch).
+// velocities.
 void batch_solve_flow(Context& ctx, uint32_t* iterations, float* residual, uint32_t* flags) {
   BatchDevice& B = batch_of(ctx);
   if (B.count == 0) throw Error(MSIM_INVALID_ARGUMENT, "no batch is uploaded");
-  hipLaunchKernelGGL(kFlowKernel, dim3(B.count), dim3(kFlowThreads), 0, ctx.stream,
-                     batch_data(B), B.params);
-  check(hipGetLastError(), "launch k_batch_flow");
+  if (B.flow_up.empty()) {
+    k_batch_flow<kFlowThreads>
+        <<<B.count, kFlowThreads, 0, ctx.stream>>>(batch_data(B), B.params);
+    check(hipGetLastError(), "launch k_batch_flow");
+  } else {
+    solve_together(ctx, B);
+  }
   B.solved = true;
   if (iterations != nullptr) {
     check(hipMemcpyAsync(iterations, B.iterations.data(), B.count * sizeof(uint32_t),

@@ -93,13 +93,17 @@ def odd_instance(nx, ny, pocket):
     [(3, 3), (8, 8), (2, 31)],            # one level: the dense inverse alone
     [(13, 5), (65, 3), (3, 65), (9, 8)],  # one coarsening, odd remainders
     [(33, 31), (129, 17), (64, 64), (37, 111)],
+    [(91, 91), (3, 3)],                          # over the whole chip: two tiled levels
+    [(701, 300), (5, 7), (300, 47)],             # four, beside a single-level instance
 ])
 @pytest.mark.parametrize("pocket", [False, True])
 def test_batch_system_at_odd_sizes(hip, oracle, sizes, pocket):
     """The device's setup and cycle at level edges: every instance converges to
     1e-10 of the oracle's own right-hand side and operator (FP64), in no more
-    iterations than a multilevel cycle needs (a wrong coarse operator or
-    inverse costs hundreds or fails)."""
+    iterations than a multilevel cycle needs: plain aggregation loses a fixed
+    factor per level, some 13 to 18 iterations of the ten digits asked for, so
+    30 per level (Jacobi alone takes several times the longer side; a wrong
+    coarse operator or inverse costs hundreds or fails)."""
     inst = [odd_instance(nx, ny, pocket and nx >= 24 and ny >= 17) for nx, ny in sizes]
     hip.batch_upload(inst, relative_tolerance=1e-10, max_iterations=4000)
     it, res, fl = hip.batch_solve_flow()
@@ -110,7 +114,10 @@ def test_batch_system_at_odd_sizes(hip, oracle, sizes, pocket):
         b = oracle.assemble(g, i.mobility, 0)["rhs"].astype(np.float64) * np.float64(np.float32(i.inlet_pressure))
         true = np.linalg.norm(b - oracle.apply(g, i.mobility, hip.batch_download(k)["pressure"])) / np.linalg.norm(b)
         assert true <= 1e-10
-        assert it[k] <= 120
+        levels, nx, ny = 1, i.nx, i.ny
+        while nx * ny > 64:
+            levels, nx, ny = levels + 1, (nx + 1) // 2, (ny + 1) // 2
+        assert it[k] <= 30 * levels
 
 
 def test_batch_step_is_the_single_grid_step(hip, oracle):
