@@ -304,7 +304,7 @@ struct AdrDevice {
   DeviceBuffer<double> implicit_sums;
   DeviceBuffer<ImplicitState> implicit_state;
   int current = 0;
-  DeviceBuffer<double> partials, ledger, mass;
+  DeviceBuffer<double> partials, ledger;
   DeviceBuffer<uint32_t> flags;              // [0]: error bits, [1]: first failed step
   DeviceBuffer<CgState> state;
   double seconds = 0.0;
