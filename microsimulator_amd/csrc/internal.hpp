@@ -132,9 +132,8 @@ constexpr uint32_t kFlagSources = 8;   // a coupled source rate not finite
 // level's residual and correction during a cycle.
 struct MgLevel {
   uint32_t nx = 0, ny = 0;
-  // xp: the iterate after pre-smoothing (read by the up pass); t: the
-  // single-workgroup kernel's intermediate sweep.
-  DeviceBuffer<float> wx, wy, bc, dinv, r, e, xp, t;
+  // xp: the iterate after pre-smoothing (read by the up pass).
+  DeviceBuffer<float> wx, wy, bc, dinv, r, e, xp;
   [[nodiscard]] std::size_t cells() const { return static_cast<std::size_t>(nx) * ny; }
 };
 

@@ -18,8 +18,7 @@
 // post-smoothing sweeps), each staging a 16 x 64 tile plus a two-site halo
 // in LDS. A second sweep on each side takes the iterations at 4096 x 2048
 // from 53 to about 33 for a quarter more work per cycle.
-// Levels of <= 4096 cells run in one single-workgroup kernel (measured at
-// 4096x2048: 16384 cost 130 us of coarse work per cycle, 4096 109 us).
+// Levels of <= 4096 cells run in one single-workgroup kernel (k_mg_tail).
 //
 // Outer solver: flexible CG (Notay's FCG(1): beta_k = -(z.q_{k-1}) /
 // (p_{k-1}.q_{k-1})) in FP32 with FP64 sums, inside the FP64 iterative
@@ -47,7 +46,15 @@ constexpr int kHY2 = kTY + 4;
 constexpr int kMgThreads = (kTX / 2) * (kTY / 2);  // one thread per 2x2 aggregate
 constexpr int kTailThreads = 1024;
 constexpr uint32_t kCoarseCells = 256;  // densely inverted
-constexpr uint32_t kTailCells = 4096;  // levels handled by the single-block kernel
+// The single-workgroup kernel takes the levels from the first of at most
+// kTailCells cells, kTailQuads aggregates per thread (a grid of one row has
+// more aggregates than a quarter of its cells) and kTailFloats of LDS. From
+// 8192 cells (two aggregates per thread) it took 27.6 us, 16.3 more, ten of
+// them to load 200 KB into one compute unit, for two launches of the tile
+// kernels saved (12 us).
+constexpr uint32_t kTailCells = 4096;
+constexpr int kTailQuads = 1;
+constexpr uint64_t kTailFloats = 38 * 1024;
 constexpr uint32_t kMaxLevels = 24;
 static_assert(4 * kCoarseCells <= kTailThreads, "the coarsest solve splits every row in parts");
 constexpr float kOmega = 0.8f;
@@ -256,77 +263,264 @@ struct TailLevel {
   const float* wy;
   const float* bc;
   const float* dinv;
-  float* r;
-  float* e;
-  float* xp;  // the pre-smoothed iterate, then the first post-smoothing sweep
-  float* t;   // the first pre-smoothing sweep, then the prolonged iterate
   uint32_t nx, ny;
+  uint32_t at;  // first float of the level's arrays in LDS
 };
 
 struct TailArgs {
   TailLevel lv[kMaxLevels];
   uint32_t count;      // levels from the first tail level to the coarsest
+  const float* r;      // the first level's residual and result
+  float* e;
   const float* cinv;   // dense inverse of the coarsest operator, transposed
   uint32_t n;          // its size
   UpDots dots;         // when the tail starts at level 0
 };
 
-// (A x)_i on a tail level at site i = fx ny + fy, with x_j = xv(j); the
-// terms in the order of the tile kernels.
-template <typename X>
-__device__ inline float tail_ax(const TailLevel& L, X xv, uint32_t i, uint32_t fx, uint32_t fy) {
-  const float xc = xv(i);
-  float ax = L.bc[i] * xc;
-  if (fx > 0) ax += L.wx[i] * (xc - xv(i - L.ny));
-  if (fx + 1 < L.nx) ax += L.wx[i + L.ny] * (xc - xv(i + L.ny));
-  if (fy > 0) ax += L.wy[i] * (xc - xv(i - 1));
-  if (fy + 1 < L.ny) ax += L.wy[i + 1] * (xc - xv(i + 1));
-  return ax;
+// Arrays of a tail level in LDS, each of its cells: the first level's x and y
+// (its operator and residual stay in registers), the coarsest level's x and r,
+// the levels' between x, y, r and the operator.
+uint32_t tail_arrays(uint32_t l, uint32_t count) { return l == 0 || l + 1 == count ? 2 : 7; }
+
+// The operator on a 2x2 aggregate: couplings to the lower cells outside it,
+// inside it and to the upper cells outside it along x (per column) and y (per
+// row), boundary terms and inverse diagonals of cell 2 a + b. Zero where the
+// grid ends.
+struct Quad {
+  float xl[2], xm[2], xu[2], yl[2], ym[2], yu[2], b[4], d[4];
+};
+
+__device__ inline Quad quad_load(const float* wx, const float* wy, const float* bc,
+                                 const float* dinv, uint32_t X, uint32_t Y, uint32_t nx,
+                                 uint32_t ny) {
+  const uint32_t fx = 2 * X, fy = 2 * Y, i = fx * ny + fy;
+  const bool x1 = fx + 1 < nx, x2 = fx + 2 < nx, y1 = fy + 1 < ny, y2 = fy + 2 < ny;
+  Quad q;
+#pragma unroll
+  for (uint32_t k = 0; k < 2; ++k) {
+    const bool yk = k == 0 || y1, xk = k == 0 || x1;
+    q.xl[k] = yk ? wx[i + k] : 0.0f;
+    q.xm[k] = x1 && yk ? wx[i + ny + k] : 0.0f;
+    q.xu[k] = x2 && yk ? wx[i + 2 * ny + k] : 0.0f;
+    q.yl[k] = xk ? wy[i + k * ny] : 0.0f;
+    q.ym[k] = y1 && xk ? wy[i + k * ny + 1] : 0.0f;
+    q.yu[k] = y2 && xk ? wy[i + k * ny + 2] : 0.0f;
+#pragma unroll
+    for (uint32_t b = 0; b < 2; ++b) {
+      const bool in = xk && (b == 0 || y1);
+      q.b[2 * k + b] = in ? bc[i + k * ny + b] : 0.0f;
+      q.d[2 * k + b] = in ? dinv[i + k * ny + b] : 0.0f;
+    }
+  }
+  return q;
 }
 
-// out = x + omega D^-1 (r - A x) on every cell of a tail level, x_j = xv(j).
-template <typename X>
-__device__ inline void tail_sweep(const TailLevel& L, X xv, float* out) {
-  const uint32_t cells = L.nx * L.ny;
-  for (uint32_t i = threadIdx.x; i < cells; i += kTailThreads) {
-    const uint32_t fx = i / L.ny, fy = i - fx * L.ny;
-    out[i] = xv(i) + kOmega * L.dinv[i] * (L.r[i] - tail_ax(L, xv, i, fx, fy));
+// Calls f(k, cell) for the aggregate's cells on the grid.
+template <class F>
+__device__ inline void quad_cells(uint32_t X, uint32_t Y, uint32_t nx, uint32_t ny, F&& f) {
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t fx = 2 * X + (k >> 1), fy = 2 * Y + (k & 1);
+    if (fx < nx && fy < ny) f(k, fx * ny + fy);
   }
 }
 
-// The cycle on the small levels in one workgroup: down passes, the dense
-// coarsest solve, up passes, with workgroup barriers between the phases.
-// The first sweep of each smoothing pair is not stored: the second sweep
-// evaluates it at the sites its stencil reads (from zero going down: omega
-// D^-1 r; going up: the prolonged iterate), so a level costs two phases each
-// way. The coarsest inverse is stored transposed, so the threads of a wave
-// read one row of it together.
+// A v on the aggregate's cells, v in LDS, and v itself; neighbours off the grid
+// are clamped to it (their coupling is zero). The terms in the order of the
+// tile kernels.
+__device__ inline void quad_ax(const Quad& q, const float* v, uint32_t X, uint32_t Y, uint32_t nx,
+                               uint32_t ny, float (&c)[4], float (&ax)[4]) {
+  const uint32_t fx = 2 * X, fy = 2 * Y;
+  const uint32_t r0 = fx * ny, r1 = fx + 1 < nx ? r0 + ny : r0;
+  const uint32_t rl = fx > 0 ? r0 - ny : r0, ru = fx + 2 < nx ? r1 + ny : r1;
+  const uint32_t c0 = fy, c1 = fy + 1 < ny ? fy + 1 : fy;
+  const uint32_t cl = fy > 0 ? fy - 1 : fy, cu = fy + 2 < ny ? fy + 2 : c1;
+  c[0] = v[r0 + c0];
+  c[1] = v[r0 + c1];
+  c[2] = v[r1 + c0];
+  c[3] = v[r1 + c1];
+  const float xl[2] = {v[rl + c0], v[rl + c1]}, xu[2] = {v[ru + c0], v[ru + c1]};
+  const float yl[2] = {v[r0 + cl], v[r1 + cl]}, yu[2] = {v[r0 + cu], v[r1 + cu]};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int a = k >> 1, b = k & 1;
+    float s = q.b[k] * c[k];
+    s += (a != 0 ? q.xm[b] : q.xl[b]) * (c[k] - (a != 0 ? c[b] : xl[b]));
+    s += (a != 0 ? q.xu[b] : q.xm[b]) * (c[k] - (a != 0 ? xu[b] : c[2 + b]));
+    s += (b != 0 ? q.ym[a] : q.yl[a]) * (c[k] - (b != 0 ? c[2 * a] : yl[a]));
+    s += (b != 0 ? q.yu[a] : q.ym[a]) * (c[k] - (b != 0 ? yu[a] : c[2 * a + 1]));
+    ax[k] = s;
+  }
+}
+
+// The cycle on the small levels in one workgroup, its vectors and the coarser
+// levels' operators in LDS: a thread owns whole aggregates, so a level costs
+// two barriers going down (x1 = omega D^-1 r, x2, the residual restricted) and
+// three going up, at LDS latency. With vectors and operators read from memory
+// in every phase a tail from 2048 cells took 17.9 us and one from 1316 cells
+// 23.3; this takes 11.3 and 11.5, of which the loads are four. The coarsest
+// inverse is stored transposed, so the threads of a wave read one row of it
+// together.
 __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TailArgs T, const CgState* st) {
+  extern __shared__ float lds[];
   __shared__ double s_red[kTailThreads / kWave];
-  if (cycle_stopped(st)) return;
-  for (uint32_t l = 0; l + 1 < T.count; ++l) {
-    const TailLevel& F = T.lv[l];
-    const TailLevel& Cl = T.lv[l + 1];
-    const float* fr = F.r;
-    const float* fd = F.dinv;
-    tail_sweep(F, [fr, fd](uint32_t j) { return kOmega * fd[j] * fr[j]; }, F.xp);
-    __syncthreads();
-    const float* fxp = F.xp;
-    const auto xp = [fxp](uint32_t j) { return fxp[j]; };
-    const uint32_t cells = Cl.nx * Cl.ny;
-    for (uint32_t c = threadIdx.x; c < cells; c += kTailThreads) {
-      const uint32_t X = c / Cl.ny, Y = c - X * Cl.ny;
-      float sum = 0.0f;
-      for (int a = 0; a < 2; ++a) {
-        for (int b = 0; b < 2; ++b) {
-          const uint32_t fx = 2 * X + a, fy = 2 * Y + b;
-          if (fx < F.nx && fy < F.ny) {
-            const uint32_t i = fx * F.ny + fy;
-            sum += F.r[i] - tail_ax(F, xp, i, fx, fy);
-          }
+  __shared__ float s_part[kTailThreads];
+  const uint32_t failure = st->failure, halt = st->halt;  // cycle_stopped, behind the loads
+  const uint32_t t = threadIdx.x, last = T.count - 1;
+  const uint32_t nx = T.lv[0].nx, ny = T.lv[0].ny, cells = nx * ny;
+  float* const x0 = lds;
+  float* const y0 = lds + cells;
+  const uint32_t cny = (ny + 1) / 2, quads = T.count == 1 ? 0 : (nx + 1) / 2 * cny;
+  Quad q[kTailQuads];
+  float r[kTailQuads][4], y[kTailQuads][4];
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      q[j] = quad_load(T.lv[0].wx, T.lv[0].wy, T.lv[0].bc, T.lv[0].dinv, X, Y, nx, ny);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) r[j][k] = 0.0f;
+      quad_cells(X, Y, nx, ny, [&](uint32_t k, uint32_t i) { r[j][k] = T.r[i]; });
+    }
+  }
+  // The coarsest inverse (below), whose columns wait for nothing: the first
+  // kAhead of the thread's range.
+  constexpr int kAhead = 16;
+  const uint32_t n = T.n;
+  const uint32_t parts = kTailThreads / n;  // n <= kCoarseCells <= kTailThreads / 4
+  const uint32_t span = (n + parts - 1) / parts;
+  const uint32_t row = t % n, part = t / n;
+  const uint32_t j0 = part * span, j1 = part < parts ? min(n, j0 + span) : 0;
+  float inverse[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j)
+    inverse[j] = j0 + j < j1 ? T.cinv[static_cast<size_t>(j0 + j) * n + row] : 0.0f;
+  // The operators of the levels between, all loads of a round in flight.
+  uint32_t operators = 0;
+  for (uint32_t l = 1; l < last; ++l) operators += 4 * T.lv[l].nx * T.lv[l].ny;
+  constexpr int kRound = 6;
+  for (uint32_t e0 = t; e0 < operators; e0 += kRound * kTailThreads) {
+    const float* from[kRound];
+    uint32_t to[kRound];
+    float v[kRound];
+    uint32_t first = 0;
+    for (uint32_t l = 1; l < last; ++l) {
+      const TailLevel L = T.lv[l];
+      const uint32_t m = L.nx * L.ny;
+#pragma unroll
+      for (int j = 0; j < kRound; ++j) {
+        const uint32_t e = e0 + static_cast<uint32_t>(j) * kTailThreads;
+        if (e >= first && e < first + 4 * m) {
+          const uint32_t in = e - first;
+          const uint32_t k = (in >= m ? 1u : 0u) + (in >= 2 * m ? 1u : 0u) + (in >= 3 * m ? 1u : 0u);
+          from[j] = (k == 0 ? L.wx : k == 1 ? L.wy : k == 2 ? L.bc : L.dinv) + (in - k * m);
+          to[j] = L.at + 3 * m + in;
         }
       }
-      Cl.r[c] = sum;
+      first += 4 * m;
+    }
+#pragma unroll
+    for (int j = 0; j < kRound; ++j) {
+      if (e0 + static_cast<uint32_t>(j) * kTailThreads < operators) v[j] = *from[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kRound; ++j) {
+      if (e0 + static_cast<uint32_t>(j) * kTailThreads < operators) lds[to[j]] = v[j];
+    }
+  }
+  if (failure != 0 || halt != 0) return;
+  if (T.count == 1) {
+    for (uint32_t i = t; i < cells; i += kTailThreads) lds[T.lv[0].at + cells + i] = T.r[i];
+  }
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      quad_cells(X, Y, nx, ny,
+                 [&](uint32_t k, uint32_t i) { x0[i] = kOmega * q[j].d[k] * r[j][k]; });
+    }
+  }
+  __syncthreads();
+  float ax[4], v[4];
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      quad_ax(q[j], x0, X, Y, nx, ny, v, ax);
+      quad_cells(X, Y, nx, ny, [&](uint32_t k, uint32_t i) {
+        y[j][k] = v[k] + kOmega * q[j].d[k] * (r[j][k] - ax[k]);
+        y0[i] = y[j][k];
+      });
+    }
+  }
+  __syncthreads();
+  // The restricted residual of aggregate c, with the next level's first sweep.
+  auto restricted = [&](uint32_t l, uint32_t c, float sum) {
+    const TailLevel& C = T.lv[l];
+    const uint32_t n = C.nx * C.ny;
+    float* at = lds + C.at;
+    if (l == last) {
+      at[n + c] = sum;
+    } else {
+      at[2 * n + c] = sum;
+      at[c] = kOmega * at[6 * n + c] * sum;
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      quad_ax(q[j], y0, X, Y, nx, ny, v, ax);
+      float sum = 0.0f;
+      quad_cells(X, Y, nx, ny, [&](uint32_t k, uint32_t) { sum += r[j][k] - ax[k]; });
+      restricted(1, c, sum);
+    }
+  }
+  __syncthreads();
+  // The levels between: one aggregate per thread at most.
+  struct Mid {
+    float *x, *y, *r;
+    Quad q;
+    uint32_t nx, ny, X, Y;
+    bool in;
+  };
+  auto mid = [&](uint32_t l) {
+    const TailLevel& L = T.lv[l];
+    const uint32_t n = L.nx * L.ny, w = (L.ny + 1) / 2;
+    Mid m;
+    m.nx = L.nx;
+    m.ny = L.ny;
+    m.X = t / w;
+    m.Y = t - m.X * w;
+    m.in = m.X < (L.nx + 1) / 2;
+    m.x = lds + L.at;
+    m.y = m.x + n;
+    m.r = m.x + 2 * n;
+    if (m.in)
+      m.q = quad_load(m.x + 3 * n, m.x + 4 * n, m.x + 5 * n, m.x + 6 * n, m.X, m.Y, L.nx, L.ny);
+    return m;
+  };
+  // out = in + omega D^-1 (r - A in) on the thread's aggregate.
+  auto sweep = [&](const Mid& m, const float* in, float* out) {
+    if (!m.in) return;
+    quad_ax(m.q, in, m.X, m.Y, m.nx, m.ny, v, ax);
+    quad_cells(m.X, m.Y, m.nx, m.ny, [&](uint32_t k, uint32_t i) {
+      out[i] = v[k] + kOmega * m.q.d[k] * (m.r[i] - ax[k]);
+    });
+  };
+  for (uint32_t l = 1; l < last; ++l) {
+    const Mid m = mid(l);
+    sweep(m, m.x, m.y);
+    __syncthreads();
+    if (m.in) {
+      quad_ax(m.q, m.y, m.X, m.Y, m.nx, m.ny, v, ax);
+      float sum = 0.0f;
+      quad_cells(m.X, m.Y, m.nx, m.ny, [&](uint32_t k, uint32_t i) { sum += m.r[i] - ax[k]; });
+      restricted(l + 1, t, sum);
     }
     __syncthreads();
   }
@@ -337,76 +531,100 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TailArgs T, const CgSt
     // rows of a wave adjacent, so each step of a thread's range is one
     // coalesced read of the transposed inverse; the ranges' sums are then
     // added in range order.
-    const TailLevel& B = T.lv[T.count - 1];
-    const bool dots = T.count == 1 && T.dots.q != nullptr;
-    __shared__ float s_r[kCoarseCells];
-    __shared__ float s_part[kTailThreads];
-    const uint32_t n = T.n;
-    for (uint32_t j = threadIdx.x; j < n; j += kTailThreads) s_r[j] = B.r[j];
-    __syncthreads();
-    const uint32_t parts = kTailThreads / n;  // n <= kCoarseCells <= kTailThreads / 4
-    const uint32_t span = (n + parts - 1) / parts;
-    if (threadIdx.x < parts * n) {
-      const uint32_t row = threadIdx.x % n, part = threadIdx.x / n;
-      const uint32_t j0 = part * span, j1 = min(n, j0 + span);
-      float v = 0.0f;
-      uint32_t j = j0;
-      for (; j + 8 <= j1; j += 8) {
+    float* e = lds + T.lv[last].at;
+    const float* s_r = e + n;
+    if (T.count == 1) __syncthreads();
+    if (part < parts) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        if (j0 + j < j1) sum += inverse[j] * s_r[j0 + j];
+      }
+      for (uint32_t j = j0 + kAhead; j < j1; j += 8) {
         float m[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) m[k] = T.cinv[static_cast<size_t>(j + k) * n + row];
+        for (uint32_t k = 0; k < 8; ++k)
+          m[k] = j + k < j1 ? T.cinv[static_cast<size_t>(j + k) * n + row] : 0.0f;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v += m[k] * s_r[j + k];
+        for (uint32_t k = 0; k < 8; ++k) {
+          if (j + k < j1) sum += m[k] * s_r[j + k];
+        }
       }
-      for (; j < j1; ++j) v += T.cinv[static_cast<size_t>(j) * n + row] * s_r[j];
-      s_part[part * n + row] = v;
+      s_part[part * n + row] = sum;
     }
     __syncthreads();
-    for (uint32_t row = threadIdx.x; row < n; row += kTailThreads) {
-      float v = 0.0f;
-      for (uint32_t part = 0; part < parts; ++part) v += s_part[part * n + row];
-      B.e[row] = v;
-      if (dots) {
-        zr += static_cast<double>(v) * static_cast<double>(s_r[row]);
-        zq += static_cast<double>(v) * static_cast<double>(T.dots.q[row]);
+    if (t < n) {
+      float sum = 0.0f;
+      for (uint32_t k = 0; k < parts; ++k) sum += s_part[k * n + t];
+      e[t] = sum;
+      if (T.count == 1) {
+        T.e[t] = sum;
+        if (T.dots.q != nullptr) {
+          zr += static_cast<double>(sum) * static_cast<double>(s_r[t]);
+          zq += static_cast<double>(sum) * static_cast<double>(T.dots.q[t]);
+        }
       }
     }
     __syncthreads();
   }
-  for (int l = static_cast<int>(T.count) - 2; l >= 0; --l) {
-    const TailLevel& F = T.lv[l];
-    const TailLevel& Cl = T.lv[l + 1];
-    const uint32_t cells = F.nx * F.ny;
-    const bool dots = l == 0 && T.dots.q != nullptr;
-    // The prolonged iterate x_pre + c P e_c, evaluated where it is read.
-    const float* fxp = F.xp;
-    const float* ce = Cl.e;
-    const uint32_t ny = F.ny, cny = Cl.ny;
-    const auto prolonged = [fxp, ce, ny, cny](uint32_t j) {
-      const uint32_t jx = j / ny, jy = j - jx * ny;
-      return fxp[j] + kCorrection * ce[(jx / 2) * cny + jy / 2];
-    };
-    tail_sweep(F, prolonged, F.t);
-    __syncthreads();
-    const float* ft = F.t;
-    const auto smoothed = [ft](uint32_t j) { return ft[j]; };
-    for (uint32_t i = threadIdx.x; i < cells; i += kTailThreads) {
-      const uint32_t fx = i / F.ny, fy = i - fx * F.ny;
-      const float ri = F.r[i];
-      const float z = F.t[i] + kOmega * F.dinv[i] * (ri - tail_ax(F, smoothed, i, fx, fy));
-      F.e[i] = z;
-      if (dots) {
-        zr += static_cast<double>(z) * static_cast<double>(ri);
-        zq += static_cast<double>(z) * static_cast<double>(T.dots.q[i]);
-      }
+  // Up: y = x_pre + c P e_c in x, its first sweep in y, the second in x.
+  for (uint32_t l = last; l-- > 1;) {
+    const Mid m = mid(l);
+    if (m.in) {
+      const float e = lds[T.lv[l + 1].at + t];
+      quad_cells(m.X, m.Y, m.nx, m.ny,
+                 [&](uint32_t, uint32_t i) { m.x[i] = m.y[i] + kCorrection * e; });
     }
     __syncthreads();
+    sweep(m, m.x, m.y);
+    __syncthreads();
+    sweep(m, m.y, m.x);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      const float e = lds[T.lv[1].at + c];
+      quad_cells(X, Y, nx, ny,
+                 [&](uint32_t k, uint32_t i) { x0[i] = y[j][k] + kCorrection * e; });
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      quad_ax(q[j], x0, X, Y, nx, ny, v, ax);
+      quad_cells(X, Y, nx, ny, [&](uint32_t k, uint32_t i) {
+        y0[i] = v[k] + kOmega * q[j].d[k] * (r[j][k] - ax[k]);
+      });
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kTailQuads; ++j) {
+    const uint32_t c = t + static_cast<uint32_t>(j) * kTailThreads;
+    if (c < quads) {
+      const uint32_t X = c / cny, Y = c - X * cny;
+      quad_ax(q[j], y0, X, Y, nx, ny, v, ax);
+      quad_cells(X, Y, nx, ny, [&](uint32_t k, uint32_t i) {
+        const float z = v[k] + kOmega * q[j].d[k] * (r[j][k] - ax[k]);
+        T.e[i] = z;
+        if (T.dots.q != nullptr) {
+          zr += static_cast<double>(z) * static_cast<double>(r[j][k]);
+          zq += static_cast<double>(z) * static_cast<double>(T.dots.q[i]);
+        }
+      });
+    }
   }
   if (T.dots.q != nullptr) {
     const uint32_t k = st->it_update + 1;
     const double a = block_sum<kTailThreads>(zr, s_red);
     const double b = block_sum<kTailThreads>(zq, s_red);
-    if (threadIdx.x == 0) {
+    if (t == 0) {
       T.dots.zr[(k & 1)] = a;
       T.dots.zq[(k & 1)] = b;
     }
@@ -805,10 +1023,20 @@ std::vector<float> coarse_inverse(const std::vector<float>& wx, const std::vecto
   return inv;
 }
 
+// The floats of LDS the levels from `tail` take.
+uint64_t tail_floats(const MgDevice& mg, uint32_t tail) {
+  const uint32_t count = static_cast<uint32_t>(mg.levels.size()) - tail;
+  uint64_t floats = 0;
+  for (uint32_t l = 0; l < count; ++l)
+    floats += tail_arrays(l, count) * mg.levels[tail + l]->cells();
+  return floats;
+}
+
 TailArgs tail_args(Context& ctx, float* r0, float* z0, const float* q0, FcgPartials parts) {
   auto& mg = ctx.flow.mg;
   const uint32_t tail = active_tail(mg);
   TailArgs T{};
+  uint32_t lds = 0;
   T.count = static_cast<uint32_t>(mg.levels.size()) - tail;
   for (uint32_t l = 0; l < T.count; ++l) {
     MgLevel& L = *mg.levels[tail + l];
@@ -817,16 +1045,16 @@ TailArgs tail_args(Context& ctx, float* r0, float* z0, const float* q0, FcgParti
     t.wy = L.wy.data();
     t.bc = L.bc.data();
     t.dinv = L.dinv.data();
-    t.r = L.r.data();
-    t.e = L.e.data();
-    t.xp = L.xp.data();
-    t.t = L.t.data();
     t.nx = L.nx;
     t.ny = L.ny;
+    t.at = lds;
+    lds += tail_arrays(l, T.count) * L.nx * L.ny;
   }
+  T.r = mg.levels[tail]->r.data();
+  T.e = mg.levels[tail]->e.data();
   if (tail == 0) {
-    T.lv[0].r = r0;
-    T.lv[0].e = z0;
+    T.r = r0;
+    T.e = z0;
     if (q0 != nullptr) T.dots = UpDots{q0, parts.zr, parts.zq};
   }
   T.cinv = mg.cinv.data();
@@ -876,7 +1104,8 @@ void launch_cycle(Context& ctx, float* r, float* z, const float* q, const hipEve
     if (l == 0 && probes != nullptr) check(hipEventRecord(probes[0], ctx.stream), "event");
   }
   if (tail == 0 && probes != nullptr) check(hipEventRecord(probes[0], ctx.stream), "event");
-  k_mg_tail<<<1, kTailThreads, 0, ctx.stream>>>(tail_args(ctx, r, z, q, parts), st);
+  k_mg_tail<<<1, kTailThreads, tail_floats(mg, tail) * sizeof(float), ctx.stream>>>(
+      tail_args(ctx, r, z, q, parts), st);
   check(hipGetLastError(), "launch k_mg_tail");
   if (tail == 0 && probes != nullptr) check(hipEventRecord(probes[1], ctx.stream), "event");
   for (int l = static_cast<int>(tail) - 1; l >= 0; --l) {
@@ -1058,7 +1287,7 @@ void mg_prepare(Context& ctx) {
   auto level0 = take(0, f.nx, f.ny);
   const size_t n = f.sites();
   for (auto* b : {&level0->wx, &level0->wy, &level0->bc, &level0->dinv, &level0->r, &level0->e,
-                  &level0->xp, &level0->t})
+                  &level0->xp})
     b->reserve(n);
   const float isx = static_cast<float>(1.0 / (static_cast<double>(f.dx) * f.dx));
   const float isy = static_cast<float>(1.0 / (static_cast<double>(f.dy) * f.dy));
@@ -1075,7 +1304,7 @@ void mg_prepare(Context& ctx) {
     MgLevel& F = *mg.levels.back();
     auto C = take(mg.levels.size(), (F.nx + 1) / 2, (F.ny + 1) / 2);
     const size_t cn = C->cells();
-    for (auto* b : {&C->wx, &C->wy, &C->bc, &C->dinv, &C->r, &C->e, &C->xp, &C->t})
+    for (auto* b : {&C->wx, &C->wy, &C->bc, &C->dinv, &C->r, &C->e, &C->xp})
       b->reserve(cn);
     const uint32_t cb = static_cast<uint32_t>((cn + 255) / 256);
     k_mg_coarsen<<<cb, 256, 0, ctx.stream>>>(view(F), C->wx.data(), C->wy.data(), C->bc.data(),
@@ -1089,7 +1318,10 @@ void mg_prepare(Context& ctx) {
   // The single-workgroup kernel takes every level from the first small one.
   mg.tail = static_cast<uint32_t>(mg.levels.size()) - 1;
   for (uint32_t l = 0; l < mg.levels.size(); ++l) {
-    if (mg.levels[l]->cells() <= kTailCells) {
+    const MgLevel& L = *mg.levels[l];
+    const uint64_t quads = static_cast<uint64_t>((L.nx + 1) / 2) * ((L.ny + 1) / 2);
+    if (L.cells() <= kTailCells && quads <= kTailQuads * kTailThreads &&
+        tail_floats(mg, l) <= kTailFloats) {
       mg.tail = l;
       break;
     }
