@@ -84,6 +84,28 @@ def test_coupled_steps_match_the_oracle(hip, oracle, kinds, scheme, integration)
         same_report(rep, ref)
 
 
+@pytest.mark.parametrize("signals", [1, 4, 5, 8])
+@pytest.mark.parametrize("cells", [1, 90])
+def test_sources_with_and_without_rates_read_ahead(hip, oracle, signals, cells):
+    """Many cells to a site, with as many signals as a site's runs hold ahead
+    (four) and more: the sums in the caller's order, bit for bit."""
+    nx, ny = 7, 5
+    kinds = TRANSPORT_KINDS[0]
+    c = random_transport_case(nx, ny, signals, kinds, 60 + signals)
+    g, prev = random_cells(signals, nx, ny, c["solid"], cells, 1.0, 0.8)
+    plan = uptake_plan(signals, 1)
+    species = np.random.default_rng(signals).random(len(prev)).astype(np.float32)
+    grid = msa.Grid(nx, ny, 1, 1.0, 0.8, 1.0, c["solid"], kinds)
+    og = OGrid(nx, ny, 1, 1.0, 0.8, 1.0, c["solid"], kinds)
+    ref_levels, ref_species, _ = oracle.advance_coupled(
+        og, c["levels"], g, species, plan, prev, 0.01,
+        **oracle_kw(c, msa.UPWIND, msa.FORWARD_EULER))
+    levels, sp, _ = hip.advance_coupled(spec_of(grid, c, msa.UPWIND, msa.FORWARD_EULER),
+                                        c["levels"], g, species, plan, prev, 0.01)
+    assert np.array_equal(levels, ref_levels)
+    assert np.array_equal(sp, ref_species)
+
+
 def test_bilinear_sample_and_scatter_known_answer(hip, oracle):
     """coupled_rates_test.cpp:45-72 on one layer: a cell at the centre of a
     2x2 box (spacing 2 x 1, level 4) samples 4, so species 10 + 0.5 * 4 = 12;
