@@ -249,8 +249,11 @@ __global__ void k_coupled_cells(CellParams P, const uint8_t* __restrict__ solid,
   const float volume_change_rate =
       P.dt == 0.0f ? 0.0f : (current_volume - previous_volume) / P.dt;
   // The rate plan (evaluate_instruction, cpu_coupled.cpp:20-85).
+  // The next instruction is read while this one runs.
+  msim_rate_instruction ahead = P.instructions > 0 ? plan[0] : msim_rate_instruction{};
   for (uint32_t index = 0; index < P.instructions; ++index) {
-    const msim_rate_instruction in = plan[index];
+    const msim_rate_instruction in = ahead;
+    if (index + 1 < P.instructions) ahead = plan[index + 1];
     const float a = in.operation >= MSIM_RATE_ADD && in.operation <= MSIM_RATE_SELECT
                         ? work[in.first * T]
                         : 0.0f;
