@@ -1,7 +1,7 @@
 // Explicit advection-diffusion-reaction step on the device, one layer.
 //
-// One marching kernel, k_adr_step, in two arithmetic forms: a block owns a
-// strip of columns and walks x, each thread advancing every signal of its
+// One marching kernel, k_adr_step, in two arithmetic forms: a wave owns a
+// strip of columns and walks x, each lane advancing every signal of its
 // site, so levels, faces, mask and occupancy are read from memory once.
 //  * FP32 levels: the reference's per-site rate in its own float order
 //    (cpp/core/signals.cpp:1145-1291 transport, 305-320 affine reaction,
