@@ -748,8 +748,8 @@ int msim_hip_learned_apply(msim_ctx* ctx, uint32_t pair, float* z);
  *
  * The pressure (FP32 Jacobi-PCG corrections with FP64 dot products inside
  * FP64 iterative refinement of an FP64 pressure, warm-started, to an FP64
- * true relative residual) is solved by msim_hip_batch_solve_flow: one launch,
- * one workgroup per instance. A step is one launch over work items (blocks of
+ * true relative residual) is solved by msim_hip_batch_solve_flow, all
+ * instances together. A step is one launch over work items (blocks of
  * rows, spread over the chip): each checks its rows' FP64 pressure residual,
  * rebuilds their face velocities and advances them one FP32 forward-Euler
  * transport step whose sites compute exactly as msim_hip_advance_signal_grid's
@@ -780,7 +780,7 @@ int msim_hip_batch_upload(msim_ctx* ctx, uint32_t count, const msim_batch_instan
                           const msim_batch_params* params);
 
 /* Solves every instance's pressure from its current one and rebuilds its
- * velocities (one launch). Per-instance outputs (count each, any may be
+ * velocities. Per-instance outputs (count each, any may be
  * NULL): FP32 CG iterations, final FP64 true relative residual, flags (1 CG
  * breakdown, 2 not converged within max_iterations, 4 a negative or
  * non-finite level). */
