@@ -19,12 +19,21 @@ constexpr int kStripWaves = kStripBlock / kWave;
 
 // Launch shape of a walk: strips of one wave, four waves per block, 12 x-rows
 // per wave, or 8 or 4 on smaller grids for at least 4096 waves (one round of 16
-// per compute unit). The explicit step at 4096x2048 with three signals (FP64
-// upwind, FP32 upwind, FP32 van Leer): 12 rows take 131, 74 and 109 us, 8 rows
-// 135, 77 and 111, 16 rows 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows
-// 151, 78 and 111: longer walks read fewer rows twice but leave a last round
-// of waves nearly empty. At 1531x769 (two signals) 4 rows instead of 8: 19.5
-// for 20.5 us FP64, 20.8 for 22.9 van Leer.
+// per compute unit), and 2 or 1 on those where 4 leave less than 3072. The
+// explicit step at 4096x2048 with three signals (FP64 upwind, FP32 upwind, FP32
+// van Leer): 12 rows take 131, 74 and 109 us, 8 rows 135, 77 and 111, 16 rows
+// 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows 151, 78 and 111: longer
+// walks read fewer rows twice but leave a last round of waves nearly empty. On
+// small grids a walk is a chain of rows, and one of a single row, whose three
+// rows are read at once, the latency of a thread per site. us with 1, 2 and 4
+// rows, three signals:
+//             FP64 upwind       FP32 upwind       FP32 van Leer     a Crank-Nicolson step
+//   256x128    6.8  8.2 10.6     5.3  6.2  8.4     9.7 10.8 13.5    190  359  418
+//   400x300   10.3  9.3 11.3     6.3  6.8  9.0    11.1 11.8 14.4    198  210  262
+//   768x512   15.7 12.9 12.9     8.4  8.2  9.2    14.3 13.9 15.0    237  228  256
+//   1024x512  18.8 16.2 15.9     9.7  9.3 10.3    16.4 15.5 17.2    277  261  290
+//   1531x769  35.4 29.1 25.8    18.1 17.2 15.4    28.9 27.5 25.2    411  398  354
+// (the 256x128 Crank-Nicolson steps are bimodal: 185 to 333 with one row).
 struct AdrShape {
   uint32_t strips, rows, blocks;
 };
@@ -37,7 +46,9 @@ inline AdrShape adr_shape(uint32_t nx, uint32_t ny, bool limited) {
   const uint32_t width = static_cast<uint32_t>(kWave) - (limited ? 4 : 2);
   const uint32_t strips = (ny + width - 1) / width;
   uint32_t rows = 12;
-  while (rows > 4 && static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows) < 4096) rows -= 4;
+  auto waves = [&] { return static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows); };
+  while (rows > 4 && waves() < 4096) rows -= 4;
+  while (rows <= 4 && rows > 1 && waves() < 3072) rows /= 2;
   return adr_shape(strips, nx, rows);
 }
 

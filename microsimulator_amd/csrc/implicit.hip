@@ -32,7 +32,9 @@ namespace msim {
 namespace {
 
 constexpr int kImplicitBlock = 256;
-constexpr int kJudgeBlock = 1024;        // of the two single-block kernels
+// Threads of the two single-block kernels, however few the partials: a step at
+// 400x300 (500 of them) takes 190 us with 1024 and 198 with 256.
+constexpr int kJudgeBlock = 1024;
 constexpr uint32_t kImplicitBatch = 16;  // iterations between host checks
 
 // The iteration's site work shared by the setup and the sweep: the site's

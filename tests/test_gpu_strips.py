@@ -1,5 +1,5 @@
 """The explicit transport step at the edges of its strips (62 columns per wave,
-60 under van Leer) and walks (4, 8 or 12 x-rows), FP32 bit for bit with the
+60 under van Leer) and walks (1, 2, 4, 8 or 12 x-rows), FP32 bit for bit with the
 oracle, which is bit-exact with the reference, and FP64 to 1e-13 relative."""
 import numpy as np
 import pytest
@@ -22,7 +22,8 @@ KINDS = [(FIXED, FIXED, NO_FLUX, FIXED, NO_FLUX, NO_FLUX),
 @pytest.mark.parametrize("shape,S", [
     ((4, 59), 1), ((5, 60), 3), ((3, 61), 1), ((13, 62), 2), ((11, 63), 3), ((12, 64), 8),
     ((25, 119), 1), ((7, 121), 2), ((6, 124), 5), ((9, 125), 1), ((2, 2), 1), ((1, 63), 1),
-    ((1500, 61), 1), ((2300, 187), 1),
+    ((1500, 61), 1), ((2300, 187), 1), ((3101, 61), 1), ((3071, 63), 2), ((8195, 63), 1),
+    ((16399, 64), 1),
 ])
 def test_step_at_strip_edges(hip, oracle, shape, S, limited, kinds):
     nx, ny = shape
@@ -85,11 +86,14 @@ def test_settle_of_a_marked_step(hip, oracle):
 
 @pytest.mark.parametrize("limited", [False, True])
 @pytest.mark.parametrize("shape,kinds", [((13, 62), KINDS[0]), ((5, 61), KINDS[1]),
-                                         ((30, 125), KINDS[2]), ((1400, 63), KINDS[0])])
+                                         ((30, 125), KINDS[2]), ((1400, 63), KINDS[0]),
+                                         ((1, 130), KINDS[2]), ((3101, 61), KINDS[1]),
+                                         ((3071, 63), KINDS[0]), ((3091, 121), KINDS[1]),
+                                         ((8195, 63), KINDS[2]), ((16399, 64), KINDS[0])])
 def test_implicit_steps_at_strip_edges(hip, oracle, shape, kinds, limited):
     """Several implicit steps on the device (the accepted iterate changes
     buffers from step to step by its parity) bit for bit with the oracle's,
-    obstacle levels included."""
+    obstacle levels included; walks of 1, 2, 4 and 8 rows with ragged ends."""
     nx, ny = shape
     c = random_transport_case(nx, ny, 2, kinds, seed=3 * nx + ny)
     scheme = msa.VAN_LEER if limited else msa.UPWIND
