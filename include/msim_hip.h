@@ -148,6 +148,26 @@ const char* msim_hip_last_error(const msim_ctx* ctx);
 /* BackendInfo::device (types.hpp:77-83): the device's name. */
 int msim_hip_device_name(msim_ctx* ctx, char* name, size_t length);
 
+/* What the persistent solves of a context may take. Jacobi-PCG on systems of up
+ * to about a million sites and the resolved flow's momentum solves of up to a
+ * million faces run as launches whose workgroups are all resident and wait for
+ * each other's words; where that is not possible, or a workgroup has waited too
+ * long because other work holds the compute units, the solve goes by separate
+ * launches instead, with the same answer to its tolerance. */
+typedef struct {
+  uint32_t workgroups; /* of one launch, at most; 0: no persistent launches. At creation one
+                          per compute unit, or 0 on a device without cooperative launches */
+  uint32_t polls;      /* how often a workgroup looks again for the others' words (about a
+                          microsecond each) before the launch is given up; 2^21 - 1 at creation */
+  uint32_t round_tag;  /* the number of the next meeting of the workgroups; counts up, and
+                          starts over before 2^32. Setting it can only raise it */
+} msim_resident_limits;
+
+int msim_hip_get_resident_limits(msim_ctx* ctx, msim_resident_limits* limits);
+
+/* Limits above those at creation are taken as those. */
+int msim_hip_set_resident_limits(msim_ctx* ctx, const msim_resident_limits* limits);
+
 /* ComputeBackend::solve_depth_averaged_flow (backend.hpp:44-46): host arrays
  * in, the velocity field out. mobility: one float per site or NULL (the
  * reference's Hele-Shaw default). x/y/z_faces: face velocities. A grid of

@@ -111,6 +111,10 @@ class _NutrientStep(C.Structure):
                 ("solve_seconds", C.c_double)]
 
 
+class _ResidentLimits(C.Structure):
+    _fields_ = [("workgroups", C.c_uint32), ("polls", C.c_uint32), ("round_tag", C.c_uint32)]
+
+
 class _FlowReport(C.Structure):
     _fields_ = [("iterations", C.c_uint32), ("refinements", C.c_uint32),
                 ("relative_residual", C.c_double), ("true_relative_residual", C.c_double),
@@ -219,7 +223,8 @@ RateOp = type("RateOp", (), {name.upper(): code for code, name in enumerate(RATE
 #: Every entry point include/msim_hip.h declares.
 EXPORTS = (
     "msim_hip_device_count", "msim_hip_create", "msim_hip_destroy", "msim_hip_last_error",
-    "msim_hip_device_name", "msim_hip_solve_depth_averaged_flow", "msim_hip_flow_prepare",
+    "msim_hip_device_name", "msim_hip_get_resident_limits", "msim_hip_set_resident_limits",
+    "msim_hip_solve_depth_averaged_flow", "msim_hip_flow_prepare",
     "msim_hip_flow_solve", "msim_hip_flow_download", "msim_hip_flow_apply",
     "msim_hip_flow_arrays", "msim_hip_flow_precondition", "msim_hip_advance_signal_grid", "msim_hip_adr_upload",
     "msim_hip_adr_run", "msim_hip_adr_download", "msim_hip_adr_seconds",
@@ -259,6 +264,8 @@ def library(path: str = LIBRARY):
         "msim_hip_destroy": (None, [P]),
         "msim_hip_last_error": (C.c_char_p, [P]),
         "msim_hip_device_name": (I, [P, C.c_char_p, C.c_size_t]),
+        "msim_hip_get_resident_limits": (I, [P, P]),
+        "msim_hip_set_resident_limits": (I, [P, P]),
         "msim_hip_solve_depth_averaged_flow": (I, [P, P, P, P, P, P, P, P]),
         "msim_hip_flow_prepare": (I, [P, P, P, U]),
         "msim_hip_flow_solve": (I, [P, P, P]),
@@ -869,6 +876,21 @@ class HipBackend:
         buf = C.create_string_buffer(256)
         self._check(self.lib.msim_hip_device_name(self.ctx, buf, 256))
         return BackendInfo(device=buf.value.decode(), device_index=self.device_index)
+
+    def resident_limits(self) -> dict:
+        """What the persistent solves of this context may take (msim_hip.h)."""
+        limits = _ResidentLimits()
+        self._check(self.lib.msim_hip_get_resident_limits(self.ctx, C.byref(limits)))
+        return {name: getattr(limits, name) for name, _ in _ResidentLimits._fields_}
+
+    def set_resident_limits(self, **limits):
+        """Changes the named limits and leaves the others."""
+        now = self.resident_limits()
+        unknown = set(limits) - set(now)
+        if unknown:
+            raise TypeError(f"unknown resident limits: {', '.join(sorted(unknown))}")
+        self._check(self.lib.msim_hip_set_resident_limits(
+            self.ctx, C.byref(_ResidentLimits(**{**now, **limits}))))
 
     def supports(self, feature: str) -> bool:
         return feature in SUPPORTED

@@ -1227,8 +1227,10 @@ int msim_hip_create(int device, msim_ctx** out) {
     ctx->impl.name = prop.name;
     if (ctx->impl.name.empty()) ctx->impl.name = prop.gcnArchName;
     if (prop.cooperativeLaunch != 0)
-      ctx->impl.resident_blocks = static_cast<uint32_t>(prop.multiProcessorCount);
+      ctx->impl.resident_most.workgroups = static_cast<uint32_t>(prop.multiProcessorCount);
   }
+  ctx->impl.resident_most.polls = msim::kRoundPolls;
+  ctx->impl.resident = ctx->impl.resident_most;
   *out = ctx;
   return MSIM_OK;
 }
@@ -1255,6 +1257,22 @@ int msim_hip_device_name(msim_ctx* ctx, char* name, size_t length) {
   return msim::guarded(ctx, [&](Context& c) {
     if (name == nullptr || length == 0) msim::invalid("name buffer must not be empty");
     std::snprintf(name, length, "%s", c.name.c_str());
+  });
+}
+
+int msim_hip_get_resident_limits(msim_ctx* ctx, msim_resident_limits* limits) {
+  return msim::guarded(ctx, [&](Context& c) {
+    if (limits == nullptr) msim::invalid("limits must not be null");
+    *limits = c.resident;
+  });
+}
+
+int msim_hip_set_resident_limits(msim_ctx* ctx, const msim_resident_limits* limits) {
+  return msim::guarded(ctx, [&](Context& c) {
+    if (limits == nullptr) msim::invalid("limits must not be null");
+    c.resident.workgroups = std::min(limits->workgroups, c.resident_most.workgroups);
+    c.resident.polls = std::min(limits->polls, c.resident_most.polls);
+    c.resident.round_tag = std::max(limits->round_tag, c.resident.round_tag);
   });
 }
 

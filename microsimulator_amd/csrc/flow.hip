@@ -447,7 +447,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
     T* __restrict__ r, T* __restrict__ xsol, T* __restrict__ p, uint64_t* words,
     const float* __restrict__ diag, const float* __restrict__ cxl, const float* __restrict__ cyl,
     const float* __restrict__ bc, uint32_t n, uint32_t ny, T isx, T isy, CgState* st,
-    uint64_t* slots, uint32_t tag, uint32_t budget, uint32_t taken) {
+    uint64_t* slots, uint32_t tag, uint32_t polls, uint32_t budget, uint32_t taken) {
   constexpr int NT = kPersistThreads;
   constexpr int kAhead = 2;  // halo values polled for with the sums, per thread
   extern __shared__ __align__(16) unsigned char s_raw[];
@@ -530,8 +530,9 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
         z = z_of(i);
       } else {
         uint64_t w[Exchange<T>::kWords];
+        if (round_stalled(L)) break;
         poll_words(
-            L, [&] { ex.load(i, w); }, [&] { return Exchange<T>::has(w, tag - 1); });
+            L, polls, [&] { ex.load(i, w); }, [&] { return Exchange<T>::has(w, tag - 1); });
         z = Exchange<T>::value(w);
       }
       s_p[halo_slot(h)] = z + beta * s_p[halo_slot(h)];
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
       }
     }
     alive = round_sums<1>(
-        pq, slots, tag++, L, [] {}, [] { return true; });
+        pq, slots, tag++, polls, L, [] {}, [] { return true; });
     if (!alive) break;
     curvature = pq[0];
     if (!isfinite(curvature) || curvature <= 0.0) {
@@ -583,7 +584,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
     }
     uint64_t w[kAhead][Exchange<T>::kWords];
     alive = round_sums<2>(
-        sums, slots, tag, L,
+        sums, slots, tag, polls, L,
         [&] {
 #pragma unroll
           for (int u = 0; u < kAhead; ++u) {
@@ -869,12 +870,12 @@ __global__ __launch_bounds__(kStream) void k_scale(float* __restrict__ faces, si
 
 uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words) {
   // Fresh memory and reused tags are cleared: a word counts by its tag.
-  const bool fresh = ctx.round_slots.size() == 0 || ctx.round_tag > 0xffffffffu - rounds;
+  const bool fresh = ctx.round_slots.size() == 0 || ctx.resident.round_tag > 0xffffffffu - rounds;
   if (fresh) {
     ctx.round_slots.reserve(kRoundSlots);
     check(hipMemsetAsync(ctx.round_slots.data(), 0, kRoundSlots * sizeof(uint64_t), ctx.stream),
           "clear rounds");
-    ctx.round_tag = 1;
+    ctx.resident.round_tag = 1;
   }
   if (words > ctx.round_words.size()) {
     ctx.round_words.reserve(words);
@@ -886,14 +887,14 @@ uint32_t take_rounds(Context& ctx, uint32_t rounds, size_t words) {
                          ctx.stream),
           "clear exchange");
   }
-  const uint32_t tag = ctx.round_tag;
-  ctx.round_tag += rounds;
+  const uint32_t tag = ctx.resident.round_tag;
+  ctx.resident.round_tag += rounds;
   return tag;
 }
 
 ResidentShape resident_shape(const Context& ctx, size_t entries, size_t halo, size_t bytes,
                              size_t lds_limit) {
-  const size_t room = std::min<size_t>(ctx.resident_blocks, kRoundBlocks);
+  const size_t room = std::min<size_t>(ctx.resident.workgroups, kRoundBlocks);
   for (int s : {1, 2, 4, 8}) {
     const size_t chunk = static_cast<size_t>(kPersistThreads) * s;
     const size_t blocks = (entries + chunk - 1) / chunk;
@@ -909,7 +910,8 @@ bool launch_resident(Context& ctx, const void* kernel, uint32_t blocks, void** a
   const hipError_t status = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads),
                                                        args, static_cast<uint32_t>(lds),
                                                        ctx.stream);
-  if (status == hipErrorCooperativeLaunchTooLarge) {
+  if (status == hipErrorCooperativeLaunchTooLarge || status == hipErrorNotSupported ||
+      status == hipErrorLaunchOutOfResources) {
     static_cast<void>(hipGetLastError());
     return false;
   }
@@ -1080,8 +1082,9 @@ bool launch_persistent(Context& ctx, const ResidentShape& shape, T* r, T* x, T* 
   CgState* st = f.state.data();
   uint32_t tag = take_rounds(ctx, 2 * budget, Exchange<T>::kWords * f.sites());
   uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
+  uint32_t polls = ctx.resident.polls;
   void* args[] = {&r, &x, &p, &words, &diag, &cxl, &cyl, &bc, &n, &ny, &isx, &isy,
-                  &st, &slots, &tag, &budget, &taken};
+                  &st, &slots, &tag, &polls, &budget, &taken};
   const void* kernel = nullptr;
   switch (shape.per_thread) {
     case 1: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 1>); break;
@@ -1093,14 +1096,17 @@ bool launch_persistent(Context& ctx, const ResidentShape& shape, T* r, T* x, T* 
 }
 
 // Runs Jacobi-PCG iterations of precision T on the prepared system from the
-// state launch_init left, until the stopping test holds, a failure, or
+// state `init` (a launch_init) leaves, until the stopping test holds, a failure, or
 // `budget` iterations (conjugate_gradient.hpp:126-166: the host looks at the
 // device's state once per `interval` iterations). The operator kernel of
 // iteration k+1 makes iteration k's stopping test; one more operator launch
 // after the budget makes the last test. Returns the iterations taken (the
-// iteration that met the test, or the budget). Throws on a CG failure.
-template <typename T>
-uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, uint32_t interval,
+// iteration that met the test, or the budget). Throws on a CG failure. Where a
+// persistent launch was given up (other work held the compute units past its
+// workgroups' patience) or the device no longer takes it, the iteration starts
+// over from `init` by launches, and so does the rest of the solve.
+template <typename T, typename Init>
+uint32_t run_cg(Context& ctx, Init&& init, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, uint32_t interval,
                 bool* converged, double* relative, KernelTimes* times) {
   auto& f = ctx.flow;
   T* buf[2] = {pa, pb};
@@ -1112,6 +1118,7 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
       ctx.probes.push_back(e);
     }
   }
+  init();
   read_state(ctx);
   if (f.host_state->done != 0) {  // r.r of the right-hand side is zero
     *converged = true;
@@ -1120,8 +1127,6 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
   }
   const double rr0 = f.host_state->rr0;
   auto judge = [&](const CgState& s) {
-    if (s.failure == kRoundStalled)
-      throw Error(MSIM_DEVICE_ERROR, "HIP depth-averaged flow conjugate gradient stalled");
     if (s.failure != 0) {
       throw Error(failure_status(s.failure),
                   std::string("HIP depth-averaged flow conjugate gradient ") +
@@ -1131,7 +1136,8 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
     *converged = s.halt != 0;
     return *converged;
   };
-  const ResidentShape shape = times == nullptr ? persist_shape<T>(ctx) : ResidentShape{};
+  const ResidentShape shape =
+      times == nullptr && !f.by_launches ? persist_shape<T>(ctx) : ResidentShape{};
   if (shape.per_thread != 0 && budget > 0) {
     // Launches of kPersistIterations, so none runs for more than some tens of
     // milliseconds; the direction stays in pa.
@@ -1140,12 +1146,13 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
       const uint32_t batch = std::min(kPersistIterations, budget - taken);
       if (!launch_persistent<T>(ctx, shape, r, x, pa, batch, taken)) break;
       read_state(ctx);
+      if (f.host_state->failure == kRoundStalled) break;
       if (judge(*f.host_state)) return f.host_state->halt;
       taken += batch;
     }
     if (taken >= budget) return budget;
-    if (taken > 0)
-      throw Error(MSIM_DEVICE_ERROR, "HIP depth-averaged flow conjugate gradient was not resumed");
+    f.by_launches = true;
+    init();
   }
   uint32_t launched = 0;  // iterations launched
   bool tested_all = false;
@@ -1194,9 +1201,11 @@ uint32_t run_cg(Context& ctx, T* r, T* x, T* q, T* pa, T* pb, uint32_t budget, u
 uint32_t jacobi_solve(Context& ctx, double tolerance, uint32_t budget, uint32_t interval,
                       bool* converged, double* relative, KernelTimes* times) {
   auto& f = ctx.flow;
-  launch_init<double, float>(ctx, f.rhs.data(), 1.0, f.r.data(), f.x.data(), f.p0.data(),
-                             tolerance);
-  const uint32_t iterations = run_cg<double>(ctx, f.r.data(), f.x.data(), f.q.data(),
+  const auto init = [&] {
+    launch_init<double, float>(ctx, f.rhs.data(), 1.0, f.r.data(), f.x.data(), f.p0.data(),
+                               tolerance);
+  };
+  const uint32_t iterations = run_cg<double>(ctx, init, f.r.data(), f.x.data(), f.q.data(),
                                              f.p0.data(), f.p1.data(), budget, interval,
                                              converged, relative, times);
   launch_residual(ctx, f.x.data(), f.res.data(), 1);
@@ -1231,11 +1240,13 @@ uint32_t jacobi_continue(Context& ctx, double tolerance, uint32_t budget, uint32
     // Half the needed reduction as the recursive target: the true residual
     // of an FP64 solve stays within a small factor of the recursive one.
     const double inner = std::max(0.5 * tolerance * bnorm / rnorm, 1.0e-15);
-    launch_init<double, double>(ctx, f.res.data(), 1.0, f.r.data(), f.xc.data(), f.p0.data(),
-                                inner);
+    const auto init = [&] {
+      launch_init<double, double>(ctx, f.res.data(), 1.0, f.r.data(), f.xc.data(), f.p0.data(),
+                                  inner);
+    };
     bool inner_converged = false;
     double inner_relative = 0.0;
-    const uint32_t taken = run_cg<double>(ctx, f.r.data(), f.xc.data(), f.q.data(), f.p0.data(),
+    const uint32_t taken = run_cg<double>(ctx, init, f.r.data(), f.xc.data(), f.q.data(), f.p0.data(),
                                           f.p1.data(), budget - iterations, interval,
                                           &inner_converged, &inner_relative, times);
     iterations += taken;
@@ -1314,6 +1325,7 @@ void flow_assemble(Context& ctx, const uint8_t* solid_host, const float* mobilit
   check(hipStreamSynchronize(ctx.stream), "assemble");
   f.prepared = true;
   f.solved = false;
+  f.by_launches = false;
   ++f.generation;
   f.mg.ready = false;
 }
@@ -1344,6 +1356,7 @@ void solve_pressure(Context& ctx, const msim_flow_params& params, msim_flow_repo
   uint32_t iterations = 0;
   bool converged = false;
   double relative = 0.0;
+  f.by_launches = false;
   if (params.solver == MSIM_SOLVER_JACOBI_FP64) {
     iterations = jacobi_solve(ctx, params.relative_tolerance, params.max_iterations, interval,
                               &converged, &relative, times);
@@ -1372,11 +1385,13 @@ void solve_pressure(Context& ctx, const msim_flow_params& params, msim_flow_repo
       }
       if (iterations >= params.max_iterations || refinements >= 64) break;
       // Inner FP32 solve of A e = res / ||res|| to `inner`.
-      launch_init<float, double>(ctx, f.res.data(), 1.0 / rnorm, f.r32.data(), f.x32.data(),
-                                 f.p032.data(), inner);
+      const auto init = [&] {
+        launch_init<float, double>(ctx, f.res.data(), 1.0 / rnorm, f.r32.data(), f.x32.data(),
+                                   f.p032.data(), inner);
+      };
       bool inner_converged = false;
       double inner_relative = 0.0;
-      const uint32_t taken = run_cg<float>(ctx, f.r32.data(), f.x32.data(), f.q32.data(),
+      const uint32_t taken = run_cg<float>(ctx, init, f.r32.data(), f.x32.data(), f.q32.data(),
                                            f.p032.data(), f.p132.data(),
                                            params.max_iterations - iterations, interval,
                                            &inner_converged, &inner_relative, times);

@@ -174,6 +174,9 @@ struct FlowDevice {
   // Counts flow solves and preparations: a transport that reads the field in
   // place records the count it was uploaded at, and is refused once it moves.
   uint64_t generation = 0;
+  // A persistent launch of this solve was given up: the rest of it goes by
+  // launches.
+  bool by_launches = false;
   // Port-driven flow: the open exterior faces and the pressures held outside
   // them (FlowEdges slots) instead of the axis boundary.
   bool ported = false;
@@ -381,11 +384,9 @@ struct Context {
   ColonyDevice colony;
   std::shared_ptr<BatchDevice> batch;
   // Persistent solves (persist.hpp): the rounds' words, the exchanged values'
-  // words and the next tag, and how many workgroups can be resident, one per
-  // compute unit (0: no cooperative launches on this device).
+  // words, and what they may take of the device and what it has.
   DeviceBuffer<uint64_t> round_slots, round_words;
-  uint32_t round_tag = 0;
-  uint32_t resident_blocks = 0;
+  msim_resident_limits resident{}, resident_most{};
 };
 
 // Summed event time and launch count of the two Krylov kernels of a solve.
@@ -412,6 +413,9 @@ void launch_assembly(hipStream_t stream, const uint8_t* solid, const float* mobi
 // A ported system: holds each open face at the pressure of its slot in
 // `pressure_host` (FlowEdges layout) and reassembles the right-hand side.
 void flow_hold_pressures(Context& ctx, const float* pressure_host);
+// msim_resident_limits::polls at creation: a look is a trip to memory of about a
+// microsecond, so some seconds.
+constexpr uint32_t kRoundPolls = (1u << 21) - 1;
 // The shape of a persistent solve over `entries` entries whose direction, with
 // `halo` entries either side, is held in LDS: 1 or 2 entries per thread while
 // that leaves at most 16 workgroups, else 4, else 8; none (per_thread 0) where

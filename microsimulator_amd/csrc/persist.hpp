@@ -27,13 +27,13 @@ constexpr int kRoundWords = 4;          // words a workgroup publishes in one ro
 // Two generations by tag parity: a workgroup can be one round ahead of the
 // slowest, never two.
 constexpr size_t kRoundSlots = 2ull * kRoundWords * kRoundBlocks;
-// A workgroup that waits this long (100 MHz ticks: 2 s) gives the solve up;
-// the others then do too, so the launch always ends.
-constexpr uint64_t kRoundTicks = 200'000'000ull;
-constexpr uint32_t kRoundStalled = 6;  // CgState::failure of a solve given up that way
+// A workgroup that has looked for the others' words as often as its launch's
+// `polls` allow gives the launch up, and the others then do too, so the launch
+// always ends; the caller starts over without it. Looks and not a clock: a
+// preempted workgroup's clock runs on.
+constexpr uint32_t kRoundStalled = 6;  // CgState::failure of a launch given up that way
 // Iterations of one persistent launch (some tens of milliseconds).
 constexpr uint32_t kPersistIterations = 4096;
-
 
 __device__ inline void word_store(uint64_t* at, uint32_t tag, uint32_t bits) {
   __hip_atomic_store(at, (static_cast<uint64_t>(tag) << 32) | bits, __ATOMIC_RELAXED,
@@ -114,20 +114,21 @@ struct RoundLds {
   int stalled;
 };
 
+// Whether a thread of this workgroup has given up.
+__device__ inline bool round_stalled(const RoundLds& L) {
+  return __hip_atomic_load(&L.stalled, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+}
+
 // Polls: `issue` loads words, `done` says whether all of them show their tag.
+// Gives up after `polls` further looks, or soon after another thread has.
 template <class Issue, class Done>
-__device__ inline void poll_words(RoundLds& L, Issue&& issue, Done&& done) {
-  uint64_t since = 0;
-  for (uint32_t spins = 1;; ++spins) {
+__device__ inline void poll_words(RoundLds& L, uint32_t polls, Issue&& issue, Done&& done) {
+  for (uint32_t left = polls;; --left) {
     issue();
     if (done()) return;
-    if ((spins & 255u) == 0) {
-      const uint64_t now = wall_clock64();
-      if (since == 0) since = now;
-      if (now - since > kRoundTicks) {
-        L.stalled = 1;
-        return;
-      }
+    if ((left & 255u) == 0 && (left == 0 || round_stalled(L))) {
+      __hip_atomic_store(&L.stalled, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      return;
     }
   }
 }
@@ -137,8 +138,8 @@ __device__ inline void poll_words(RoundLds& L, Issue&& issue, Done&& done) {
 // fixed tree. Consecutive rounds take consecutive tags. The words `issue`
 // loads are polled for along with the sums. False: stalled.
 template <int K, class Issue, class Done>
-__device__ inline bool round_sums(double (&v)[K], uint64_t* slots, uint32_t tag, RoundLds& L,
-                                  Issue&& issue, Done&& done) {
+__device__ inline bool round_sums(double (&v)[K], uint64_t* slots, uint32_t tag, uint32_t polls,
+                                  RoundLds& L, Issue&& issue, Done&& done) {
   static_assert(2 * K <= kRoundWords);
   constexpr int kWaves = kPersistThreads / kWave;
   const int t = threadIdx.x, wave = t / kWave;
@@ -164,7 +165,7 @@ __device__ inline bool round_sums(double (&v)[K], uint64_t* slots, uint32_t tag,
   for (int j = 0; j < 2 * K; ++j) w[j] = static_cast<uint64_t>(tag) << 32;  // 0.0
   const bool reads = t < static_cast<int>(gridDim.x);
   poll_words(
-      L,
+      L, polls,
       [&] {
         if (reads) {
 #pragma unroll

@@ -9,6 +9,8 @@ allowance of 2 (tests/conformance/flow_conformance_test.cpp:259-263). Their
 fields differ by what an iteration leaves at the stated residual, bounded for
 these systems by 1e-5 of the largest speed as in the other solver-form tests.
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -62,6 +64,85 @@ def test_persistent_matches_launches(nx, ny, solver):
         again, same = solve(hip, solver, 1e-8, False)
         assert again.iterations == rep.iterations
         assert np.array_equal(same, faces)
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 48), (512, 256), (40, 1400)])
+@pytest.mark.parametrize("solver", [msa.SOLVER_JACOBI_FP64, msa.SOLVER_MIXED])
+def test_a_persistent_launch_given_up_falls_back_to_launches(nx, ny, solver):
+    # No patience: every workgroup gives up at its first look in vain and exits,
+    # and the solve starts over by launches, to their bits. Then as before.
+    grid, mobility = system(nx, ny, 3)
+    with msa.HipBackend(0) as hip:
+        hip.flow_prepare(grid, mobility, 0)
+        limits = hip.resident_limits()
+        rep, faces = solve(hip, solver, 1e-8, False)
+        hip.set_resident_limits(workgroups=0)
+        ref, expected = solve(hip, solver, 1e-8, False)
+        hip.set_resident_limits(workgroups=limits["workgroups"], polls=0)
+        got, fell_back = solve(hip, solver, 1e-8, False)
+        assert got.iterations == ref.iterations
+        assert np.array_equal(fell_back, expected)
+        hip.set_resident_limits(polls=limits["polls"])
+        again, same = solve(hip, solver, 1e-8, False)
+        assert again.iterations == rep.iterations
+        assert np.array_equal(same, faces)
+
+
+def test_resident_limits_are_clamped_and_checked():
+    with msa.HipBackend(0) as hip:
+        most = hip.resident_limits()
+        assert most["workgroups"] > 0 and most["polls"] > 0
+        hip.set_resident_limits(workgroups=0xffffffff, polls=0xffffffff, round_tag=9)
+        hip.set_resident_limits(round_tag=3)
+        assert hip.resident_limits() == {**most, "round_tag": 9}
+        with pytest.raises(TypeError):
+            hip.set_resident_limits(blocks=1)
+
+
+@pytest.mark.parametrize("solver", [msa.SOLVER_JACOBI_FP64, msa.SOLVER_MIXED])
+def test_meetings_start_over_before_their_number_wraps(solver):
+    grid, mobility = system(131, 77, 1)
+    with msa.HipBackend(0) as hip:
+        hip.flow_prepare(grid, mobility, 0)
+        rep, faces = solve(hip, solver, 1e-8, False)
+        hip.set_resident_limits(round_tag=0xffffffff - 3 * 8192)
+        for _ in range(6):
+            again, same = solve(hip, solver, 1e-8, False)
+            assert again.iterations == rep.iterations
+            assert np.array_equal(same, faces)
+        assert hip.resident_limits()["round_tag"] < 0x80000000
+
+
+def test_two_contexts_solve_at_once():
+    # Each context has its own words: solves of different systems in two
+    # threads give what each gives alone.
+    cases = [(131, 77, msa.SOLVER_JACOBI_FP64), (512, 256, msa.SOLVER_MIXED)]
+    alone = []
+    for nx, ny, solver in cases:
+        grid, mobility = system(nx, ny, 2)
+        with msa.HipBackend(0) as hip:
+            hip.flow_prepare(grid, mobility, 0)
+            alone.append(solve(hip, solver, 1e-8, False))
+    out = [[], []]
+
+    def work(k):
+        nx, ny, solver = cases[k]
+        grid, mobility = system(nx, ny, 2)
+        with msa.HipBackend(0) as hip:
+            hip.flow_prepare(grid, mobility, 0)
+            for _ in range(8):
+                out[k].append(solve(hip, solver, 1e-8, False))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (rep, faces), results in zip(alone, out):
+        assert len(results) == 8
+        for again, same in results:
+            assert again.iterations == rep.iterations
+            assert np.array_equal(same, faces)
 
 
 def test_persistent_resumes_and_stops_at_its_budget():
