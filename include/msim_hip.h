@@ -159,6 +159,9 @@ typedef struct {
                           per compute unit, or 0 on a device without cooperative launches */
   uint32_t polls;      /* how often a workgroup looks again for the others' words (about a
                           microsecond each) before the launch is given up; 2^21 - 1 at creation */
+  uint32_t iterations; /* of one launch, at most (at least 1); 4096 at creation. A longer pressure
+                          solve goes on in further launches, a resolved solve one of whose
+                          momentum solves takes more by separate launches */
   uint32_t round_tag;  /* the number of the next meeting of the workgroups; counts up, and
                           starts over before 2^32. Setting it can only raise it */
 } msim_resident_limits;

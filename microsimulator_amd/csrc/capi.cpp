@@ -1230,6 +1230,7 @@ int msim_hip_create(int device, msim_ctx** out) {
       ctx->impl.resident_most.workgroups = static_cast<uint32_t>(prop.multiProcessorCount);
   }
   ctx->impl.resident_most.polls = msim::kRoundPolls;
+  ctx->impl.resident_most.iterations = msim::kPersistIterations;
   ctx->impl.resident = ctx->impl.resident_most;
   *out = ctx;
   return MSIM_OK;
@@ -1272,6 +1273,7 @@ int msim_hip_set_resident_limits(msim_ctx* ctx, const msim_resident_limits* limi
     if (limits == nullptr) msim::invalid("limits must not be null");
     c.resident.workgroups = std::min(limits->workgroups, c.resident_most.workgroups);
     c.resident.polls = std::min(limits->polls, c.resident_most.polls);
+    c.resident.iterations = std::clamp(limits->iterations, 1u, c.resident_most.iterations);
     c.resident.round_tag = std::max(limits->round_tag, c.resident.round_tag);
   });
 }

@@ -1139,11 +1139,10 @@ uint32_t run_cg(Context& ctx, Init&& init, T* r, T* x, T* q, T* pa, T* pb, uint3
   const ResidentShape shape =
       times == nullptr && !f.by_launches ? persist_shape<T>(ctx) : ResidentShape{};
   if (shape.per_thread != 0 && budget > 0) {
-    // Launches of kPersistIterations, so none runs for more than some tens of
-    // milliseconds; the direction stays in pa.
+    // The direction stays in pa from launch to launch.
     uint32_t taken = 0;
     while (taken < budget) {
-      const uint32_t batch = std::min(kPersistIterations, budget - taken);
+      const uint32_t batch = std::min(ctx.resident.iterations, budget - taken);
       if (!launch_persistent<T>(ctx, shape, r, x, pa, batch, taken)) break;
       read_state(ctx);
       if (f.host_state->failure == kRoundStalled) break;

@@ -416,6 +416,9 @@ void flow_hold_pressures(Context& ctx, const float* pressure_host);
 // msim_resident_limits::polls at creation: a look is a trip to memory of about a
 // microsecond, so some seconds.
 constexpr uint32_t kRoundPolls = (1u << 21) - 1;
+// msim_resident_limits::iterations at creation: tens of milliseconds of a
+// pressure solve, 0.12 s of a momentum solve on a million faces.
+constexpr uint32_t kPersistIterations = 4096;
 // The shape of a persistent solve over `entries` entries whose direction, with
 // `halo` entries either side, is held in LDS: 1 or 2 entries per thread while
 // that leaves at most 16 workgroups, else 4, else 8; none (per_thread 0) where

@@ -32,8 +32,6 @@ constexpr size_t kRoundSlots = 2ull * kRoundWords * kRoundBlocks;
 // always ends; the caller starts over without it. Looks and not a clock: a
 // preempted workgroup's clock runs on.
 constexpr uint32_t kRoundStalled = 6;  // CgState::failure of a launch given up that way
-// Iterations of one persistent launch (some tens of milliseconds).
-constexpr uint32_t kPersistIterations = 4096;
 
 __device__ inline void word_store(uint64_t* at, uint32_t tag, uint32_t bits) {
   __hip_atomic_store(at, (static_cast<uint64_t>(tag) << 32) | bits, __ATOMIC_RELAXED,

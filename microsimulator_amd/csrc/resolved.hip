@@ -658,7 +658,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
     st->relative = relative;
     st->stop1 = met || failure != 0 ? 1u : 0u;
     st->stop2 = 0;
-    st->failure1 = alive ? failure : MSIM_DEVICE_ERROR;
+    st->failure1 = alive ? failure : kRoundStalled;
     st->failure2 = 0;
   }
 }
@@ -1107,7 +1107,6 @@ void judge_momentum(ResDevice& D, const ResState& s, uint64_t& inner) {
       throw Error(MSIM_CG_BREAKDOWN, label + "encountered a preconditioner breakdown");
     case MSIM_CG_DIRECTION:
       throw Error(MSIM_CG_DIRECTION, label + "produced a non-finite direction");
-    case MSIM_DEVICE_ERROR: throw Error(MSIM_DEVICE_ERROR, label + "stalled");
     default: break;
   }
   if (s.stop1 == 0 && s.stop2 == 0) {
@@ -1116,19 +1115,24 @@ void judge_momentum(ResDevice& D, const ResState& s, uint64_t& inner) {
   }
 }
 
-// The preconditioner by one persistent launch, on grids that fit and up to
-// kMomentumLimit iterations (one launch takes them all: well under a second);
-// false where it is not taken.
-constexpr uint32_t kMomentumLimit = 1u << 16;
+// Whether a persistent momentum solve ended short of its answer: given up, or
+// at its launch's iterations and not the caller's.
+bool momentum_undone(const ResState& s, uint32_t max_iterations) {
+  return s.failure1 == kRoundStalled ||
+         (s.failure1 == 0 && s.stop1 == 0 && s.iterations < max_iterations);
+}
 
+// The preconditioner by one persistent launch, on grids that fit; false where
+// it is not taken.
 bool precondition_persistent(Context& ctx, ResDevice& D, const double* in, double* out,
                              float tolerance, uint32_t max_iterations, ResState* state) {
-  if (D.persist.per_thread == 0 || max_iterations == 0 || max_iterations > kMomentumLimit) return false;
-  uint32_t tag = take_rounds(ctx, 2 * max_iterations + 1, 2 * D.V.nf);
+  if (D.persist.per_thread == 0 || max_iterations == 0) return false;
+  uint32_t limit = std::min(max_iterations, ctx.resident.iterations);
+  uint32_t tag = take_rounds(ctx, 2 * limit + 1, 2 * D.V.nf);
   uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
   uint32_t polls = ctx.resident.polls;
   void* args[] = {&D.V, &in,    &out,            &words,          &slots,     &tag,
-                  &polls, &D.persist_halo, &max_iterations, &tolerance, &state};
+                  &polls, &D.persist_halo, &limit,          &tolerance,      &state};
   const void* kernel = nullptr;
   switch (D.persist.per_thread) {
     case 1: kernel = reinterpret_cast<const void*>(&k_cg_momentum<1>); break;
@@ -1213,7 +1217,7 @@ void apply_system(Context& ctx, ResDevice& D, const double* in, double* out) {
 }
 
 // The preconditioner; true where the momentum solve's state is still to be
-// judged once the device has it (judge_momentum).
+// judged once the device has it (momentum_undone, judge_momentum).
 bool precondition(Context& ctx, ResDevice& D, const double* in, double* out, float tolerance,
                   uint32_t max_iterations, ResState* state, uint64_t& inner) {
   if (precondition_persistent(ctx, D, in, out, tolerance, max_iterations, state)) return true;
@@ -1372,14 +1376,16 @@ BlockSolve block_solve(Context& ctx, ResDevice& D, const std::vector<double>& rh
               "read Arnoldi column");
         check(hipEventRecord(D.column_read[j & 1u], ctx.stream), "event");
       };
-      // Takes step j's column into the least-squares problem; true where the
-      // cycle ends with it.
+      // Takes step j's column into the least-squares problem; `ended`: the
+      // cycle ends with it. False where the step's momentum solve is undone.
+      bool ended = false;
       auto take = [&](uint32_t j, bool judge) {
         check(hipEventSynchronize(D.column_read[j & 1u]), "Arnoldi step");
         const double* col = D.host_columns + (j & 1u) * kColumnSlots;
         if (judge) {
           ResState state{};
           std::memcpy(&state, col + kColumn, sizeof(state));
+          if (momentum_undone(state, max_inner)) return false;
           judge_momentum(D, state, out.inner);
         }
         for (uint32_t i = 0; i <= j; ++i) {
@@ -1406,20 +1412,29 @@ BlockSolve block_solve(Context& ctx, ResDevice& D, const std::vector<double>& rh
         gv[j] *= cosine[j];
         ++iterations;
         used = j + 1;
-        return happy || std::abs(gv[j + 1]) <= tolerance * rhs_norm;
+        ended = happy || std::abs(gv[j + 1]) <= tolerance * rhs_norm;
+        return true;
+      };
+      // Step j again, and the rest of the solve, by launches.
+      auto redo = [&](uint32_t j) {
+        D.persist = ResidentShape{};
+        enqueue(j);
+        take(j, false);
       };
       // A step's column is read while the next step runs: where the cycle ends
       // with it, that step's vectors and counts are dropped (one of some 300
       // us; waiting for each column left the device idle 45 us a step).
       // Momentum solves whose state the host reads itself cannot run ahead.
-      bool ended = false;
       for (uint32_t j = 0; j < count && !ended; ++j) {
         const bool ahead = pending;
         enqueue(j);
-        if (ahead) ended = take(j - 1, true);
-        if (!ended && !pending) ended = take(j, false);
+        if (ahead && !take(j - 1, true)) {
+          redo(--j);
+          continue;
+        }
+        if (!ended && !pending) take(j, false);
       }
-      if (pending && !ended) take(count - 1, true);
+      if (pending && !ended && !take(count - 1, true)) redo(count - 1);
       std::vector<double> weights(used);
       for (uint32_t i = used; i-- > 0;) {
         double value = gv[i];

@@ -1,7 +1,7 @@
 """Jacobi-PCG as one persistent launch (small and medium systems) against the
 same iteration as two launches each: the pressure's, which a profiled solve
 takes by launches, and the resolved flow's momentum solves, which take launches
-where more than 65536 iterations are allowed.
+on a context that allows no resident workgroups.
 
 Both stop on the same test of the same recurrence and differ in the order of
 their FP64 sums only, so the iteration counts agree within the reference's own
@@ -145,6 +145,18 @@ def test_two_contexts_solve_at_once():
             assert np.array_equal(same, faces)
 
 
+def test_persistent_launches_of_few_iterations_go_on_to_the_same_bits():
+    grid, mobility = system(131, 77, 4)
+    with msa.HipBackend(0) as hip:
+        hip.flow_prepare(grid, mobility, 0)
+        rep, faces = solve(hip, msa.SOLVER_JACOBI_FP64, 1e-8, False)
+        for iterations in (1, 37):
+            hip.set_resident_limits(iterations=iterations)
+            again, same = solve(hip, msa.SOLVER_JACOBI_FP64, 1e-8, False)
+            assert again.iterations == rep.iterations
+            assert np.array_equal(same, faces)
+
+
 def test_persistent_resumes_and_stops_at_its_budget():
     # A long thin channel: more iterations than one launch takes (4096), each
     # solve resumed from the last launch's state; then a budget it cannot meet.
@@ -168,6 +180,55 @@ def test_persistent_resumes_and_stops_at_its_budget():
         assert rep2.iterations == rep.iterations and np.array_equal(faces2, faces)
 
 
+def resolved_system(dims):
+    rng = np.random.default_rng(sum(dims))
+    solid = (rng.random(dims) < 0.06).astype(np.uint8)
+    solid[0] = solid[-1] = 0
+    grid = msa.Grid(*dims, 1.0, 0.9, 1.1, solid.reshape(-1))
+    return grid, (rng.random(dims) * 2.0).astype(np.float32).reshape(-1)
+
+
+def resolved(hip, grid, drag, tolerance, most=50_000):
+    field, rep = hip.solve_resolved_flow(grid, drag, msa.ResolvedFlowParameters(
+        mean_inlet_speed=1.0, axis=0, relative_tolerance=tolerance, max_outer_iterations=4000,
+        max_inner_iterations=most))
+    return field.concatenated(), rep
+
+
+# Given up at the first look in vain; at the launch's iterations, from the first
+# momentum solve on (3) or a later one (between the shortest and the longest).
+@pytest.mark.parametrize("limit", [dict(polls=0), dict(iterations=3), dict(iterations=None)])
+@pytest.mark.parametrize("dims", [(12, 9, 7), (7, 40, 30), (40, 20, 18)])
+def test_a_momentum_launch_left_undone_falls_back_to_launches(dims, limit):
+    grid, drag = resolved_system(dims)
+    with msa.HipBackend(0) as hip:
+        limits = hip.resident_limits()
+        faces, rep = resolved(hip, grid, drag, 1e-6)
+        hip.set_resident_limits(workgroups=0)
+        expected, ref = resolved(hip, grid, drag, 1e-6)
+        hip.set_resident_limits(workgroups=limits["workgroups"])
+        mean = rep.inner_iterations // rep.outer_iterations
+        limit = {k: mean if v is None else v for k, v in limit.items()}
+        hip.set_resident_limits(**limit)
+        got, again = resolved(hip, grid, drag, 1e-6)
+        # Steps before the one redone were the persistent form's.
+        assert abs(again.outer_iterations - ref.outer_iterations) <= 1
+        if "polls" in limit or limit["iterations"] == 3:
+            assert again.inner_iterations == ref.inner_iterations
+            assert np.array_equal(got, expected)
+        else:
+            assert np.abs(got - expected).max() <= 3e-5 * np.abs(expected).max()
+        # The caller's own limit on the iterations is what is refused, in either
+        # form, also where it is past the launch's.
+        for most in (2, 5):
+            with pytest.raises(msa.NotConverged, match="momentum conjugate gradient did not"):
+                resolved(hip, grid, drag, 1e-6, most)
+        hip.set_resident_limits(**limits)
+        same, once = resolved(hip, grid, drag, 1e-6)
+        assert once.inner_iterations == rep.inner_iterations
+        assert np.array_equal(same, faces)
+
+
 # Faces per workgroup are 512, 1024, 2048 or 4096 by the count; the halo is a
 # plane of the lattice either side, here also more than a workgroup's faces.
 @pytest.mark.parametrize("dims,tolerance", [
@@ -175,18 +236,12 @@ def test_persistent_resumes_and_stops_at_its_budget():
     ((7, 40, 30), 1e-6), ((40, 20, 18), 1e-5), ((3, 60, 61), 1e-6), ((72, 50, 49), 1e-2),
 ])
 def test_momentum_persistent_matches_launches(dims, tolerance):
-    rng = np.random.default_rng(sum(dims))
-    solid = (rng.random(dims) < 0.06).astype(np.uint8)
-    solid[0] = solid[-1] = 0
-    grid = msa.Grid(*dims, 1.0, 0.9, 1.1, solid.reshape(-1))
-    drag = (rng.random(dims) * 2.0).astype(np.float32).reshape(-1)
+    grid, drag = resolved_system(dims)
     out = []
     with msa.HipBackend(0) as hip:
-        for most in (50_000, 100_000):
-            field, rep = hip.solve_resolved_flow(grid, drag, msa.ResolvedFlowParameters(
-                mean_inlet_speed=1.0, axis=0, relative_tolerance=tolerance,
-                max_outer_iterations=4000, max_inner_iterations=most))
-            out.append((field.concatenated(), rep))
+        for workgroups in (hip.resident_limits()["workgroups"], 0):
+            hip.set_resident_limits(workgroups=workgroups)
+            out.append(resolved(hip, grid, drag, tolerance))
     (faces, rep), (expected, ref) = out
     # The same FP64 recurrences with their sums in another order: an inner
     # solve may stop one iteration apart, an outer cycle one step.
