@@ -162,6 +162,8 @@ typedef struct {
   uint32_t iterations; /* of one launch, at most (at least 1); 4096 at creation. A longer pressure
                           solve goes on in further launches, a resolved solve one of whose
                           momentum solves takes more by separate launches */
+  uint32_t lds_bytes;  /* of one workgroup, at most: the device's at creation. Also of the
+                          multilevel cycle's single workgroup, from the next preparation on */
   uint32_t round_tag;  /* the number of the next meeting of the workgroups; counts up, and
                           starts over before 2^32. Setting it can only raise it */
 } msim_resident_limits;

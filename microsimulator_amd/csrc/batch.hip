@@ -1308,10 +1308,11 @@ constexpr uint32_t kFlowBodies = 4;  // bodies between two looks at the finished
 // takes some 45 us of launches and dependent reads, and the sites of all. In us
 // per iteration, alone and together: 1 x 64x64 31 and 46, 1 x 96x80 52 and 54,
 // 1 x 128x96 67 and 58, 64 x 128x96 78 and 81, 256 x 128x96 92 and 144,
-// 64 x 256x128 187 and 121, 256 x 256x128 291 and 328, 64 x 512x256 903 and 344.
+// 64 x 256x128 187 and 121, 256 x 256x128 291 and 328, 64 x 512x256 903 and 344
+// (256 compute units).
 constexpr uint64_t kAloneSites = 8192;
-bool solve_alone(uint64_t sites, uint64_t largest) {
-  return largest <= kAloneSites || 256 * sites >= largest * largest;
+bool solve_alone(uint64_t units, uint64_t sites, uint64_t largest) {
+  return largest <= kAloneSites || units * sites >= largest * largest;
 }
 
 }  // namespace
@@ -1521,7 +1522,7 @@ void plan_flow(Context& ctx, BatchDevice& B) {
   B.flow_down.clear();
   B.flow_up.clear();
   const BatchDesc& largest = B.desc[B.order[0]];
-  if (solve_alone(B.sites, static_cast<uint64_t>(largest.nx) * largest.ny)) return;
+  if (solve_alone(ctx.compute_units, B.sites, static_cast<uint64_t>(largest.nx) * largest.ny)) return;
   std::vector<FlowSpan> span(B.count);
   std::vector<std::vector<FlowTile>> down, up;
   auto cut = [](std::vector<FlowTile>& to, uint32_t inst, uint32_t cells, uint32_t tile) {

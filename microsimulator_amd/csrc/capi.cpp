@@ -1226,8 +1226,10 @@ int msim_hip_create(int device, msim_ctx** out) {
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
     ctx->impl.name = prop.name;
     if (ctx->impl.name.empty()) ctx->impl.name = prop.gcnArchName;
+    ctx->impl.compute_units = static_cast<uint32_t>(prop.multiProcessorCount);
+    ctx->impl.resident_most.lds_bytes = static_cast<uint32_t>(prop.sharedMemPerBlock);
     if (prop.cooperativeLaunch != 0)
-      ctx->impl.resident_most.workgroups = static_cast<uint32_t>(prop.multiProcessorCount);
+      ctx->impl.resident_most.workgroups = ctx->impl.compute_units;
   }
   ctx->impl.resident_most.polls = msim::kRoundPolls;
   ctx->impl.resident_most.iterations = msim::kPersistIterations;
@@ -1274,6 +1276,7 @@ int msim_hip_set_resident_limits(msim_ctx* ctx, const msim_resident_limits* limi
     c.resident.workgroups = std::min(limits->workgroups, c.resident_most.workgroups);
     c.resident.polls = std::min(limits->polls, c.resident_most.polls);
     c.resident.iterations = std::clamp(limits->iterations, 1u, c.resident_most.iterations);
+    c.resident.lds_bytes = std::min(limits->lds_bytes, c.resident_most.lds_bytes);
     c.resident.round_tag = std::max(limits->round_tag, c.resident.round_tag);
   });
 }

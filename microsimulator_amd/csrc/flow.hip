@@ -899,7 +899,8 @@ ResidentShape resident_shape(const Context& ctx, size_t entries, size_t halo, si
     const size_t chunk = static_cast<size_t>(kPersistThreads) * s;
     const size_t blocks = (entries + chunk - 1) / chunk;
     const size_t lds = (std::min(chunk, entries) + 2 * halo) * bytes;
-    if (blocks <= (s < 4 ? std::min<size_t>(room, 16) : room) && lds <= lds_limit)
+    if (blocks <= (s < 4 ? std::min<size_t>(room, 16) : room) && lds <= lds_limit &&
+        lds + sizeof(RoundLds) <= ctx.resident.lds_bytes)
       return ResidentShape{s, static_cast<uint32_t>(blocks), lds};
   }
   return ResidentShape{};

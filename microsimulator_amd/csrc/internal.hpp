@@ -387,6 +387,7 @@ struct Context {
   // words, and what they may take of the device and what it has.
   DeviceBuffer<uint64_t> round_slots, round_words;
   msim_resident_limits resident{}, resident_most{};
+  uint32_t compute_units = 0;
 };
 
 // Summed event time and launch count of the two Krylov kernels of a solve.

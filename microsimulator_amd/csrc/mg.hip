@@ -48,13 +48,16 @@ constexpr int kTailThreads = 1024;
 constexpr uint32_t kCoarseCells = 256;  // densely inverted
 // The single-workgroup kernel takes the levels from the first of at most
 // kTailCells cells, kTailQuads aggregates per thread (a grid of one row has
-// more aggregates than a quarter of its cells) and kTailFloats of LDS. From
+// more aggregates than a quarter of its cells) and kTailFloats of LDS, or what
+// the device has (64 KB: a level later from 4096 cells). From
 // 8192 cells (two aggregates per thread) it took 27.6 us, 16.3 more, ten of
 // them to load 200 KB into one compute unit, for two launches of the tile
 // kernels saved (12 us).
 constexpr uint32_t kTailCells = 4096;
 constexpr int kTailQuads = 1;
 constexpr uint64_t kTailFloats = 38 * 1024;
+constexpr uint64_t kTailFixed =  // s_red and s_part
+    kTailThreads / kWave * sizeof(double) + kTailThreads * sizeof(float);
 constexpr uint32_t kMaxLevels = 24;
 static_assert(4 * kCoarseCells <= kTailThreads, "the coarsest solve splits every row in parts");
 constexpr float kOmega = 0.8f;
@@ -1316,12 +1319,15 @@ void mg_prepare(Context& ctx) {
     mg.levels.push_back(std::move(C));
   }
   // The single-workgroup kernel takes every level from the first small one.
+  const uint64_t lds = ctx.resident.lds_bytes;
+  const uint64_t most =
+      std::min(kTailFloats, lds > kTailFixed ? (lds - kTailFixed) / sizeof(float) : 0);
   mg.tail = static_cast<uint32_t>(mg.levels.size()) - 1;
   for (uint32_t l = 0; l < mg.levels.size(); ++l) {
     const MgLevel& L = *mg.levels[l];
     const uint64_t quads = static_cast<uint64_t>((L.nx + 1) / 2) * ((L.ny + 1) / 2);
     if (L.cells() <= kTailCells && quads <= kTailQuads * kTailThreads &&
-        tail_floats(mg, l) <= kTailFloats) {
+        tail_floats(mg, l) <= most) {
       mg.tail = l;
       break;
     }

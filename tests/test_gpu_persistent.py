@@ -88,6 +88,20 @@ def test_a_persistent_launch_given_up_falls_back_to_launches(nx, ny, solver):
         assert np.array_equal(same, faces)
 
 
+@pytest.mark.parametrize("solver", [msa.SOLVER_JACOBI_FP64, msa.SOLVER_MIXED])
+def test_a_device_with_less_lds_takes_launches(solver):
+    # 512x256 FP64 sites: 2048 own and 2 x 256 beside them, 20.5 KB.
+    grid, mobility = system(512, 256, 3)
+    with msa.HipBackend(0) as hip:
+        hip.flow_prepare(grid, mobility, 0)
+        hip.set_resident_limits(workgroups=0)
+        ref, expected = solve(hip, solver, 1e-8, False)
+        hip.set_resident_limits(workgroups=256, lds_bytes=8192)
+        got, faces = solve(hip, solver, 1e-8, False)
+        assert got.iterations == ref.iterations
+        assert np.array_equal(faces, expected)
+
+
 def test_resident_limits_are_clamped_and_checked():
     with msa.HipBackend(0) as hip:
         most = hip.resident_limits()
