@@ -725,7 +725,9 @@ __global__ __launch_bounds__(NT) void k_batch_flow(BatchData D, BatchParams P) {
     if (rr64 <= threshold || ref == kRefinements || it >= P.max_iterations) break;
     double rr = rr64, rz_old = 0.0;
     const double inner = kInner * kInner * rr64;
-    for (uint32_t k = 0; rr > inner && it < P.max_iterations; ++k, ++it) {
+    // The first is taken also where the residual is not finite: its product
+    // then is not either, and the instance is flagged.
+    for (uint32_t k = 0; (k == 0 || rr > inner) && it < P.max_iterations; ++k, ++it) {
       float* p = (k & 1u) != 0 ? D.p2 + I.site : D.p + I.site;
       float* pn = (k & 1u) != 0 ? D.p + I.site : D.p2 + I.site;
       double rz[1] = {batch_cycle<NT>(D, V, I.site, 0)};

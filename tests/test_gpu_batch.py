@@ -210,3 +210,24 @@ def test_batch_rejects_bad_instances(hip):
         hip.batch_upload(inst)
     with pytest.raises(msa.InvalidArgument):
         hip.batch_upload(inst[:1], relative_tolerance=0.0)
+
+
+@pytest.mark.parametrize("shape", [(16, 12), (128, 96)])  # one workgroup; the whole chip
+def test_a_solve_without_a_finite_residual_is_flagged(hip, shape):
+    """A conductance past the largest float leaves no finite residual: the
+    instance is flagged as broken down, and its neighbour solves as ever.
+    (The one-workgroup form ended without a flag.)"""
+    nx, ny = shape
+    mobility = np.ones((nx, ny), np.float32)
+    wild = mobility.copy()
+    wild[nx // 2:] = 3.0e38
+
+    def instance(m):
+        return msa.BatchInstance(nx=nx, ny=ny, mobility=m, inlet_pressure=1.0, reservoir=1.0,
+                                 diffusion=1.0, dx=1.0, dy=1.0, dz=10.0)
+
+    hip.batch_upload([instance(wild), instance(mobility)], relative_tolerance=1e-8,
+                     max_iterations=2000)
+    it, res, flags = hip.batch_solve_flow()
+    assert flags[0] & 1
+    assert flags[1] == 0 and res[1] <= 1e-8 and it[1] > 0
