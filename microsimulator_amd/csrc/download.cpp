@@ -8,8 +8,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -25,16 +25,16 @@ constexpr size_t kMostThreads = 8;
 constexpr size_t kThreadedBytes = size_t(4) << 20;
 
 // The process's pinned slots: handed out to one download at a time, kept for
-// the next, freed with the last context.
+// the next, freed with the last context. Held in place, so that handing them
+// out and back cannot fail.
 class SlotPool {
  public:
-  std::vector<void*> take(size_t wanted) {
+  size_t take(void** out, size_t wanted) {
     std::lock_guard<std::mutex> hold(lock_);
-    std::vector<void*> out;
-    while (out.size() < wanted) {
-      if (!free_.empty()) {
-        out.push_back(free_.back());
-        free_.pop_back();
+    size_t n = 0;
+    while (n < wanted) {
+      if (kept_ > 0) {
+        out[n++] = free_[--kept_];
         continue;
       }
       if (made_ == kMostSlots) break;
@@ -44,13 +44,13 @@ class SlotPool {
         break;
       }
       ++made_;
-      out.push_back(ptr);
+      out[n++] = ptr;
     }
-    return out;
+    return n;
   }
-  void give(const std::vector<void*>& slots) {
+  void give(void* const* slots, size_t count) {
     std::lock_guard<std::mutex> hold(lock_);
-    free_.insert(free_.end(), slots.begin(), slots.end());
+    for (size_t k = 0; k < count; ++k) free_[kept_++] = slots[k];
     if (users_ == 0) release();
   }
   void enter() {
@@ -64,13 +64,12 @@ class SlotPool {
 
  private:
   void release() {
-    for (void* p : free_) static_cast<void>(hipHostFree(p));
-    made_ -= free_.size();
-    free_.clear();
+    made_ -= kept_;
+    while (kept_ > 0) static_cast<void>(hipHostFree(free_[--kept_]));
   }
   std::mutex lock_;
-  std::vector<void*> free_;
-  size_t made_ = 0, users_ = 0;
+  void* free_[kMostSlots] = {};
+  size_t kept_ = 0, made_ = 0, users_ = 0;
 };
 
 SlotPool g_slots;
@@ -99,13 +98,17 @@ void download(Context& ctx, void* dst, const void* src, size_t bytes, const char
   if (bytes < kThreadedBytes || registered(dst)) return plain();
   const size_t chunks = (bytes + kSlotBytes - 1) / kSlotBytes;
   const size_t cores = std::max<size_t>(std::thread::hardware_concurrency(), 1);
-  const std::vector<void*> slots = g_slots.take(std::min({kMostThreads, cores, chunks}));
-  if (slots.size() < 2) {
-    g_slots.give(slots);
+  std::vector<std::thread> threads;
+  threads.reserve(kMostThreads);
+  void* slots[kMostThreads];
+  const size_t count = g_slots.take(slots, std::min({kMostThreads, cores, chunks}));
+  if (count < 2) {
+    g_slots.give(slots, count);
     return plain();
   }
   // Every chunk is taken by exactly one thread; whatever fails, all are joined
-  // and the slots go back only after the stream has drained.
+  // and the slots go back only after the stream has drained. Nothing from here
+  // to there throws.
   std::atomic<size_t> next{0};
   std::atomic<int> failed{hipSuccess};
   auto work = [&](void* slot) {
@@ -128,17 +131,16 @@ void download(Context& ctx, void* dst, const void* src, size_t bytes, const char
       failed.compare_exchange_strong(none, e);
     }
   };
-  std::vector<std::thread> threads;
-  threads.reserve(slots.size());
   try {
-    for (size_t k = 1; k < slots.size(); ++k) threads.emplace_back(work, slots[k]);
-  } catch (const std::system_error&) {
-    // Fewer threads then: the others take every chunk.
+    for (size_t k = 1; k < count; ++k) threads.emplace_back(work, slots[k]);
+  } catch (const std::exception&) {
+    // Fewer threads then (no more of them, or no memory): the others take every
+    // chunk.
   }
   work(slots[0]);
   for (auto& t : threads) t.join();
   const hipError_t drained = hipStreamSynchronize(ctx.stream);
-  g_slots.give(slots);
+  g_slots.give(slots, count);
   check(static_cast<hipError_t>(failed.load()), what);
   check(drained, what);
 }

@@ -25,7 +25,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("what", ["registered"])
+@pytest.mark.parametrize("what", ["registered", "allocations"])
 def test_download(program, what):
     done = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     assert done.returncode == 0, done.stdout + done.stderr
