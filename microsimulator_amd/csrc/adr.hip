@@ -965,11 +965,11 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 void* g_scratch[kStaticDevices] = {};
 std::mutex g_scratch_lock[kStaticDevices];
 
-// Blocks whose partials the scratch holds room for: strips of 62, 126 or 254
-// columns (60, 124 or 252 under van Leer; whichever takes the fewest threads)
+// The scratch holds 49 doubles for each of these blocks: strips of 62, 126 or
+// 254 columns (60, 124 or 252 under van Leer; whichever takes the fewest threads)
 // by 16 x-rows, or fewer down to 4 for 2048 blocks. A formula of its own, so
 // that the grids that fit the scratch stay the same whatever shape a step is
-// launched in.
+// launched in (of which it needs one double a block).
 uint32_t static_blocks(const AdrParams& P) {
   uint64_t best = ~0ull, strips = 1;
   for (uint32_t threads : {256u, 128u, 64u}) {
@@ -1043,18 +1043,16 @@ void adr_step_static(Context& ctx, const msim_signal_grid& grid, float dt, float
   AdrParams P = transport_params(grid);
   const uint32_t S = P.signals;
   const size_t n = static_cast<size_t>(P.nx) * P.ny;
-  AdrShape sh = adr_shape(P.nx, P.ny, P.limited != 0);
-  // Longer walks where the shape has more blocks than that.
-  const uint32_t room = static_blocks(P);
-  while (sh.blocks > room && sh.rows < P.nx) sh = adr_shape(sh.strips, P.nx, sh.rows + 4);
+  const AdrShape sh = adr_shape(P.nx, P.ny, P.limited != 0);
   const uint32_t survey_blocks = std::min<uint32_t>(site_blocks(n), 2048);
   ScratchLayout at;
   const size_t o_state = at.take(sizeof(CgState));
   const size_t o_flags = at.take(3 * sizeof(uint32_t));
   const size_t o_mass = at.take(kMaxSignals * sizeof(double));
   const size_t o_parts = at.take(
-      std::max<size_t>(static_cast<size_t>(3 * kMaxSignals * 2 + 1) * std::max(room, sh.blocks),
-                       static_cast<size_t>(kMaxSignals + 1) * survey_blocks) *
+      std::max({static_cast<size_t>(3 * kMaxSignals * 2 + 1) * static_blocks(P),
+                static_cast<size_t>(kMaxSignals + 1) * survey_blocks,
+                static_cast<size_t>(sh.blocks)}) *
       sizeof(double));
   const size_t o_solid = at.take(n);
   const size_t nxf = static_cast<size_t>(P.nx + 1) * P.ny, nyf = static_cast<size_t>(P.nx) * (P.ny + 1);
@@ -1137,8 +1135,9 @@ void adr_step_static(Context& ctx, const msim_signal_grid& grid, float dt, float
                           dt);
   if (dt == 0.0f) return;
   const AdrView v{&P, solid, phi, source, loss, flags};
-  LedgerParts L{parts, nullptr, sh.blocks};
-  double* largest = parts + static_cast<size_t>(3 * kMaxSignals * 2) * sh.blocks;
+  // FP32 levels keep no ledger: the block maxima are all the step leaves.
+  LedgerParts L{nullptr, nullptr, sh.blocks};
+  double* largest = parts;
   switch (S) {
     case 1: launch_static_step<1>(stream, v, sh, xf, yf, lv_a, lv_b, dt, L, largest); break;
     case 2: launch_static_step<2>(stream, v, sh, xf, yf, lv_a, lv_b, dt, L, largest); break;

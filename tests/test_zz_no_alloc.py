@@ -86,3 +86,44 @@ def test_static_step_limits(hip):
     small.integration = msa.CRANK_NICOLSON
     with pytest.raises(msa.Unsupported):
         hip.advance_signal_grid_static(small, levels, 0.1)
+
+
+def _scratch(nx, ny, S, scheme):
+    """Bytes a field-less step over nx x ny sites takes of the scratch array:
+    strips of at most 254 columns (252 under van Leer) by 16 x-rows (or fewer,
+    down to 4, for 2048 blocks), 49 doubles a block, and the staged mask and
+    levels."""
+    halo = 4 if scheme == msa.VAN_LEER else 2
+    strips = min((-(-ny // (t - halo)) * t, -(-ny // (t - halo))) for t in (256, 128, 64))[1]
+    rows = 16
+    while rows > 4 and strips * -(-nx // rows) < 2048:
+        rows //= 2
+    blocks = max(strips * -(-nx // rows), 24)
+    survey = min(-(-nx * ny // 256), 2048)
+    regions = [176, 12, 64, 8 * max(49 * blocks, 9 * survey), nx * ny, 4 * S * nx * ny,
+               4 * S * nx * ny]
+    return sum(-(-r // 256) * 256 for r in regions)
+
+
+@pytest.mark.parametrize("nx,scheme", [(1, msa.UPWIND), (3, msa.VAN_LEER), (4, msa.UPWIND),
+                                       (5, msa.VAN_LEER), (40, msa.UPWIND)])
+def test_static_step_takes_what_the_scratch_array_holds(hip, nx, scheme):
+    """The widest grid that fits is taken, one column more refused, also where a
+    grid has more walks than the blocks the array has partials for."""
+    limit = hip.lib.msim_hip_static_scratch_bytes()
+    lo, hi = 1, limit // nx
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if _scratch(nx, mid, 1, scheme) <= limit else (lo, mid)
+
+    def step(ny, entry):
+        levels = np.random.default_rng(ny).random(nx * ny).astype(np.float32)
+        spec = msa.SignalGridSpec(msa.Grid(nx, ny, 1, 1.0, 1.0, 1.0, None, KINDS),
+                                  np.ones(1, np.float32), np.zeros(6, np.float32),
+                                  advection_scheme=scheme)
+        return entry(spec, levels, 0.1)[0]
+
+    assert np.array_equal(step(lo, hip.advance_signal_grid_static),
+                          step(lo, hip.advance_signal_grid))
+    with pytest.raises(msa.InvalidArgument, match="bytes of device scratch"):
+        step(lo + 1, hip.advance_signal_grid_static)
