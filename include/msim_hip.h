@@ -157,11 +157,10 @@ int msim_hip_device_name(msim_ctx* ctx, char* name, size_t length);
 typedef struct {
   uint32_t workgroups; /* of one launch, at most; 0: no persistent launches. At creation one
                           per compute unit, or 0 on a device without cooperative launches */
-  uint32_t polls;      /* how often a workgroup looks again for the others' words (about a
-                          microsecond each) before the launch is given up; 2^21 - 1 at creation */
-  uint32_t iterations; /* of one launch, at most (at least 1); 4096 at creation. A longer pressure
-                          solve goes on in further launches, a resolved solve one of whose
-                          momentum solves takes more by separate launches */
+  uint32_t iterations; /* of one launch, at most; 4096 at creation. A longer pressure solve goes
+                          on in further launches, a resolved solve one of whose momentum solves
+                          takes more by separate launches. 0: every persistent launch ends
+                          without an iteration, as one that waited too long does */
   uint32_t lds_bytes;  /* of one workgroup, at most: the device's at creation. Also of the
                           multilevel cycle's single workgroup, from the next preparation on */
   uint32_t round_tag;  /* the number of the next meeting of the workgroups; counts up, and

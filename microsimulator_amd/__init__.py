@@ -112,8 +112,8 @@ class _NutrientStep(C.Structure):
 
 
 class _ResidentLimits(C.Structure):
-    _fields_ = [("workgroups", C.c_uint32), ("polls", C.c_uint32), ("iterations", C.c_uint32),
-                ("lds_bytes", C.c_uint32), ("round_tag", C.c_uint32)]
+    _fields_ = [("workgroups", C.c_uint32), ("iterations", C.c_uint32), ("lds_bytes", C.c_uint32),
+                ("round_tag", C.c_uint32)]
 
 
 class _FlowReport(C.Structure):

@@ -1231,7 +1231,6 @@ int msim_hip_create(int device, msim_ctx** out) {
     if (prop.cooperativeLaunch != 0)
       ctx->impl.resident_most.workgroups = ctx->impl.compute_units;
   }
-  ctx->impl.resident_most.polls = msim::kRoundPolls;
   ctx->impl.resident_most.iterations = msim::kPersistIterations;
   ctx->impl.resident = ctx->impl.resident_most;
   *out = ctx;
@@ -1274,8 +1273,7 @@ int msim_hip_set_resident_limits(msim_ctx* ctx, const msim_resident_limits* limi
   return msim::guarded(ctx, [&](Context& c) {
     if (limits == nullptr) msim::invalid("limits must not be null");
     c.resident.workgroups = std::min(limits->workgroups, c.resident_most.workgroups);
-    c.resident.polls = std::min(limits->polls, c.resident_most.polls);
-    c.resident.iterations = std::clamp(limits->iterations, 1u, c.resident_most.iterations);
+    c.resident.iterations = std::min(limits->iterations, c.resident_most.iterations);
     c.resident.lds_bytes = std::min(limits->lds_bytes, c.resident_most.lds_bytes);
     c.resident.round_tag = std::max(limits->round_tag, c.resident.round_tag);
   });

@@ -447,7 +447,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
     T* __restrict__ r, T* __restrict__ xsol, T* __restrict__ p, uint64_t* words,
     const float* __restrict__ diag, const float* __restrict__ cxl, const float* __restrict__ cyl,
     const float* __restrict__ bc, uint32_t n, uint32_t ny, T isx, T isy, CgState* st,
-    uint64_t* slots, uint32_t tag, uint32_t polls, uint32_t budget, uint32_t taken) {
+    uint64_t* slots, uint32_t tag, uint32_t budget, uint32_t taken) {
   constexpr int NT = kPersistThreads;
   constexpr int kAhead = 2;  // halo values polled for with the sums, per thread
   extern __shared__ __align__(16) unsigned char s_raw[];
@@ -530,9 +530,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
         z = z_of(i);
       } else {
         uint64_t w[Exchange<T>::kWords];
-        if (round_stalled(L)) break;
         poll_words(
-            L, polls, [&] { ex.load(i, w); }, [&] { return Exchange<T>::has(w, tag - 1); });
+            L, [&] { ex.load(i, w); }, [&] { return Exchange<T>::has(w, tag - 1); });
         z = Exchange<T>::value(w);
       }
       s_p[halo_slot(h)] = z + beta * s_p[halo_slot(h)];
@@ -556,7 +555,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
       }
     }
     alive = round_sums<1>(
-        pq, slots, tag++, polls, L, [] {}, [] { return true; });
+        pq, slots, tag++, L, [] {}, [] { return true; });
     if (!alive) break;
     curvature = pq[0];
     if (!isfinite(curvature) || curvature <= 0.0) {
@@ -584,7 +583,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persistent(
     }
     uint64_t w[kAhead][Exchange<T>::kWords];
     alive = round_sums<2>(
-        sums, slots, tag, polls, L,
+        sums, slots, tag, L,
         [&] {
 #pragma unroll
           for (int u = 0; u < kAhead; ++u) {
@@ -1083,9 +1082,8 @@ bool launch_persistent(Context& ctx, const ResidentShape& shape, T* r, T* x, T* 
   CgState* st = f.state.data();
   uint32_t tag = take_rounds(ctx, 2 * budget, Exchange<T>::kWords * f.sites());
   uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
-  uint32_t polls = ctx.resident.polls;
   void* args[] = {&r, &x, &p, &words, &diag, &cxl, &cyl, &bc, &n, &ny, &isx, &isy,
-                  &st, &slots, &tag, &polls, &budget, &taken};
+                  &st, &slots, &tag, &budget, &taken};
   const void* kernel = nullptr;
   switch (shape.per_thread) {
     case 1: kernel = reinterpret_cast<const void*>(&k_cg_persistent<T, 1>); break;
@@ -1146,7 +1144,7 @@ uint32_t run_cg(Context& ctx, Init&& init, T* r, T* x, T* q, T* pa, T* pb, uint3
       const uint32_t batch = std::min(ctx.resident.iterations, budget - taken);
       if (!launch_persistent<T>(ctx, shape, r, x, pa, batch, taken)) break;
       read_state(ctx);
-      if (f.host_state->failure == kRoundStalled) break;
+      if (f.host_state->failure == kRoundStalled || batch == 0) break;
       if (judge(*f.host_state)) return f.host_state->halt;
       taken += batch;
     }

@@ -414,9 +414,6 @@ void launch_assembly(hipStream_t stream, const uint8_t* solid, const float* mobi
 // A ported system: holds each open face at the pressure of its slot in
 // `pressure_host` (FlowEdges layout) and reassembles the right-hand side.
 void flow_hold_pressures(Context& ctx, const float* pressure_host);
-// msim_resident_limits::polls at creation: a look is a trip to memory of about a
-// microsecond, so some seconds.
-constexpr uint32_t kRoundPolls = (1u << 21) - 1;
 // msim_resident_limits::iterations at creation: tens of milliseconds of a
 // pressure solve, 0.12 s of a momentum solve on a million faces.
 constexpr uint32_t kPersistIterations = 4096;

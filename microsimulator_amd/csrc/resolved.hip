@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_step(ResView V, double* __rest
 template <int S>
 __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
     ResView V, const double* __restrict__ in, double* __restrict__ out, uint64_t* words,
-    uint64_t* slots, uint32_t tag, uint32_t polls, uint32_t halo, uint32_t limit, float tolerance,
+    uint64_t* slots, uint32_t tag, uint32_t halo, uint32_t limit, float tolerance,
     ResState* st) {
   constexpr int NT = kPersistThreads;
   constexpr int kAhead = 3;
@@ -551,7 +551,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
     }
   };
   aim(t);
-  bool alive = round_sums<2>(sums, slots, tag, polls, L, issue, [&] { return done(tag); });
+  bool alive = round_sums<2>(sums, slots, tag, L, issue, [&] { return done(tag); });
   double rho = sums[1];
   const double rhs_norm = sqrt(sums[0]);
   double beta = 0.0, relative = 1.0;
@@ -565,9 +565,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
     }
     advance(t, beta);
     for (uint32_t h0 = t + kAhead * NT; h0 < 2 * halo; h0 += kAhead * NT) {
-      if (round_stalled(L)) break;
       aim(h0);
-      poll_words(L, polls, issue, [&] { return done(tag); });
+      poll_words(L, issue, [&] { return done(tag); });
       advance(h0, beta);
     }
     aim(t);
@@ -603,7 +602,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
       }
     }
     alive = round_sums<1>(
-        pq, slots, tag++, polls, L, [] {}, [] { return true; });
+        pq, slots, tag++, L, [] {}, [] { return true; });
     if (!alive) break;
     if (!isfinite(pq[0]) || pq[0] <= 0.0) {
       failure = MSIM_CG_CURVATURE;
@@ -627,7 +626,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_momentum(
         sums[1] += rv[s] * zv[s];
       }
     }
-    alive = round_sums<2>(sums, slots, tag, polls, L, issue, [&] { return done(tag); });
+    alive = round_sums<2>(sums, slots, tag, L, issue, [&] { return done(tag); });
     if (!alive) break;
     ++k;
     const double now = sqrt(sums[0] > 0.0 ? sums[0] : 0.0) / rhs_norm;
@@ -1130,9 +1129,8 @@ bool precondition_persistent(Context& ctx, ResDevice& D, const double* in, doubl
   uint32_t limit = std::min(max_iterations, ctx.resident.iterations);
   uint32_t tag = take_rounds(ctx, 2 * limit + 1, 2 * D.V.nf);
   uint64_t *slots = ctx.round_slots.data(), *words = ctx.round_words.data();
-  uint32_t polls = ctx.resident.polls;
   void* args[] = {&D.V, &in,    &out,            &words,          &slots,     &tag,
-                  &polls, &D.persist_halo, &limit,          &tolerance,      &state};
+                  &D.persist_halo, &limit,          &tolerance,      &state};
   const void* kernel = nullptr;
   switch (D.persist.per_thread) {
     case 1: kernel = reinterpret_cast<const void*>(&k_cg_momentum<1>); break;

@@ -69,8 +69,8 @@ def test_persistent_matches_launches(nx, ny, solver):
 @pytest.mark.parametrize("nx,ny", [(64, 48), (512, 256), (40, 1400)])
 @pytest.mark.parametrize("solver", [msa.SOLVER_JACOBI_FP64, msa.SOLVER_MIXED])
 def test_a_persistent_launch_given_up_falls_back_to_launches(nx, ny, solver):
-    # No patience: every workgroup gives up at its first look in vain and exits,
-    # and the solve starts over by launches, to their bits. Then as before.
+    # A launch that ends without an iteration, as one given up does: the solve
+    # starts over by launches, to their bits. Then as before.
     grid, mobility = system(nx, ny, 3)
     with msa.HipBackend(0) as hip:
         hip.flow_prepare(grid, mobility, 0)
@@ -78,11 +78,11 @@ def test_a_persistent_launch_given_up_falls_back_to_launches(nx, ny, solver):
         rep, faces = solve(hip, solver, 1e-8, False)
         hip.set_resident_limits(workgroups=0)
         ref, expected = solve(hip, solver, 1e-8, False)
-        hip.set_resident_limits(workgroups=limits["workgroups"], polls=0)
+        hip.set_resident_limits(workgroups=limits["workgroups"], iterations=0)
         got, fell_back = solve(hip, solver, 1e-8, False)
         assert got.iterations == ref.iterations
         assert np.array_equal(fell_back, expected)
-        hip.set_resident_limits(polls=limits["polls"])
+        hip.set_resident_limits(iterations=limits["iterations"])
         again, same = solve(hip, solver, 1e-8, False)
         assert again.iterations == rep.iterations
         assert np.array_equal(same, faces)
@@ -105,8 +105,9 @@ def test_a_device_with_less_lds_takes_launches(solver):
 def test_resident_limits_are_clamped_and_checked():
     with msa.HipBackend(0) as hip:
         most = hip.resident_limits()
-        assert most["workgroups"] > 0 and most["polls"] > 0
-        hip.set_resident_limits(workgroups=0xffffffff, polls=0xffffffff, round_tag=9)
+        assert most["workgroups"] > 0 and most["iterations"] > 0
+        hip.set_resident_limits(workgroups=0xffffffff, iterations=0xffffffff,
+                                lds_bytes=0xffffffff, round_tag=9)
         hip.set_resident_limits(round_tag=3)
         assert hip.resident_limits() == {**most, "round_tag": 9}
         with pytest.raises(TypeError):
@@ -209,11 +210,12 @@ def resolved(hip, grid, drag, tolerance, most=50_000):
     return field.concatenated(), rep
 
 
-# Given up at the first look in vain; at the launch's iterations, from the first
-# momentum solve on (3) or a later one (between the shortest and the longest).
-@pytest.mark.parametrize("limit", [dict(polls=0), dict(iterations=3), dict(iterations=None)])
+# Launches that end without an iteration, as one given up does; that end at
+# their iterations, from the first momentum solve on (3) or a later one (None:
+# between the shortest and the longest).
+@pytest.mark.parametrize("iterations", [0, 3, None])
 @pytest.mark.parametrize("dims", [(12, 9, 7), (7, 40, 30), (40, 20, 18)])
-def test_a_momentum_launch_left_undone_falls_back_to_launches(dims, limit):
+def test_a_momentum_launch_left_undone_falls_back_to_launches(dims, iterations):
     grid, drag = resolved_system(dims)
     with msa.HipBackend(0) as hip:
         limits = hip.resident_limits()
@@ -222,12 +224,11 @@ def test_a_momentum_launch_left_undone_falls_back_to_launches(dims, limit):
         expected, ref = resolved(hip, grid, drag, 1e-6)
         hip.set_resident_limits(workgroups=limits["workgroups"])
         mean = rep.inner_iterations // rep.outer_iterations
-        limit = {k: mean if v is None else v for k, v in limit.items()}
-        hip.set_resident_limits(**limit)
+        hip.set_resident_limits(iterations=mean if iterations is None else iterations)
         got, again = resolved(hip, grid, drag, 1e-6)
         # Steps before the one redone were the persistent form's.
         assert abs(again.outer_iterations - ref.outer_iterations) <= 1
-        if "polls" in limit or limit["iterations"] == 3:
+        if iterations is not None:
             assert again.inner_iterations == ref.inner_iterations
             assert np.array_equal(got, expected)
         else:
