@@ -1,7 +1,7 @@
 """The batched sweep on the GPU through the C ABI.
 
-- Pressure: FP32 Jacobi-PCG corrections (FP64 dot products) inside FP64
-  refinement of each instance's FP64 pressure, to FP64 true relative residual
+- Pressure: FP32 corrections by conjugate gradient with the multilevel cycle
+  (FP64 dot products) inside FP64 refinement of each instance's FP64 pressure, to FP64 true relative residual
   1e-10, against the FP64 oracle's solve of the same instance (mo_flow_solve,
   unscaled, times the inlet pressure, to 1e-13): the device's residual equals
   the one recomputed with the oracle's operator (mo_flow_apply) to 1e-6

@@ -27,7 +27,7 @@ SHAPES = [
     (40, 700), (5, 1100),            # rows wider than a workgroup's sites
     (512, 256), (343, 383),          # 512 x 256 sites exactly; just past it
     (513, 511), (700, 751), (1023, 1025),
-    (520, 2017), (300, 3600),        # more sites; halo past the LDS limit
+    (520, 2017), (300, 3600),        # more sites than are taken: the same launches
 ]
 
 
@@ -158,6 +158,29 @@ def test_two_contexts_solve_at_once():
         for again, same in results:
             assert again.iterations == rep.iterations
             assert np.array_equal(same, faces)
+
+
+@pytest.mark.parametrize("nx,ny,solver,taken", [
+    (500, 1792, msa.SOLVER_JACOBI_FP64, True),    # 60 KB of LDS to the byte
+    (500, 1793, msa.SOLVER_JACOBI_FP64, False),
+    (280, 3600, msa.SOLVER_JACOBI_FP64, False),
+    (280, 3600, msa.SOLVER_MIXED, True),          # half of it
+])
+def test_the_lds_limit_decides(nx, ny, solver, taken):
+    # Fewer sites than the most that are taken: the halo of ny sites either side
+    # decides. By launches the bits are the launches'; the persistent form adds
+    # its sums in another order.
+    grid, mobility = system(nx, ny, 6)
+    with msa.HipBackend(0) as hip:
+        hip.flow_prepare(grid, mobility, 0)
+        workgroups = hip.resident_limits()["workgroups"]
+        hip.set_resident_limits(workgroups=0)
+        ref, expected = solve(hip, solver, 1e-8, False)
+        hip.set_resident_limits(workgroups=workgroups)
+        rep, faces = solve(hip, solver, 1e-8, False)
+    assert abs(rep.iterations - ref.iterations) <= 2 * max(1, rep.refinements)
+    assert np.abs(faces - expected).max() <= 1e-5 * np.abs(expected).max()
+    assert np.array_equal(faces, expected) != taken
 
 
 def test_persistent_launches_of_few_iterations_go_on_to_the_same_bits():
