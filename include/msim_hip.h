@@ -88,10 +88,15 @@ typedef struct {
                                   0: return the raw Dirichlet (1 -> 0) field */
   uint32_t check_interval;     /* iterations between host convergence checks; 0 = the
                                   form's own: 64 for Jacobi-PCG (FP64 and MIXED), 8 for
-                                  flexible CG (MULTIGRID, LEARNED) */
+                                  flexible CG (MULTIGRID, LEARNED). Persistent solves
+                                  (msim_resident_limits) check every iteration on the
+                                  device and do not use it */
   double inner_tolerance;      /* MIXED/LEARNED: inner FP32 relative tolerance; 0 = auto */
   uint32_t fallback_iterations;/* LEARNED: iteration cap before the Jacobi-PCG fallback */
-  uint32_t profile;            /* 1: time every Krylov kernel launch with events */
+  uint32_t profile;            /* 1: time every Krylov kernel launch with events. Jacobi-PCG
+                                  then goes by separate launches, also where an unprofiled
+                                  solve would be persistent: the same iteration with its
+                                  sums in another order */
   /* DepthAveragedFlowParameters::body_force (flow.hpp:24-25): the in-plane body
    * force per column in pressure-gradient units, (fx, fy) pairs, x-major,
    * y-minor; NULL for none. A forced flow solves the system a second time with
@@ -117,7 +122,7 @@ typedef struct {
   uint32_t fell_back;            /* LEARNED: 1 when Jacobi-PCG finished the solve */
   double seconds;                /* device time of the solve and reconstruction */
   /* With params.profile: summed event time and launch count of the two
-   * Krylov kernels (operator+direction, and update+dots). */
+   * Krylov kernels (operator+direction, and update+dots) of the launches form. */
   double apply_seconds;
   uint32_t apply_launches;
   double update_seconds;
@@ -770,10 +775,11 @@ int msim_hip_learned_apply(msim_ctx* ctx, uint32_t pair, float* z);
  * fixed reservoirs beyond x = 0 (`reservoir`) and x = nx (0), no-flux walls
  * in y and Monod uptake vmax phi c / (K + c).
  *
- * The pressure (FP32 Jacobi-PCG corrections with FP64 dot products inside
- * FP64 iterative refinement of an FP64 pressure, warm-started, to an FP64
- * true relative residual) is solved by msim_hip_batch_solve_flow, all
- * instances together. A step is one launch over work items (blocks of
+ * The pressure (FP32 conjugate-gradient corrections with each instance's
+ * multilevel cycle and FP64 dot products, inside FP64 iterative refinement of an
+ * FP64 pressure, warm-started, to an FP64 true relative residual) is solved by
+ * msim_hip_batch_solve_flow: batches of small or of many equal instances one
+ * workgroup per instance, others all instances together. A step is one launch over work items (blocks of
  * rows, spread over the chip): each checks its rows' FP64 pressure residual,
  * rebuilds their face velocities and advances them one FP32 forward-Euler
  * transport step whose sites compute exactly as msim_hip_advance_signal_grid's

@@ -5,7 +5,7 @@
 // (docs/architecture/0005-batch-execution.md:30); each instance follows the
 // reference's single-grid algorithms:
 //   pressure  -- the assembled operator (flow_system.hpp:522-695) solved by
-//                FP32 Jacobi-PCG corrections (cpp/cpu/cpu_flow.cpp:65-140; FP64
+//                FP32 conjugate-gradient corrections (cpp/cpu/cpu_flow.cpp:65-140; FP64
 //                dot products) inside FP64 iterative refinement of an FP64
 //                pressure, warm-started, to an FP64 true relative residual;
 //   velocity  -- face velocities and lift (flow_system.hpp:711-736, 424-445)

@@ -420,8 +420,8 @@ __global__ __launch_bounds__(kStream) void k_cg_init(const S* __restrict__ sourc
   }
 }
 
-// Jacobi-PCG iterations in one persistent launch, for systems of at most
-// kPersistSites sites. Each workgroup owns kPersistThreads * S consecutive
+// Jacobi-PCG iterations in one persistent launch, for the systems that
+// persist_shape takes. Each workgroup owns kPersistThreads * S consecutive
 // sites and holds their x, r, coefficients and half of q's use in registers;
 // the direction p of its sites and of the ny sites either side (every site its
 // stencils read) lives in LDS. Per iteration the workgroups meet twice
