@@ -528,8 +528,9 @@ void adr_upload(Context& ctx, const msim_signal_grid& grid, const void* levels,
   a.flags.reserve(3);
   a.state.reserve(2);  // the second holds the survey's masses
   // Ledger partials [2][3 * kMaxSignals][blocks], then the van Leer block
-  // maxima [blocks]; the survey's partials reuse the front.
-  const uint32_t step_parts = adr_shape(P.nx, P.ny, P.limited != 0).blocks;
+  // maxima [blocks]; the survey's partials reuse the front. FP32's shape has
+  // the more blocks.
+  const uint32_t step_parts = adr_shape(P.nx, P.ny, P.limited != 0, 32).blocks;
   a.partials.reserve(std::max<size_t>(
       static_cast<size_t>(3 * kMaxSignals * 2 + 1) * step_parts,
       static_cast<size_t>(kMaxSignals + 1) * 2048));
@@ -736,7 +737,7 @@ void launch_candidate(Context& ctx, float dt, const float* in, float* out, uint3
                       const float* xf, const float* yf) {
   auto& a = ctx.adr;
   const bool limited = a.params.limited != 0;
-  AdrShape sh = adr_shape(a.params.nx, a.params.ny, limited);
+  AdrShape sh = adr_shape(a.params.nx, a.params.ny, limited, 32);
   LedgerParts L{a.partials.data(), a.ledger.data(), sh.blocks};
   double* largest = a.partials.data() + static_cast<size_t>(3 * kMaxSignals * 2) * sh.blocks;
   const auto* src = reinterpret_cast<const uint8_t*>(in);
@@ -755,7 +756,7 @@ void launch_steps(Context& ctx, float dt, uint32_t steps, const float* xf, const
   auto& a = ctx.adr;
   const auto& P = a.params;
   const bool limited = P.limited != 0;
-  AdrShape sh = adr_shape(P.nx, P.ny, limited);
+  AdrShape sh = adr_shape(P.nx, P.ny, limited, a.precision);
   LedgerParts L{a.partials.data(), a.ledger.data(), sh.blocks};
   double* largest = a.partials.data() + static_cast<size_t>(3 * kMaxSignals * 2) * sh.blocks;
   const AdrView v = view_of(ctx);
@@ -1043,7 +1044,7 @@ void adr_step_static(Context& ctx, const msim_signal_grid& grid, float dt, float
   AdrParams P = transport_params(grid);
   const uint32_t S = P.signals;
   const size_t n = static_cast<size_t>(P.nx) * P.ny;
-  const AdrShape sh = adr_shape(P.nx, P.ny, P.limited != 0);
+  const AdrShape sh = adr_shape(P.nx, P.ny, P.limited != 0, 32);
   const uint32_t survey_blocks = std::min<uint32_t>(site_blocks(n), 2048);
   ScratchLayout at;
   const size_t o_state = at.take(sizeof(CgState));

@@ -19,20 +19,22 @@ constexpr int kStripWaves = kStripBlock / kWave;
 
 // Launch shape of a walk: strips of one wave, four waves per block, 12 x-rows
 // per wave, or 8 or 4 on smaller grids for at least 4096 waves (one round of 16
-// per compute unit), and 2 or 1 on those where 4 leave less than 3072. The
-// explicit step at 4096x2048 with three signals (FP64 upwind, FP32 upwind, FP32
-// van Leer): 12 rows take 131, 74 and 109 us, 8 rows 135, 77 and 111, 16 rows
-// 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows 151, 78 and 111: longer
-// walks read fewer rows twice but leave a last round of waves nearly empty. On
-// small grids a walk is a chain of rows, and one of a single row, whose three
-// rows are read at once, the latency of a thread per site. us with 1, 2 and 4
-// rows, three signals:
-//             FP64 upwind       FP32 upwind       FP32 van Leer     a Crank-Nicolson step
-//   256x128    6.8  8.2 10.6     5.3  6.2  8.4     9.7 10.8 13.5    190  359  418
-//   400x300   10.3  9.3 11.3     6.3  6.8  9.0    11.1 11.8 14.4    198  210  262
-//   768x512   15.7 12.9 12.9     8.4  8.2  9.2    14.3 13.9 15.0    237  228  256
-//   1024x512  18.8 16.2 15.9     9.7  9.3 10.3    16.4 15.5 17.2    277  261  290
-//   1531x769  35.4 29.1 25.8    18.1 17.2 15.4    28.9 27.5 25.2    411  398  354
+// per compute unit). The explicit step at 4096x2048 with three signals (FP64
+// upwind, FP32 upwind, FP32 van Leer): 12 rows take 131, 74 and 109 us, 8 rows
+// 135, 77 and 111, 16 rows 138, 84 and 111, 20 rows 128, 91 and 121, 28 rows
+// 151, 78 and 111: longer walks read fewer rows twice but leave a last round of
+// waves nearly empty.
+// FP32 walks take 2 rows where 4 leave less than 3072 waves, and 1 where 2 leave
+// less than 2048: on small grids a walk is a chain of rows, and one of a single
+// row, whose three rows are read at once, the latency of a thread per site. FP64
+// walks stay at 4, since with three signals their bytes count sooner: two rows
+// lose 5 % at 790x512, one 6 % at 420x350. us with 1, 2 and 4 rows, three signals:
+//             FP32 upwind       FP32 van Leer     a Crank-Nicolson step   FP64 upwind
+//   256x128    5.3  6.2  8.4     9.7 10.8 13.5    190  359  418             6.8  8.2 10.6
+//   400x300    6.3  6.8  9.0    11.1 11.8 14.4    198  210  262            10.3  9.3 11.3
+//   768x512    8.4  8.2  9.2    14.3 13.9 15.0    237  228  256            15.7 12.9 12.9
+//   1024x512   9.7  9.3 10.3    16.4 15.5 17.2    277  261  290            18.8 16.2 15.9
+//   1531x769  18.1 17.2 15.4    28.9 27.5 25.2    411  398  354            35.4 29.1 25.8
 // (the 256x128 Crank-Nicolson steps are bimodal: 185 to 333 with one row).
 struct AdrShape {
   uint32_t strips, rows, blocks;
@@ -42,13 +44,16 @@ inline AdrShape adr_shape(uint32_t strips, uint32_t nx, uint32_t rows) {
   return AdrShape{strips, rows, (strips * ((nx + rows - 1) / rows) + kStripWaves - 1) / kStripWaves};
 }
 
-inline AdrShape adr_shape(uint32_t nx, uint32_t ny, bool limited) {
+inline AdrShape adr_shape(uint32_t nx, uint32_t ny, bool limited, uint32_t precision) {
   const uint32_t width = static_cast<uint32_t>(kWave) - (limited ? 4 : 2);
   const uint32_t strips = (ny + width - 1) / width;
   uint32_t rows = 12;
   auto waves = [&] { return static_cast<uint64_t>(strips) * ((nx + rows - 1) / rows); };
   while (rows > 4 && waves() < 4096) rows -= 4;
-  while (rows <= 4 && rows > 1 && waves() < 3072) rows /= 2;
+  if (precision == 32) {
+    if (rows == 4 && waves() < 3072) rows = 2;
+    if (rows == 2 && waves() < 2048) rows = 1;
+  }
   return adr_shape(strips, nx, rows);
 }
 

@@ -483,7 +483,7 @@ void implicit_steps(Context& ctx, float dt, uint32_t steps, const float* xf, con
   // The sweeps of several layers (adr3.hip) leave a partial per `blocks` and
   // neither write obstacle sites nor look for negative levels.
   const bool layered = a.params.nz > 1;
-  const AdrShape shape = adr_shape(a.params.nx, a.params.ny, kLimited);
+  const AdrShape shape = adr_shape(a.params.nx, a.params.ny, kLimited, 32);
   const uint32_t parts_swept = layered ? blocks : shape.blocks;
   for (uint32_t step = 0; step < steps; ++step) {
     // The step's levels stay untouched in `old` until it is accepted: the
@@ -604,7 +604,8 @@ void implicit_run(Context& ctx, float dt, uint32_t steps, const float* xf, const
   a.rhs.reserve(static_cast<size_t>(a.params.signals) * n);
   a.levels_c.reserve(static_cast<size_t>(a.params.signals) * n * sizeof(float));
   if (a.params.has_monod != 0) a.lagged.reserve(static_cast<size_t>(a.params.signals) * n);
-  const uint32_t swept = adr_shape(a.params.nx, a.params.ny, a.params.limited != 0).blocks;
+  const uint32_t swept =
+      adr_shape(a.params.nx, a.params.ny, a.params.limited != 0, 32).blocks;
   a.implicit_sums.reserve(std::max(blocks, swept));
   a.implicit_least.reserve(std::max(blocks, swept));
   a.implicit_state.reserve(1);

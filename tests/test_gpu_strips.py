@@ -88,7 +88,7 @@ def test_settle_of_a_marked_step(hip, oracle):
 @pytest.mark.parametrize("shape,kinds", [((13, 62), KINDS[0]), ((5, 61), KINDS[1]),
                                          ((30, 125), KINDS[2]), ((1400, 63), KINDS[0]),
                                          ((1, 130), KINDS[2]), ((3101, 61), KINDS[1]),
-                                         ((3071, 63), KINDS[0]), ((3091, 121), KINDS[1]),
+                                         ((3071, 63), KINDS[0]), ((2067, 121), KINDS[1]),
                                          ((8195, 63), KINDS[2]), ((16399, 64), KINDS[0])])
 def test_implicit_steps_at_strip_edges(hip, oracle, shape, kinds, limited):
     """Several implicit steps on the device (the accepted iterate changes
